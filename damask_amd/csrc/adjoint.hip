@@ -78,7 +78,7 @@ __global__ void __launch_bounds__(ADJ_WG) adj_assemble_kernel(AdjKArgs a, const 
   double* X = sc.x + e;      // entry r at X[r * N]
   for (int q = 0; q < 9; q++) {
     double xl[9], xs[DMK_NSL_MAX], w[DMK_NSL_MAX];
-    adj_tangent_rhs(ph, pt, f, acc, q, xl, xs, w);
+    adj_tangent_rhs(ph, pt, xi, f, acc, q, xl, xs, w);
     for (int i = 0; i < 9; i++) X[(size_t)(q * sc.nmax + i) * a.N] = xl[i];
     for (int i = 0; i < ph.nsl; i++) X[(size_t)(q * sc.nmax + 9 + i) * a.N] = xs[i];
   }
@@ -242,7 +242,9 @@ __global__ void __launch_bounds__(ADJ_WG) adj_vjp_kernel(AdjKArgs a, const DmkPh
   fld_to_rm(Pb, Pr);
   load_rm(a.Fpb_in, N, e, Fpb);
   adj_vjp_rhs(ph, pt, f, Pr, Fpb, xib, lam, Fb, Fp0ib);
+  adj_scale(xi, ph.nsl, lam, false);
   adj_solve_t(acc, 9 + ph.nsl, lam);
+  adj_scale(xi, ph.nsl, lam, true);
   if (MODE == 0) {
     AdjVec none{nullptr, 0, 0};
     adj_vjp_finish(ph, pt, f, xi, acc, lam, Fb, Fp0ib, false, nullptr, none, none, 0);
@@ -446,7 +448,7 @@ extern "C" int dmk_adjoint_point_host(const dmk_phase_desc* d, double dt, const 
   if (adj_forward(ph, pt, X, f, acc)) return DMK_ERR_ARG;
   if (residual) *residual = adj_residual(ph, pt, X, X0, acc, 1.0e-6, 1.0e-8, 1.0e-6);
   if (adj_factor(ph, pt, X, acc)) return DMK_ERR_ARG;
-  if (A) adj_tangent(ph, pt, f, acc, A);
+  if (A) adj_tangent(ph, pt, X, f, acc, A);
   double Pr[9], Fpr[9], Fb[9], Fp0b[9], x0b[DMK_NSL_MAX];
   fld_to_rm(Pbar, Pr);
   if (Fpbar) fld_to_rm(Fpbar, Fpr);

@@ -156,11 +156,16 @@ DHI double adj_residual(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjVec&
   return res;
 }
 
-// Jacobian G_y of the increment equations
+// Jacobian G_y of the increment equations, in the unknowns (L_p, xi_a / x_a) and
+// with the xi equations over x_a, x_a the recorded xi_a (adj_scale below): in
+// plain units its blocks span 1e-9 .. 1e8 and the pivoting, which then picks
+// xi rows for their units, loses half of the digits (measured on an 8^3 tension
+// gradient: 1e-8 of change for a last-bit change of the cotangent, with any
+// linear-solver tolerance).
 DHI void adj_assemble(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjVec& xi, const AdjAcc& acc) {
   const int m = ph.nsl;
   const double dt = pt.dt;
-  // d G1 / d L_p = I - sum_b P_b kt_b T_b^T ; d G1 / d xi_b = P_b n_b gdot_b / xi_b
+  // (before scaling) d G1 / d L_p = I - sum_b P_b kt_b T_b^T ; d G1 / d xi_b = P_b n_b gdot_b / xi_b
   for (int k = 0; k < 9; k++) {
     double row[9];
     for (int l = 0; l < 9; l++) row[l] = k == l ? 1.0 : 0.0;
@@ -170,12 +175,12 @@ DHI void adj_assemble(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjVec& x
         for (int l = 0; l < 9; l++) row[l] = fma(-c, acc.v(AV_T + l, b), row[l]);
     }
     for (int l = 0; l < 9; l++) acc.G(k, l) = row[l];
-    for (int b = 0; b < m; b++) acc.G(k, 9 + b) = ph.P[b][k] * ph.n[b] * acc.v(AV_GD, b) / xi(b);
+    for (int b = 0; b < m; b++) acc.G(k, 9 + b) = ph.P[b][k] * ph.n[b] * acc.v(AV_GD, b);
   }
   // d G2_a / d L_p = -dt hf_a phi_a sum_b H_ab s_b kt_b T_b ;
   // d G2_a / d xi_b = delta_ab (1 - dt hf_a phi'_a r_a) + dt hf_a phi_a H_ab n_b |gdot_b| / xi_b
   for (int a = 0; a < m; a++) {
-    double ca = -dt * ph.hf[a] * acc.v(AV_PHI, a);
+    const double ca = -dt * ph.hf[a] * acc.v(AV_PHI, a) / xi(a);
     double row[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int b = 0; b < m; b++) {
       double c = ca * ph.H[a][b] * acc.v(AV_SG, b) * acc.v(AV_KT, b);
@@ -185,8 +190,14 @@ DHI void adj_assemble(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjVec& x
     for (int l = 0; l < 9; l++) acc.G(9 + a, l) = row[l];
     for (int b = 0; b < m; b++)
       acc.G(9 + a, 9 + b) = (a == b ? 1.0 - dt * ph.hf[a] * acc.v(AV_DPHI, a) * acc.v(AV_R, a) : 0.0)
-                          - ca * ph.H[a][b] * ph.n[b] * fabs(acc.v(AV_GD, b)) / xi(b);
+                          - ca * ph.H[a][b] * ph.n[b] * fabs(acc.v(AV_GD, b));
   }
+}
+
+// right-hand side (inverse = false) and solution (true) of G_y^T lambda = b
+// between plain units and those of the assembled Jacobian
+DHI void adj_scale(const AdjVec& xi, int m, double* lam, bool inverse) {
+  for (int a = 0; a < m; a++) lam[9 + a] = inverse ? lam[9 + a] / xi(a) : lam[9 + a] * xi(a);
 }
 
 // LU factorisation with partial pivoting in place (row interchanges in piv;
@@ -258,10 +269,10 @@ DHI void adj_solve_t(const AdjAcc& acc, int n, double* x) {
 // dP/dF of the increment map with the internal variables re-equilibrated,
 // one direction dF = e_q0 (x) e_q1 (q = q0 + 3 q1) at a time:
 // right-hand side -dG/dF dF of G_y dy = -dG/dF dF: L_p part in xl (9), xi
-// part in xs (m); w (m) is workspace.  The xi rows are formed one at a time
+// part in xs (m, over xi as in adj_assemble); w (m) is workspace.  The xi rows are formed one at a time
 // from the rate changes so that nothing accumulates through memory.
-DHI void adj_tangent_rhs(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjFwd& f, const AdjAcc& acc, int q,
-                         double* xl, double* xs, double* w) {
+DHI void adj_tangent_rhs(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjVec& xi, const AdjFwd& f,
+                         const AdjAcc& acc, int q, double* xl, double* xs, double* w) {
   const int m = ph.nsl, q0 = q % 3, q1 = q / 3;
   const double dt = pt.dt;
   double dA0[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -285,7 +296,7 @@ DHI void adj_tangent_rhs(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjFwd
   for (int a = 0; a < m; a++) {
     double s = 0.0;
     for (int b = 0; b < m; b++) s = fma(ph.H[a][b], w[b], s);
-    xs[a] = dt * ph.hf[a] * acc.v(AV_PHI, a) * s;
+    xs[a] = dt * ph.hf[a] * acc.v(AV_PHI, a) * s / xi(a);
   }
 }
 
@@ -332,10 +343,11 @@ DHI void adj_tangent_col(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjFwd
   adj_tangent_dP(ph, pt, f, q, x, A + 9 * q);
 }
 
-DHI void adj_tangent(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjFwd& f, const AdjAcc& acc, double* A) {
+DHI void adj_tangent(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjVec& xi, const AdjFwd& f, const AdjAcc& acc,
+                     double* A) {
   for (int q = 0; q < 9; q++) {
     double x[9 + DMK_NSL_MAX], w[DMK_NSL_MAX];
-    adj_tangent_rhs(ph, pt, f, acc, q, x, x + 9, w);
+    adj_tangent_rhs(ph, pt, xi, f, acc, q, x, x + 9, w);
     adj_solve(acc, 9 + ph.nsl, x);
     adj_tangent_col(ph, pt, f, q, x, A);
   }
@@ -463,6 +475,8 @@ DHI void adj_vjp(const DmkPhaseDev& ph, const AdjPoint& pt, const AdjFwd& f, con
                  const AdjVec& xi0b, const AdjVec& thb, int ldth) {
   double lam[9 + DMK_NSL_MAX], Fp0ib[9];
   adj_vjp_rhs(ph, pt, f, Pb, Fpb, xib, lam, Fb, Fp0ib);
+  adj_scale(xi, ph.nsl, lam, false);
   adj_solve_t(acc, 9 + ph.nsl, lam);
+  adj_scale(xi, ph.nsl, lam, true);
   adj_vjp_finish(ph, pt, f, xi, acc, lam, Fb, Fp0ib, params, Fp0b, xi0b, thb, ldth);
 }
