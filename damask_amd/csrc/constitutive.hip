@@ -13,18 +13,23 @@
 // L_i = 0 throughout; the 3x3x3x3 chains of the reference then collapse to
 // rank-N_sl updates of the 9x9 identity:
 //   dR_Lp/dL_p = I9 + dt * sum_a dgamma_a vec(P_a) vec(G^T Q_a)^T,  G = F_e^T A,
-//   Q_a = C : P_nS,a (tabulated per phase), vec row-major (math_33to9),
-// which is assembled in registers and solved by Householder QR (dmk_dense.h).
+//   Q_a = C : P_nS,a,
+// whose rank is at most that of the symmetric tensors the Q_a span, 5 with the
+// Schmid law and 6 with non-Schmid terms: the Newton step and the consistent
+// tangent are solved in that space (integrate_stress, tangent_kernel), by
+// Householder QR in registers (dmk_dense.h).
 //
-// Register budget.  The 8x8 Newton system (64 doubles) is the only large
-// register object.  Slip-system loops are rolled (the kinetics loop by two) so
-// the phase tables are read through scalar loads inside the loop instead of
-// being hoisted into VGPRs; the per-system vectors of a lane (xi, rates, rate
-// derivatives) and its sub-step bookkeeping live in LDS, [system][lane], one
-// wavefront per work-group.  Sub-step start values, the state-rate history of
-// the fixed-point iteration and the line search's fallback live in global
-// scratch; which start values apply is a per-lane flag, not a per-lane
-// pointer, so no 64-bit addresses stay live across the Newton loop.
+// What bounds the stress kernel: FP64 issue and the latency of a wavefront's own
+// chain (Newton steps in sequence, each with a QR and scalar table loads), not
+// HBM.  64^3 cells of the cF tension, 5.5 Newton iterations a cell: 0.275 ms a
+// launch, 0.69 ms as an 8x8 system per Newton step with the state in global
+// scratch; 45x50x54 cells with 24 systems 0.36 against 0.95 ms; 16^3 cells (one
+// wavefront a CU) 0.09 against 0.21 ms.
+// Register budget: between the Newton steps only A and L_p live in registers;
+// per-system values (1/xi, d rate / d tau, rates), the Newton direction and the
+// sub-step bookkeeping live in LDS, [system][lane], one wavefront per
+// work-group; the state-rate history of the fixed-point iteration is in global
+// scratch.
 #include <cmath>
 
 #include "dmk_common.h"
@@ -35,13 +40,13 @@ namespace {
 
 constexpr int SWG = DMK_STRESS_WG;   // work-group of the per-cell kernels: one wavefront
 
-// The stress kernel runs two waves per SIMD: measured on the 64^3 tension
-// workload this is 20 % faster than one wave per SIMD without spills, the
-// second wave hiding the scalar-load and dependency latency of the slip loops
-// (at the cost of spilling a few loop-carried tensors around the QR solve).
-#ifndef DMK_STRESS_WAVES
-#define DMK_STRESS_WAVES 2
-#endif
+// Wavefronts per SIMD.  12 systems: two (256 registers, a few spills) hide each
+// other's latency: 0.275 ms a launch at 64^3 against 0.36 ms with one and no
+// spills.  24 systems: the LDS vectors leave room for five work-groups a CU and
+// the state update holds 144 values, so one (512 registers): 0.36 ms at
+// 45x50x54 against 0.66 ms with two; non-Schmid terms alike (0.59 against 1.17 ms
+// at 48^3 with half the cells in such a phase).
+constexpr int stress_waves(int nsl) { return nsl > 12 ? 1 : 2; }
 
 // Library transcendental functions are kept out of line: inlined, their
 // polynomial constants are hoisted out of every enclosing loop and stay live
@@ -93,78 +98,366 @@ __global__ void pow_law_kernel(const double* __restrict__ x, const double* __res
   if (i < n) out[i] = pow_law<QP>(x[i], y[i]);
 }
 
+// Coordinates of the per-cell algebra.  The Schmid tensors are traceless, and
+// with them every plastic quantity lies in the span of eight constant tensors:
+// five symmetric deviators E_1 = diag(1,-1,0)/sqrt2, E_2 = diag(1,1,-2)/sqrt6,
+// E_3..E_5 = (e_i e_j + e_j e_i)/sqrt2 for (ij) = (12), (02), (01), and three
+// skew ones R_m = (e_i e_j - e_j e_i)/sqrt2 for the same pairs, an orthonormal
+// set.  Cubic elasticity is diagonal in E (C11 - C12, C11 - C12, 2 C44 x 3), and
+// a resolved stress is S : P_nS_a with S symmetric, so of the projections only
+// the E part acts: 5 numbers per system, with non-Schmid terms 6
+// (E_6 = I/sqrt3, modulus C11 + 2 C12).  Per phase: sp = (E, R) of P_a, qp / qm =
+// E of P_nS_a in the positive / negative sense.
+constexpr double R2 = 0.70710678118654752440;   // 1/sqrt2
+constexpr double R3 = 0.57735026918962576451;   // 1/sqrt3
+constexpr double R6 = 0.40824829046386301637;   // 1/sqrt6
+
+// The phase tables are read through the constant address space: the addresses
+// are uniform, so every read is a scalar load.  Through a plain pointer the
+// compiler takes vector loads in loops that also store, 2000 a wavefront, each a
+// trip to L2 in the Newton's dependency chain (0.53 instead of 0.35 ms at 64^3
+// when this was measured alone).
+using PhPtr = const __attribute__((address_space(4))) DmkPhaseDev*;
+
+template <bool NS>
+constexpr int sym_rank() { return NS ? 6 : 5; }
+
+// E_k : X of any 3x3
+template <int RK>
+DI void sym_proj(const double* X, double* t) {
+  t[0] = (X[0] - X[4]) * R2;
+  t[1] = (X[0] + X[4] - 2.0 * X[8]) * R6;
+  t[2] = (X[5] + X[7]) * R2;
+  t[3] = (X[2] + X[6]) * R2;
+  t[4] = (X[1] + X[3]) * R2;
+  if (RK == 6) t[5] = (X[0] + X[4] + X[8]) * R3;
+}
+
+// sum_k h_k E_k + sum_m k_m R_m
+DI void from_basis(const double* h, const double* k, double* X) {
+  const double a = h[0] * R2, b = h[1] * R6;
+  X[0] = b + a;
+  X[4] = b - a;
+  X[8] = -2.0 * b;
+  double s = h[2] * R2, q = k[0] * R2;
+  X[5] = s + q; X[7] = s - q;
+  s = h[3] * R2; q = k[1] * R2;
+  X[2] = s + q; X[6] = s - q;
+  s = h[4] * R2; q = k[2] * R2;
+  X[1] = s + q; X[3] = s - q;
+}
+
+// modulus of E_k
+template <int RK>
+DI double modulus(PhPtr ph, int k) {
+  return k < 2 ? ph->C11 - ph->C12 : (k < 5 ? 2.0 * ph->C44 : ph->C11 + 2.0 * ph->C12);
+}
+
+// E_k : S of S = C : (Fe^T Fe - I)/2.  The diagonal sums start at -1, so that
+// their roundings are those of the small strain's last steps.
+template <int RK>
+DI void stress_coords(PhPtr ph, const double* Fe, double* s) {
+  double c[6];   // Fe^T Fe - I: 00, 11, 22, 12, 02, 01
+#pragma unroll
+  for (int q = 0; q < 6; q++) {
+    const int i = q < 3 ? q : (q == 3 ? 1 : 0), j = q < 3 ? q : (q == 5 ? 1 : 2);
+    double v = q < 3 ? fma(Fe[i], Fe[j], -1.0) : Fe[i] * Fe[j];
+    v = fma(Fe[3 + i], Fe[3 + j], v);
+    c[q] = fma(Fe[6 + i], Fe[6 + j], v);
+  }
+  const double d = 0.5 * (ph->C11 - ph->C12), g = ph->C44;
+  s[0] = (c[0] - c[1]) * (d * R2);
+  s[1] = (c[0] + c[1] - 2.0 * c[2]) * (d * R6);
+  s[2] = c[3] * (2.0 * R2 * g);
+  s[3] = c[4] * (2.0 * R2 * g);
+  s[4] = c[5] * (2.0 * R2 * g);
+  if (RK == 6) s[5] = (c[0] + c[1] + c[2]) * (0.5 * R3 * (ph->C11 + 2.0 * ph->C12));
+}
+
 // per-lane slip-system vectors, entry a of a lane at [a][lane]
 template <int NSL>
 struct SlipLds {
-  double xi[NSL][SWG];    // critical resolved shear stress of the current state
-  double g[NSL][SWG];     // slip rates (signed), |rate| once the state rate is formed
-  double w[NSL][SWG];     // d rate / d tau in the stress Newton loop, xi rate in the state loop
+  double g[NSL][SWG];     // d rate / d tau in the stress Newton loop, |rate| in the state loop
+  double w[NSL][SWG];     // 1 / xi in the stress Newton loop, xi rate in the state loop
+  double dir[9][SWG];     // the Newton direction, read back when a step is rejected
   // sub-step bookkeeping of a lane, kept out of the registers the Newton needs
-  double frac[SWG], step[SWG], dt_done[SWG];
+  double frac[SWG], step[SWG];
   int nsub[SWG], fpi[SWG];
 };
 
-// kinetics_sl (src/phase_mechanical_plastic_phenopowerlaw.f90:449-488) for all
-// systems of one lane: rates -> gs, derivatives -> ws (DERIV), and
-// L_p = sum_a rate_a P_a (src/phase_mechanical_plastic_phenopowerlaw.f90:325-338) when LP.
-template <int NSL, bool QP, bool DERIV, bool LP>
-DI void kinetics(const DmkPhaseDev* __restrict__ ph, const double* Mp, const double* xs, double* gs,
-                 double* ws, double* Lp) {
-  if (LP) {
+// The slip-system loops take CH systems at once, so that their chains overlap,
+// and read the phase tables in batches of GRP systems (64 scalar registers);
+// batch_end keeps the compiler from loading the batches all together, which are
+// more values than there are scalar registers.  What a loop leaves for another
+// goes through LDS, [system][lane].
+constexpr int CH = 12, GRP = 4;
+
+DI void batch_end() { __builtin_amdgcn_sched_barrier(0); }
+
+// resolved stress of system a: signed tau with the Schmid law, max(tau+, tau-)
+// with non-Schmid terms (pos: the positive sense acts)
+template <bool NS>
+DI double resolved(PhPtr ph, int a, const double* s, bool& pos) {
+  // the Schmid law projects on P itself
+  double tp = s[0] * (NS ? ph->qp[a][0] : ph->sp[a][0]);
 #pragma unroll
-    for (int k = 0; k < 9; k++) Lp[k] = 0.0;
+  for (int k = 1; k < sym_rank<NS>(); k++) tp = fma(s[k], NS ? ph->qp[a][k] : ph->sp[a][k], tp);
+  if (!NS) {
+    pos = tp > 0.0;
+    return tp;
   }
-  const bool nonschmid = ph->nonschmid;
-#pragma unroll 2
-  for (int a = 0; a < NSL; a++) {
-    double tp = 0.0;
+  double tn = s[0] * ph->qm[a][0];
 #pragma unroll
-    for (int k = 0; k < 9; k++) tp = fma(Mp[k], ph->Pp[a][k], tp);
-    double tn;
-    if (nonschmid) {
-      tn = 0.0;
+  for (int k = 1; k < sym_rank<NS>(); k++) tn = fma(s[k], ph->qm[a][k], tn);
+  pos = tp > tn;
+  return fmax(tp, tn);
+}
+
+// x_j^(k/4) of n values with one binary powering of x, sqrt(x) or sqrt(sqrt(x)),
+// as pow_law takes one: the branches are taken once and the products are n
+// independent chains
+template <int n>
+DI void quarter_power(double* x, int k) {
+  if (k & 3) {
 #pragma unroll
-      for (int k = 0; k < 9; k++) tn = fma(Mp[k], ph->Pm[a][k], tn);
+    for (int j = 0; j < n; j++) x[j] = sqrt(x[j]);
+    if (k & 1) {
+#pragma unroll
+      for (int j = 0; j < n; j++) x[j] = sqrt(x[j]);
     } else {
-      tn = -tp;
+      k >>= 1;
     }
-    double sgn = tp > tn ? 1.0 : -1.0;
-    double tmax = fmax(tp, tn);
-    double gg = sgn * ph->g0[a] * pow_law<QP>(tmax / xs[a * SWG], ph->n[a]);
-    gs[a * SWG] = gg;
-    if (DERIV) ws[a * SWG] = !dEq0(gg) ? gg * ph->n[a] / tmax : 0.0;
-    if (LP) {
+  } else {
+    k >>= 2;
+  }
+  double r[n];
 #pragma unroll
-      for (int k = 0; k < 9; k++) Lp[k] = fma(gg, ph->P[a][k], Lp[k]);
+  for (int j = 0; j < n; j++) r[j] = 1.0;
+  while (k) {
+    if (k & 1) {
+#pragma unroll
+      for (int j = 0; j < n; j++) r[j] *= x[j];
+    }
+    k >>= 1;
+    if (k) {
+#pragma unroll
+      for (int j = 0; j < n; j++) x[j] *= x[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < n; j++) x[j] = r[j];
+}
+
+// kinetics_sl (src/phase_mechanical_plastic_phenopowerlaw.f90:449-488) of all
+// systems of one lane at the stress coordinates s; ixs: 1/xi per system (LDS).
+// NEWTON: gs <- d rate / d tau (0 where the rate is 0), L_p = sum_a rate_a P_a in
+// basis coordinates l (E) and k3 (R), posm: bit a set where the positive sense
+// of system a acts; otherwise gs <- |rate|.
+// A phase whose systems share one exponent n >= 1, a multiple of 1/4 (n_k = 4 n),
+// takes x^(n-1) of CH systems by one powering, then x^n = x^(n-1) x and
+// n x^(n-1) / xi without a division; others take one power after the other
+// (rolled: the out-of-line pow then has one call site).
+template <int NSL, bool QP, bool NS, bool NEWTON>
+DI void kinetics(PhPtr ph, const double* s, const double* ixs, double* gs, double* l,
+                 double* k3, unsigned& posm) {
+  if (NEWTON) {
+#pragma unroll
+    for (int k = 0; k < 5; k++) l[k] = 0.0;
+#pragma unroll
+    for (int m = 0; m < 3; m++) k3[m] = 0.0;
+    posm = 0;
+  }
+  const int nk = QP ? ph->n_k : 0;
+#pragma unroll 1
+  for (int a0 = 0; a0 < NSL; a0 += CH) {
+    double x[CH], r[CH];
+    unsigned pm = 0;
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      bool pos;
+      x[j] = resolved<NS>(ph, a0 + j, s, pos) * ixs[(a0 + j) * SWG];
+      if (NS && pos) pm |= 1u << j;
+      if (j % GRP == GRP - 1) batch_end();
+    }
+    if (NEWTON) posm |= pm << a0;
+    if (QP && nk) {
+#pragma unroll
+      for (int j = 0; j < CH; j++) r[j] = NS ? x[j] : fabs(x[j]);
+      quarter_power<CH>(r, nk - 4);                    // x^(n-1)
+    } else {
+#pragma unroll
+      for (int j = 0; j < CH; j++) gs[(a0 + j) * SWG] = NS ? x[j] : fabs(x[j]);
+#pragma unroll 1
+      for (int j = a0; j < a0 + CH; j++) gs[j * SWG] = pow_law<QP>(gs[j * SWG], ph->n[j]);
+#pragma unroll
+      for (int j = 0; j < CH; j++) r[j] = gs[(a0 + j) * SWG];
+    }
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      const int a = a0 + j;
+      const double ixi = ixs[a * SWG];
+      const bool pos = NS ? (pm >> j) & 1u : x[j] > 0.0;
+      double g, w;
+      if (QP && nk) {
+        const double f = NS && !pos ? -ph->g0[a] : ph->g0[a];
+        g = f * (r[j] * x[j]);
+        w = f * ph->n[a] * (r[j] * ixi);
+      } else {
+        g = (pos ? ph->g0[a] : -ph->g0[a]) * r[j];
+        w = g * ph->n[a] * ixi * dmk_rcp(x[j]);
+      }
+      if (NEWTON) {
+        gs[a * SWG] = !dEq0(g) ? w : 0.0;
+#pragma unroll
+        for (int k = 0; k < 5; k++) l[k] = fma(g, ph->sp[a][k], l[k]);
+#pragma unroll
+        for (int m = 0; m < 3; m++) k3[m] = fma(g, ph->sp[a][5 + m], k3[m]);
+        if (j % GRP == GRP - 1) batch_end();
+      } else {
+        gs[a * SWG] = fabs(g);
+      }
     }
   }
 }
 
+// |rate| from the derivatives that kinetics left in gs: rate = tau (d rate / d tau) / n
+template <int NSL, bool NS>
+DI void rates_of_derivatives(PhPtr ph, const double* s, double* gs) {
+#pragma unroll 1
+  for (int a0 = 0; a0 < NSL; a0 += CH) {
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      bool pos;
+      const int a = a0 + j;
+      gs[a * SWG] = fabs(gs[a * SWG] * resolved<NS>(ph, a, s, pos) * ph->inv_n[a]);
+      if (j % GRP == GRP - 1) batch_end();
+    }
+  }
+}
+
+// W_l = sum_a u_a q_al P_a, u_a = scale * us_a (LDS), for the acting projections
+// q (E coordinates): its E coordinates H[k][l] and R coordinates K[m][l].  With
+// the Schmid law q = p of the same system and H is symmetric (15 products
+// instead of 25).
+template <int NSL, bool NS>
+DI void slip_moments(PhPtr ph, const double* us, double scale, unsigned posm,
+                     double (*H)[sym_rank<NS>()], double (*K)[sym_rank<NS>()]) {
+  constexpr int RK = sym_rank<NS>(), G = NS ? 2 : GRP;
+#pragma unroll
+  for (int l = 0; l < RK; l++) {
+#pragma unroll
+    for (int k = 0; k < 5; k++) H[k][l] = 0.0;
+#pragma unroll
+    for (int m = 0; m < 3; m++) K[m][l] = 0.0;
+  }
+#pragma unroll 1
+  for (int a0 = 0; a0 < NSL; a0 += G) {
+#pragma unroll
+    for (int j = 0; j < G; j++) {
+      const int a = a0 + j;
+      const bool pos = (posm >> a) & 1u;
+      const double u = scale * us[a * SWG];
+#pragma unroll
+      for (int l = 0; l < RK; l++) {
+        const double v = u * (NS ? (pos ? ph->qp[a][l] : ph->qm[a][l]) : ph->sp[a][l]);
+#pragma unroll
+        for (int k = NS ? 0 : l; k < 5; k++) H[k][l] = fma(v, ph->sp[a][k], H[k][l]);
+#pragma unroll
+        for (int m = 0; m < 3; m++) K[m][l] = fma(v, ph->sp[a][5 + m], K[m][l]);
+      }
+    }
+  }
+  if (!NS) {
+#pragma unroll
+    for (int l = 1; l < RK; l++)
+#pragma unroll
+      for (int k = 0; k < l; k++) H[k][l] = H[l][k];
+  }
+}
+
+// The 9x9 systems of the material point (identity plus one rank-1 term per
+// slip system) reduced to the RK symmetric directions: with W_l as above and
+// t_k(X) = E_k : (G X), N_kl = delta_kl / C_k + t_k(W_l).
+template <int RK>
+DI void reduced_matrix(PhPtr ph, const double* G, const double (*H)[RK],
+                       const double (*K)[RK], double* N) {
+#pragma unroll
+  for (int l = 0; l < RK; l++) {
+    double h[5], k3[3], W[9], GW[9], t[6];
+#pragma unroll
+    for (int k = 0; k < 5; k++) h[k] = H[k][l];
+#pragma unroll
+    for (int m = 0; m < 3; m++) k3[m] = K[m][l];
+    from_basis(h, k3, W);
+    m_mul(G, W, GW);
+    sym_proj<RK>(GW, t);
+#pragma unroll
+    for (int k = 0; k < RK; k++) N[RK * k + l] = t[k];
+  }
+#pragma unroll
+  for (int k = 0; k < RK; k++) N[(RK + 1) * k] += 1.0 / modulus<RK>(ph, k);
+}
+
+// sum_l y_l W_l
+template <int RK>
+DI void moments_apply(const double (*H)[RK], const double (*K)[RK], const double* y, double* X) {
+  double h[5], k3[3];
+#pragma unroll
+  for (int k = 0; k < 5; k++) {
+    h[k] = H[k][0] * y[0];
+#pragma unroll
+    for (int l = 1; l < RK; l++) h[k] = fma(H[k][l], y[l], h[k]);
+  }
+#pragma unroll
+  for (int m = 0; m < 3; m++) {
+    k3[m] = K[m][0] * y[0];
+#pragma unroll
+    for (int l = 1; l < RK; l++) k3[m] = fma(K[m][l], y[l], k3[m]);
+  }
+  from_basis(h, k3, X);
+}
+
 // phenopowerlaw_dotState without twins (src/phase_mechanical_plastic_phenopowerlaw.f90:356-397)
-// from the slip rates in gs: gs <- |rate| (gamma rate), ws <- xi rate.
+// from the gamma rates gs = |slip rate|: ws = 1/xi -> xi rate.
 // xi_sat = xi_inf + f_sat sqrt(sum F_tw) and hf = h_0 (1 + c_1 (sum F_tw)^c_2) at sum F_tw = 0
 // are tabulated per phase.  Returns true when a rate is NaN.
 template <int NSL, bool QP>
-DI bool dot_state(const DmkPhaseDev* __restrict__ ph, const double* xs, double* gs, double* ws) {
+DI bool dot_state(PhPtr ph, const double* gs, double* ws) {
+  const int ak = QP ? ph->a_k : 0;
+#pragma unroll 1
+  for (int r0 = 0; r0 < NSL; r0 += CH) {
+    double x[CH], p[CH];
+#pragma unroll
+    for (int j = 0; j < CH; j++) x[j] = 1.0 - dmk_rcp(ws[(r0 + j) * SWG] * ph->xi_sat[r0 + j]);   // 1 - xi / xi_sat
+    if (QP && ak) {
+#pragma unroll
+      for (int j = 0; j < CH; j++) p[j] = fabs(x[j]);
+      quarter_power<CH>(p, ak);
+    } else {
+#pragma unroll
+      for (int j = 0; j < CH; j++) ws[(r0 + j) * SWG] = fabs(x[j]);
+#pragma unroll 1
+      for (int j = r0; j < r0 + CH; j++) ws[j * SWG] = pow_law<QP>(ws[j * SWG], ph->a[j]);
+#pragma unroll
+      for (int j = 0; j < CH; j++) p[j] = ws[(r0 + j) * SWG];
+    }
+#pragma unroll
+    for (int j = 0; j < CH; j++) ws[(r0 + j) * SWG] = ph->hf[r0 + j] * copysign(p[j], x[j]);
+  }
   double hg[NSL];
 #pragma unroll
   for (int r = 0; r < NSL; r++) hg[r] = 0.0;
   bool nan = false;
-#pragma unroll 1
+#pragma unroll 48 / NSL
   for (int a = 0; a < NSL; a++) {
-    double ga = fabs(gs[a * SWG]);
-    gs[a * SWG] = ga;
+    const double ga = gs[a * SWG];
     nan |= (ga != ga);
 #pragma unroll
-    for (int r = 0; r < NSL; r++) hg[r] = fma(ph->H[r][a], ga, hg[r]);
+    for (int r = 0; r < NSL; r++) hg[r] = fma(ph->Hc[a][r], ga, hg[r]);
   }
 #pragma unroll
-  for (int r = 0; r < NSL; r++) ws[r * SWG] = hg[r];
-#pragma unroll 1
   for (int r = 0; r < NSL; r++) {
-    double x = 1.0 - xs[r * SWG] / ph->xi_sat[r];
-    double left = copysign(pow_law<QP>(fabs(x), ph->a[r]), x);
-    double d = ph->hf[r] * left * ws[r * SWG];
+    const double d = ws[r * SWG] * hg[r];
     ws[r * SWG] = d;
     nan |= (d != d);
   }
@@ -172,7 +465,7 @@ DI bool dot_state(const DmkPhaseDev* __restrict__ ph, const double* xs, double* 
 }
 
 // E = (Fe^T Fe - I)/2 and S = C:E (lattice frame)
-DI void hooke(const DmkPhaseDev* __restrict__ ph, const double* Fe, double* S) {
+DI void hooke(PhPtr ph, const double* Fe, double* S) {
   double E[9];
   m_mul_tn(Fe, Fe, E);
   E[0] -= 1.0; E[4] -= 1.0; E[8] -= 1.0;
@@ -181,310 +474,330 @@ DI void hooke(const DmkPhaseDev* __restrict__ ph, const double* Fe, double* S) {
   hooke_sym(ph->C11, ph->C12, ph->C44, E, S);
 }
 
-// a per-lane flag re-read in every loop iteration, so that pointers selected
-// by it are formed where they are used instead of being kept live across loops
-DI bool live_flag(bool f) {
-  int v = f ? 1 : 0;
-  asm volatile("" : "+v"(v));
-  return v != 0;
+// The material-point arguments are read through the constant address space
+// too, where they are used: an argument pointer is a scalar load away, while keeping
+// all of them (and the component bases formed from them) in scalar registers
+// across the Newton loop spills them into vector lanes.
+using MpPtr = const __attribute__((address_space(4))) DmkMPDev*;
+
+DI MpPtr fresh(MpPtr m) {
+  asm volatile("" : "+s"(m));
+  return m;
 }
 
-DI void copy9(double* dst, const double* src, const Lane& l) {
-#pragma unroll
-  for (int c = 0; c < 9; c++) st(dst, l, c, ld(src, l, c));
-}
-
-// per-cell scratch of the stress integration ([DMK_SUB_ROWS][N]): sub-step
-// F_0, sub-step F, F_p0 and L_p0 (the last two once a sub-step has completed),
-// and the Newton line search's last accepted L_p and direction
-enum { SUB_F0 = 0, SUB_F = 9, SUB_FP0 = 18, SUB_LP0 = 27, SUB_LSOLD = 36, SUB_LSDIR = 45 };
-static_assert(SUB_LSDIR + 9 <= DMK_SUB_ROWS, "sub-step scratch rows");
-
-// integrateStress (src/phase_mechanical.f90:379-584) with F_i = I, L_i = 0, for
-// the sub-step F (scratch row SUB_F) and sub-step F_p0 (Fp0_p), starting from
-// the L_p in mp.Lp (the previous call's result: phase_mechanical_Lp is not
-// restored between calls).  On success the converged L_p goes back to mp.Lp
-// and S is returned in registers.  P, F_p and F_e follow from (F, F_p0, L_p, S)
-// alone, so they are formed once, by finish_point, after the state integration
-// has converged instead of after every call.
-template <int NSL, bool QP>
-DI int integrate_stress(const DmkPhaseDev* __restrict__ ph, const DmkNumMech& num, const DmkMPDev& mp,
-                        const Lane& ln, bool started, double dt, SlipLds<NSL>& sh, int lane, int& newton,
-                        double* S) {
-  const double* Fsub_p = mp.sub + SUB_F * ln.sN;
-  const double* xs = &sh.xi[0][lane];
-  double* gs = &sh.g[0][lane];
-  double* ws = &sh.w[0][lane];
-  double A[9];
-  {
-    const double* Fp0_p = live_flag(started) ? mp.sub + SUB_FP0 * ln.sN : mp.Fp0;
-    double Fp0[9], invFp0[9], F[9];
-    m_load(Fp0_p, ln, Fp0);
-    if (m_invert(Fp0, invFp0)) return ST_FAIL_STRESS;
-    m_load(Fsub_p, ln, F);
-    m_mul(F, invFp0, A);
+// a field's value where a sub-step has completed (started) comes from the
+// sub-step scratch q, else from the increment's field f.  Almost no wavefront
+// holds a started cell: the scratch is read only in those that do.
+DI double ld_start(const double* f, const double* q, bool started, const Lane& l, int c) {
+  double v = ld(f, l, c);
+  if (__builtin_expect(__any(started), 0)) {
+    const double u = ld(q, l, c);
+    v = started ? u : v;
   }
-  double Lpg[9];
-  m_load(mp.Lp, ln, Lpg);
-  // the line search's last accepted iterate and direction live in the
-  // scratch (read back only when a step is rejected, and to form the next
-  // iterate), out of the registers the Newton system needs; the first
-  // iteration is always accepted, so both are written before they are read
-  double* ls_old = mp.sub + SUB_LSOLD * ln.sN;
-  double* ls_dir = mp.sub + SUB_LSDIR * ln.sN;
+  return v;
+}
+
+DI void m_load_start(const double* f, const double* q, bool started, const Lane& l, double* T) {
+  m_load(f, l, T);
+  if (__builtin_expect(__any(started), 0)) {
+    double U[9];
+    m_load(q, l, U);
+#pragma unroll
+    for (int k = 0; k < 9; k++) T[k] = started ? U[k] : T[k];
+  }
+}
+
+// per-cell scratch of the stress integration ([DMK_SUB_ROWS][N]), written once
+// a sub-step has completed: its F, F_p and L_p, where the next one starts
+enum { SUB_F0 = 0, SUB_FP0 = 9, SUB_LP0 = 18 };
+static_assert(SUB_LP0 + 9 <= DMK_SUB_ROWS, "sub-step scratch rows");
+
+// F of a sub-step: its start plus step (F - F_0)
+DI void sub_F(MpPtr m, const double* Ftarget, bool started, const Lane& ln, double step, double* F) {
+  MpPtr q = fresh(m);
+  double F0[9], Ft[9];
+  m_load(q->F0, ln, F0);
+  m_load(Ftarget, ln, Ft);
+  m_load_start(q->F0, q->sub + SUB_F0 * ln.sN, started, ln, F);
+#pragma unroll
+  for (int k = 0; k < 9; k++) F[k] = fma(step, Ft[k] - F0[k], F[k]);
+}
+
+// I - dt L_p
+DI void flow(double dt, const double* Lp, double* B) {
+#pragma unroll
+  for (int k = 0; k < 9; k++) B[k] = ((k % 4) == 0 ? 1.0 : 0.0) - dt * Lp[k];
+}
+
+// F_e = A (I - dt L_p) as A - dt (A L_p): one rounding at the size of F_e per
+// entry.  The stress, and n times as much the rates, see this rounding through
+// the elastic stiffness; it is the floor of the Newton iteration's residual
+// (about 1e-11 of L_p).
+DI void elastic_F(double dt, const double* A, const double* Lp, double* Fe) {
+  m_mul(A, Lp, Fe);
+#pragma unroll
+  for (int k = 0; k < 9; k++) Fe[k] = fma(-dt, Fe[k], A[k]);
+}
+
+// integrateStress (src/phase_mechanical.f90:379-584) with F_i = I, L_i = 0 for
+// A = F F_p0^-1, starting from Lp, which holds the converged L_p on success.
+// ixs (LDS): 1/xi per system; on success sh.g holds the |slip rates| at (S, xi).
+// S, P, F_p and F_e follow from (A, F_p0, L_p) alone, so they are formed once, by
+// finish_point, after the state integration has converged.
+//
+// The Newton system (I9 + sum_a u_a vec(P_a) vec(G^T C:P_nS_a)^T) x = res,
+// G = F_e^T A, u_a = dt d rate_a / d tau_a, is the identity plus a map that sees
+// x only through t_k(x) = E_k : (G x): with y_l = C_l t_l(x),
+//   x = res - sum_l y_l W_l,   N y = t(res),   N_kl = delta_kl / C_k + t_k(W_l),
+// W_l = sum_a u_a q_al P_a.  So a 5x5 system (6x6 with non-Schmid terms) is
+// assembled and solved instead of an 8x8 one: the same Newton step.
+template <int NSL, bool QP, bool NS>
+DI int integrate_stress(PhPtr ph, const DmkNumMech& num, const double* A, double det_Fp0,
+                        double dt, SlipLds<NSL>& sh, int lane, int& newton, double* Lp) {
+  constexpr int RK = sym_rank<NS>();
+  const double* ixs = &sh.w[0][lane];
+  double* gs = &sh.g[0][lane];
+  double* dir = &sh.dir[0][lane];
+#pragma unroll
+  for (int k = 0; k < 9; k++) dir[k * SWG] = 0.0;
+  // norms are compared squared
+  const double er2 = num.eps_rel_Lp * num.eps_rel_Lp, ea2 = num.eps_abs_Lp * num.eps_abs_Lp;
   double step = 1.0, res_old = DBL_MAX;
   int it = 0;
   for (;;) {
     it++;
     if (it > num.N_iter_Lp_max) return ST_FAIL_LP_MAXIT;
     newton++;
+    double Fe[9], res[9];
+    unsigned posm;
     {
-      double B[9], Fe[9];
+      double s[6], l[5], k3[3], Lpc[9];
+      elastic_F(dt, A, Lp, Fe);
+      stress_coords<RK>(ph, Fe, s);
+      kinetics<NSL, QP, NS, true>(ph, s, ixs, gs, l, k3, posm);
+      from_basis(l, k3, Lpc);
+      const double ng = m_norm2(Lp), nc = m_norm2(Lpc);
 #pragma unroll
-      for (int k = 0; k < 9; k++) B[k] = ((k % 4) == 0 ? 1.0 : 0.0) - dt * Lpg[k];
-      m_mul(A, B, Fe);
-      hooke(ph, Fe, S);
-    }
-    double Lpc[9];
-    kinetics<NSL, QP, true, true>(ph, S, xs, gs, ws, Lpc);
-    double ng = m_norm(Lpg), nc = m_norm(Lpc);
-    double atol = fmax(num.eps_rel_Lp * fmax(ng, nc), num.eps_abs_Lp);
-    double res[9];
-    bool nan = false;
+      for (int k = 0; k < 9; k++) res[k] = Lp[k] - Lpc[k];
+      const double nres = m_norm2(res);
+      if (nres != nres) return ST_FAIL_LP_NAN;
+      if (nres < fmax(er2 * fmax(ng, nc), ea2)) {
+        rates_of_derivatives<NSL, NS>(ph, s, gs);
+        double B[9];
+        flow(dt, Lp, B);
+        // the reference's error exit when the new plastic deformation is singular
+        // (math_invert33 of F_p0^-1 (I - dt L_p))
+        return dEq0(m_det(B) / det_Fp0) ? ST_FAIL_STRESS : ST_OK;
+      }
+      if (!(nres < res_old)) {
+        // back along the direction from the last accepted L_p
+        const double back = num.r_linesearch_Lp * step - step;
+        step = num.r_linesearch_Lp * step;
 #pragma unroll
-    for (int k = 0; k < 9; k++) { res[k] = Lpg[k] - Lpc[k]; nan |= (res[k] != res[k]); }
-    double nres = m_norm(res);
-    if (nan) return ST_FAIL_LP_NAN;
-    if (nres < atol) break;
-    if (nres < res_old) {
+        for (int k = 0; k < 9; k++) Lp[k] = fma(dir[k * SWG], back, Lp[k]);
+        continue;
+      }
       res_old = nres;
-#pragma unroll
-      for (int k = 0; k < 9; k++) st(ls_old, ln, k, Lpg[k]);
       step = 1.0;
-    } else {
-      step = num.r_linesearch_Lp * step;
-#pragma unroll
-      for (int k = 0; k < 9; k++) Lpg[k] = fma(ld(ls_dir, ln, k), step, ld(ls_old, ln, k));
-      continue;
     }
-    // Jacobian, rebuilt every iteration (f_update_jacobi_Lp = 1):
-    // J = I9 + sum_a u_a vec(P_a) vec(Y_a)^T.  The Schmid tensors P_a are
-    // traceless, so tr(J x) = tr(x) and the solution of J x = res has
-    // x_22 = tr(res) - x_00 - x_11.  Substituting it into rows 0..7 leaves an
-    // 8x8 system (columns 0 and 4 reduced by column 8), which is what is
-    // assembled: J8 = rows/columns 0..7, j8 = column 8 of rows 0..7.
-    double G[9];
+    // Jacobian, rebuilt every iteration (f_update_jacobi_Lp = 1)
+    double H[5][RK], K[3][RK], y[6];
+    slip_moments<NSL, NS>(ph, gs, dt, posm, H, K);
     {
-      // F_e again (cheaper than keeping it live across the kinetics loop)
-      double B[9], Fe[9];
-#pragma unroll
-      for (int k = 0; k < 9; k++) B[k] = ((k % 4) == 0 ? 1.0 : 0.0) - dt * Lpg[k];
-      m_mul(A, B, Fe);
+      double G[9], N[RK * RK], GX[9], rd[RK], v0[RK], tau[RK];
       m_mul_tn(Fe, A, G);
+      reduced_matrix<RK>(ph, G, H, K, N);
+      m_mul(G, res, GX);
+      sym_proj<RK>(GX, y);
+      if (dmk_qr_factor<RK>(N, rd, v0, tau)) return ST_FAIL_LP_DGESV;
+      dmk_qr_apply_solve<RK>(N, rd, v0, tau, y);
     }
-    // The trace substitution x_22 = tr(res) - x_00 - x_11 is applied per slip
-    // system: column 8 of each rank-1 term is subtracted from columns 0 and 4
-    // and its product with tr(res) from the right-hand side, so no ninth column
-    // is kept.
-    double J[64];
-#pragma unroll
-    for (int r = 0; r < 64; r++) J[r] = (r % 9 == 0) ? 1.0 : 0.0;
-    const double tr = res[0] + res[4] + res[8];
-    const bool nonschmid = ph->nonschmid;
-#pragma unroll 1
-    for (int a = 0; a < NSL; a++) {
-      double u = dt * ws[a * SWG];
-      const bool pos = gs[a * SWG] > 0.0;
-      double Y[9];
-      if (nonschmid) {
-        double Q[9];
-#pragma unroll
-        for (int k = 0; k < 9; k++) Q[k] = pos ? ph->Qp[a][k] : ph->Qm[a][k];
-        m_mul_tn(G, Q, Y);
-      } else {
-        // Schmid law: Q_neg = -Q_pos exactly, folded into the sign of u
-        m_mul_tn(G, ph->Qp[a], Y);
-        u = pos ? u : -u;
-      }
-      Y[0] -= Y[8];
-      Y[4] -= Y[8];
-      const double y8tr = Y[8] * tr;
-#pragma unroll
-      for (int r = 0; r < 8; r++) {
-        double pr = u * ph->P[a][r];
-#pragma unroll
-        for (int c = 0; c < 8; c++) J[8 * r + c] = fma(pr, Y[c], J[8 * r + c]);
-        res[r] = fma(-pr, y8tr, res[r]);
-      }
-    }
-    if (dmk_qr_solve<8>(J, res)) return ST_FAIL_LP_DGESV;
-    res[8] = tr - res[0] - res[4];
-    // the accepted iterate was just stored: L_p is read back instead of being
-    // kept live across the solve
+    double X[9];
+    moments_apply<RK>(H, K, y, X);
 #pragma unroll
     for (int k = 0; k < 9; k++) {
-      const double d = -res[k];
-      st(ls_dir, ln, k, d);
-      Lpg[k] = fma(d, step, ld(ls_old, ln, k));
+      const double d = X[k] - res[k];
+      dir[k * SWG] = d;
+      Lp[k] += d;
     }
   }
-  // the reference's error exit when the new plastic deformation is singular
-  // (math_invert33 of F_p0^-1 (I - dt L_p))
-  {
-    const double* Fp0_p = live_flag(started) ? mp.sub + SUB_FP0 * ln.sN : mp.Fp0;
-    double Fp0[9], invFp0[9], B[9], invFp_new[9], Fp_new[9];
-    m_load(Fp0_p, ln, Fp0);
-    m_invert(Fp0, invFp0);
-#pragma unroll
-    for (int k = 0; k < 9; k++) B[k] = ((k % 4) == 0 ? 1.0 : 0.0) - dt * Lpg[k];
-    m_mul(invFp0, B, invFp_new);
-    if (m_invert(invFp_new, Fp_new)) return ST_FAIL_STRESS;
-  }
-  m_store(mp.Lp, ln, Lpg);
-  return ST_OK;
 }
 
-// The end of integrateStress (src/phase_mechanical.f90:571-581) for the
-// converged L_p (mp.Lp) and S (mp.S) of a sub-step with F (scratch row SUB_F),
-// F_p0 (Fp0_p) and time step dt: the regularised F_p = F_p,new / det(F_p,new)^(1/3)
-// goes to Fp_dst; with OUT also P = F F_p,new^-1 S F_p,new^-T and F_e = F F_p,new^-1.
+// The end of integrateStress (src/phase_mechanical.f90:571-581) of a sub-step:
+// F_e = A (I - dt L_p) and S = C:(F_e^T F_e - I)/2; the regularised
+// F_p = F_p,new / det(F_p,new)^(1/3) goes to Fp_dst; with OUT also
+// P = F_e S F_p,new^-T and F_e.
 template <bool OUT>
-DI void finish_point(const DmkMPDev& mp, const Lane& ln, const double* Fp0_p, double dt, double* Fp_dst) {
-  double invFp_new[9], Fp_new[9];
+DI void finish_point(PhPtr ph, MpPtr m, const Lane& ln, bool started, const double* A,
+                     const double* Lp, double dt, double* Fp_dst) {
+  double invFp_new[9], Fp_new[9], Fe[9], S[9];
   {
-    double Fp0[9], invFp0[9], B[9], Lp[9];
-    m_load(Fp0_p, ln, Fp0);
+    double Fp0[9], invFp0[9], B[9];
+    MpPtr q = fresh(m);
+    m_load_start(q->Fp0, q->sub + SUB_FP0 * ln.sN, started, ln, Fp0);
     m_invert(Fp0, invFp0);
-    m_load(mp.Lp, ln, Lp);
-#pragma unroll
-    for (int k = 0; k < 9; k++) B[k] = ((k % 4) == 0 ? 1.0 : 0.0) - dt * Lp[k];
+    flow(dt, Lp, B);
     m_mul(invFp0, B, invFp_new);
   }
-  m_invert(invFp_new, Fp_new);
+  elastic_F(dt, A, Lp, Fe);
+  hooke(ph, Fe, S);
+  m_store(fresh(m)->S, ln, S);
   if (OUT) {
-    double T1[9], P[9];
-    {
-      double F[9], T2[9], S[9];
-      m_load(mp.sub + SUB_F * ln.sN, ln, F);
-      m_load(mp.S, ln, S);
-      m_mul(F, invFp_new, T1);
-      m_mul_nt(S, invFp_new, T2);
-      m_mul(T1, T2, P);
-    }
-    m_store(mp.Pph, ln, P);
-    m_store(mp.Fe, ln, T1);
+    double T[9], P[9];
+    m_mul_nt(S, invFp_new, T);
+    m_mul(Fe, T, P);
+    m_store(fresh(m)->Pph, ln, P);
+    m_store(fresh(m)->Fe, ln, Fe);
   }
+  m_invert(invFp_new, Fp_new);
   double d = pow_ool(m_det(Fp_new), 1.0 / 3.0);
 #pragma unroll
   for (int k = 0; k < 9; k++) Fp_new[k] = Fp_new[k] / d;
   m_store(Fp_dst, ln, Fp_new);
 }
 
-// integrateStateFPI (src/phase_mechanical.f90:591-676).  State = (xi, gamma):
-// xi in LDS, gamma in mp.gam; its start values xi0_p / gam0_p (the converged
-// increment, or st0s after a completed sub-step); the two previous state
-// rates (dotState_last) in the ping-pong buffers mp.last1 / mp.last2.  The
-// initial rate is taken at the stress S_p (S_0 after a restore, else the
-// previous sub-step's S); on success the S of the converged iterate is stored
-// in mp.S.
-template <int NSL, bool QP>
-DI int integrate_state_fpi(const DmkPhaseDev* __restrict__ ph, const DmkNumMech& num, const DmkMPDev& mp,
-                           const Lane& ln, bool started, bool s_cur, double dt, SlipLds<NSL>& sh, int lane,
-                           int& newton) {
-  double* xs = &sh.xi[0][lane];
+// integrateStateFPI (src/phase_mechanical.f90:591-676).  State = (xi, gamma),
+// started from xi0 / gam0 (the converged increment, or st0s after a completed
+// sub-step).  Every iterate of the state is its start plus dt times the last
+// damped rate, so only the rates are kept: the two previous ones
+// (dotState_last) in the ping-pong buffers mp.last1 / mp.last2; xi and gamma are
+// written once, on success.  The initial rate is taken at the stress S_0 after a
+// restore, else at the previous sub-step's S (s_cur).  A and Lp stay in
+// registers; on success Lp holds the converged L_p.
+template <int NSL, bool QP, bool NS>
+DI int integrate_state_fpi(PhPtr ph, const DmkNumMech& num, MpPtr m,
+                           const double* Ftarget, const Lane& ln, bool started, bool s_cur, double step, double dt,
+                           SlipLds<NSL>& sh, int lane, int& newton, double* A, double* Lp) {
+  constexpr int RK = sym_rank<NS>();
   double* gs = &sh.g[0][lane];
   double* ws = &sh.w[0][lane];
+  double det_Fp0;
   {
-    double S0[9];
-    m_load(s_cur ? mp.S : mp.S0, ln, S0);
-    kinetics<NSL, QP, false, false>(ph, S0, xs, gs, nullptr, nullptr);
+    double Fp0[9], invFp0[9], F[9];
+    MpPtr q = fresh(m);
+    m_load_start(q->Fp0, q->sub + SUB_FP0 * ln.sN, started, ln, Fp0);
+    sub_F(m, Ftarget, started, ln, step, F);
+    if (m_invert(Fp0, invFp0)) return ST_FAIL_STRESS;
+    m_mul(F, invFp0, A);
+    det_Fp0 = m_det(Fp0);
   }
-  if (dot_state<NSL, QP>(ph, xs, gs, ws)) return ST_FAIL_STATE;
-#pragma unroll 1
-  for (int r = 0; r < NSL; r++) {
-    double dx = ws[r * SWG], dgm = gs[r * SWG];
-    const bool stf = live_flag(started);
-    xs[r * SWG] = fma(dx, dt, ld(stf ? mp.st0s : mp.xi0, ln, r));
-    st(mp.gam, ln, r, fma(dgm, dt, ld(stf ? mp.st0s + NSL * ln.sN : mp.gam0, ln, r)));
-    st(mp.last1, ln, r, dx);
-    st(mp.last1, ln, NSL + r, dgm);
+  // row r of the state's start
+  auto xi_start = [&](MpPtr q, int r) { return ld_start(q->xi0, q->st0s, started, ln, r); };
+  auto gam_start = [&](MpPtr q, int r) {
+    return ld_start(q->gam0, q->st0s + NSL * ln.sN, started, ln, r);
+  };
+  {
+    double S0[9], s[6], x0[NSL];
+    unsigned posm;
+    MpPtr q = fresh(m);
+#pragma unroll
+    for (int r = 0; r < NSL; r++) x0[r] = xi_start(q, r);
+    m_load(s_cur ? q->S : q->S0, ln, S0);
+#pragma unroll
+    for (int r = 0; r < NSL; r++) ws[r * SWG] = dmk_rcp(x0[r]);
+    sym_proj<RK>(S0, s);
+    kinetics<NSL, QP, NS, false>(ph, s, ws, gs, nullptr, nullptr, posm);
+    if (dot_state<NSL, QP>(ph, gs, ws)) return ST_FAIL_STATE;
+    MpPtr q2 = fresh(m);
+#pragma unroll
+    for (int r = 0; r < NSL; r++) {
+      const double dx = ws[r * SWG];
+      st(q2->last1, ln, r, dx);
+      st(q2->last1, ln, NSL + r, gs[r * SWG]);
+      ws[r * SWG] = dmk_rcp(fma(dx, dt, x0[r]));
+    }
   }
-  int status = ST_FAIL_STATE;
-  bool cur = false;                   // last1 holds dotState_last(:,1) when !cur
+  bool cur = false;                   // last1 holds dotState_last(:,1) when !cur (uniform in the wavefront)
   for (int it = 1; it <= num.N_iter_state_max; it++) {
     sh.fpi[lane]++;
-    double S[9];
-    status = integrate_stress<NSL, QP>(ph, num, mp, ln, started, dt, sh, lane, newton, S);
-    if (status != ST_OK) break;
-    m_store(mp.S, ln, S);
+    const int status = integrate_stress<NSL, QP, NS>(ph, num, A, det_Fp0, dt, sh, lane, newton, Lp);
+    if (status != ST_OK) return status;
+    MpPtr q = fresh(m);
+    const double* w1p = cur ? q->last2 : q->last1;
+    double* w2p = cur ? q->last1 : q->last2;
+    double w1[2 * NSL], w2[2 * NSL], s0[2 * NSL];
+#pragma unroll
+    for (int r = 0; r < 2 * NSL; r++) w1[r] = ld(w1p, ln, r);
+#pragma unroll
+    for (int r = 0; r < 2 * NSL; r++) w2[r] = 0.0;
+    if (it > 1) {
+#pragma unroll
+      for (int r = 0; r < 2 * NSL; r++) w2[r] = ld(w2p, ln, r);
+    }
     // the converged Newton iterate evaluated kinetics_sl at this (S, xi): rates
     // are in gs.  A NaN rate ends the iteration with the status of the stress
     // integration, as the reference's exit does (phase_mechanical.f90:638)
-    if (dot_state<NSL, QP>(ph, xs, gs, ws)) break;
-    const double* w1p = opaque(cur ? mp.last2 : mp.last1);
-    double* w2p = opaque(cur ? mp.last1 : mp.last2);
-    const bool stf = live_flag(started);
-    const double* x0 = opaque(stf ? mp.st0s : mp.xi0);
-    const double* g0 = opaque(stf ? mp.st0s + NSL * ln.sN : mp.gam0);
+    const bool nan = dot_state<NSL, QP>(ph, gs, ws);
+#pragma unroll
+    for (int r = 0; r < NSL; r++) s0[r] = xi_start(q, r);
+#pragma unroll
+    for (int r = 0; r < NSL; r++) s0[NSL + r] = gam_start(q, r);
     // damper (src/phase_mechanical.f90:653-674)
-    double w1v[2 * NSL];
     double d12 = 0.0, d22 = 0.0, d01 = 0.0;
 #pragma unroll
     for (int r = 0; r < 2 * NSL; r++) {
-      double w1 = ld(w1p, ln, r);
-      double w2 = it > 1 ? ld(w2p, ln, r) : 0.0;
-      double d0 = r < NSL ? ws[r * SWG] : gs[(r - NSL) * SWG];
-      w1v[r] = w1;
-      d12 = fma(d0 - w1, w1 - w2, d12);
-      d22 = fma(w1 - w2, w1 - w2, d22);
-      d01 = fma(d0, w1, d01);
+      const double d0 = r < NSL ? ws[r * SWG] : gs[(r - NSL) * SWG], c = w1[r] - w2[r];
+      d12 = fma(d0 - w1[r], c, d12);
+      d22 = fma(c, c, d22);
+      d01 = fma(d0, w1[r], d01);
     }
-    double zeta = (fmin(d01, d12) < 0.0 && d22 > 0.0) ? 0.75 + 0.25 * tanh_ool(2.0 + 4.0 * d12 / d22) : 1.0;
+    const double zeta = (fmin(d01, d12) < 0.0 && d22 > 0.0) ? 0.75 + 0.25 * tanh_ool(2.0 + 4.0 * d12 / d22) : 1.0;
+    MpPtr q3 = fresh(m);
     bool conv = true;
+    // the next iterate start + dt d, d the damped rate: it differs from the last
+    // one, start + dt w1, by the residual dt (w1 - d).  With a NaN rate the state
+    // stays the last iterate.
 #pragma unroll
     for (int r = 0; r < 2 * NSL; r++) {
-      double w1 = w1v[r];
-      double d0 = r < NSL ? ws[r * SWG] : gs[(r - NSL) * SWG];
-      double d = d0 * zeta + w1 * (1.0 - zeta);
-      st(w2p, ln, r, d);             // dotState_last(:,1) of the next iteration
-      double s0 = r < NSL ? ld(x0, ln, r) : ld(g0, ln, r - NSL);
-      double s = r < NSL ? xs[r * SWG] : ld(mp.gam, ln, r - NSL);
-      double res = s - s0 - d * dt;
-      s = s - res;
-      double atol = r < NSL ? ph->atol_xi : ph->atol_gamma;
-      conv = conv && (fabs(res) <= fmax(atol, num.eps_rel_state * fabs(s)));
-      if (r < NSL) xs[r * SWG] = s; else st(mp.gam, ln, r - NSL, s);
+      const double d0 = r < NSL ? ws[r * SWG] : gs[(r - NSL) * SWG];
+      const double d = nan ? w1[r] : d0 * zeta + w1[r] * (1.0 - zeta);
+      st(w2p, ln, r, d);               // dotState_last(:,1) of the next iteration
+      const double s = fma(d, dt, s0[r]), res = (w1[r] - d) * dt;
+      conv = conv && (fabs(res) <= fmax(r < NSL ? ph->atol_xi : ph->atol_gamma, num.eps_rel_state * fabs(s)));
+      if (r < NSL) {
+        st(q3->xi, ln, r, s);
+        ws[r * SWG] = dmk_rcp(s);      // for the next stress integration
+      } else {
+        st(q3->gam, ln, r - NSL, s);
+      }
     }
     cur = !cur;
-    if (conv) { status = ST_OK; break; }
+    if (nan || conv) return ST_OK;
   }
-  return status;
+  return ST_FAIL_STATE;
 }
 
-// one material point update per lane: block `blk` of the cells of mp
-template <int NSL, bool QP>
-DI void stress_body(const DmkMPDev& mp, const double* __restrict__ Ftarget, const DmkPhaseDev* __restrict__ ph,
-                    int phase_id, const DmkNumMech& num, double dt, int blk, SlipLds<NSL>& sh) {
+// one material point update per lane: block `blk` of the cells of m
+template <int NSL, bool QP, bool NS>
+DI void stress_body(MpPtr m, const double* __restrict__ Ftarget, PhPtr ph, int phase_id,
+                    const DmkNumMech& num, double dt, int blk, SlipLds<NSL>& sh) {
   const int lane = threadIdx.x;
   const int e = blk * SWG + lane;
-  if (e >= mp.N) return;
-  if (mp.phase[e] != phase_id) return;
-  const Lane ln = make_lane(mp.N, e);
-  double* xs = &sh.xi[0][lane];
-  double* sub = mp.sub;
+  if (e >= m->N) return;
+  if (m->phase[e] != phase_id) return;
+  const Lane ln = make_lane(m->N, e);
 
   // isostrain partition (src/homogenization_mechanical_isostrain.f90:60-75)
-  copy9(mp.Fphase, Ftarget, ln);
+  {
+    double F[9];
+    m_load(Ftarget, ln, F);
+    m_store(m->Fphase, ln, F);
+  }
   // start values of the sub-step: those of the converged increment until a
   // sub-step completes (started), then copies in the sub-step scratch / st0s;
   // the initial state rate is taken at S_0 until a sub-step completes, then at
   // the last completed sub-step's S (s_cur)
   bool started = false, s_cur = false;
+  // the last L_p (phase_mechanical_Lp is not restored between calls) and
+  // A = F F_p0^-1 of the sub-step in progress
+  double Lp[9], A[9];
+  m_load(m->Lp, ln, Lp);
+#pragma unroll
+  for (int k = 0; k < 9; k++) A[k] = 0.0;
 
   int newton = 0;
   sh.fpi[lane] = 0;
   sh.nsub[lane] = 0;
-  sh.dt_done[lane] = 0.0;            // time step of the last completed sub-step
   // phase_mechanical_constitutive substepping; the first pass takes the
   // cut-back branch, which is phase_restore (src/phase_mechanical.f90:1096-1115)
   sh.frac[lane] = 0.0;
@@ -493,80 +806,95 @@ DI void stress_body(const DmkMPDev& mp, const double* __restrict__ Ftarget, cons
   bool todo = true;
   while (todo) {
     if (status == ST_OK) {
-      const double stepFrac = sh.frac[lane] + sh.step[lane];
-      const double step = fmin(1.0 - stepFrac, num.r_increase * sh.step[lane]);
+      const double done = sh.step[lane], stepFrac = sh.frac[lane] + done;
+      const double step = fmin(1.0 - stepFrac, num.r_increase * done);
       sh.frac[lane] = stepFrac;
-      sh.step[lane] = step;
       todo = step > 0.0;
       if (todo) {
-        // the completed sub-step's F_p becomes the next one's F_p0
-        finish_point<false>(mp, ln, started ? sub + SUB_FP0 * ln.sN : mp.Fp0, sh.dt_done[lane], sub + SUB_FP0 * ln.sN);
-        copy9(sub + SUB_F0 * ln.sN, sub + SUB_F * ln.sN, ln);
-        copy9(sub + SUB_LP0 * ln.sN, mp.Lp, ln);
+        // the completed sub-step's F, F_p, L_p and state are the next one's start
+        double F[9];
+        sub_F(m, Ftarget, started, ln, done, F);
+        MpPtr q = fresh(m);
+        double* sub = q->sub;
+        finish_point<false>(ph, m, ln, started, A, Lp, done * dt, sub + SUB_FP0 * ln.sN);
+        m_store(sub + SUB_F0 * ln.sN, ln, F);
+        m_store(sub + SUB_LP0 * ln.sN, ln, Lp);
 #pragma unroll 1
         for (int r = 0; r < NSL; r++) {
-          st(mp.st0s, ln, r, xs[r * SWG]);
-          st(mp.st0s, ln, NSL + r, ld(mp.gam, ln, r));
+          st(q->st0s, ln, r, ld(q->xi, ln, r));
+          st(q->st0s, ln, NSL + r, ld(q->gam, ln, r));
         }
+        sh.step[lane] = step;
         started = true;
+        s_cur = true;
       }
     } else {
       // cut back: restore the sub-step start (F_p, S = S_0, L_p for an actual
-      // cut-back, state).  F_p, S and gamma are outputs only until they are
-      // read again, so they are restored where they are read: F_p0 and S come
-      // from the sub-step start / S_0, and gamma is overwritten by the state
-      // integration
+      // cut-back, state).  F_p, S and the state are outputs only until they are
+      // read again, so they are restored where they are read: the state
+      // integration starts from the sub-step start / S_0
       const double step = num.r_cutback * sh.step[lane];
       sh.step[lane] = step;
       s_cur = false;
-      if (step < 1.0) copy9(mp.Lp, started ? sub + SUB_LP0 * ln.sN : mp.Lp0, ln);
-#pragma unroll 1
-      for (int r = 0; r < NSL; r++) xs[r * SWG] = ld(started ? mp.st0s : mp.xi0, ln, r);
+      if (step < 1.0) {
+        MpPtr q = fresh(m);
+        m_load_start(q->Lp0, q->sub + SUB_LP0 * ln.sN, started, ln, Lp);
+      }
       todo = step > num.r_cutback_min;
     }
     if (todo) {
-      const double* pF0 = started ? sub + SUB_F0 * ln.sN : mp.F0;
-#pragma unroll
-      for (int c = 0; c < 9; c++)
-        st(sub + SUB_F * ln.sN, ln, c, fma(sh.step[lane], ld(Ftarget, ln, c) - ld(mp.F0, ln, c), ld(pF0, ln, c)));
-      status = integrate_state_fpi<NSL, QP>(ph, num, mp, ln, started, s_cur, sh.step[lane] * dt, sh, lane, newton);
+      status = integrate_state_fpi<NSL, QP, NS>(ph, num, m, Ftarget, ln, started, s_cur, sh.step[lane],
+                                                sh.step[lane] * dt, sh, lane, newton, A, Lp);
       sh.nsub[lane]++;
-      if (status == ST_OK) {
-        s_cur = true;
-        sh.dt_done[lane] = sh.step[lane] * dt;
-      }
     }
   }
+  MpPtr q = fresh(m);
+  m_store(q->Lp, ln, Lp);
   if (status == ST_OK) {
-    finish_point<true>(mp, ln, started ? sub + SUB_FP0 * ln.sN : mp.Fp0, sh.dt_done[lane], mp.Fp);
+    finish_point<true>(ph, m, ln, started, A, Lp, sh.step[lane] * dt, q->Fp);
   } else {
     // the restored sub-step start, as the last cut-back left it
-    copy9(mp.Fp, started ? sub + SUB_FP0 * ln.sN : mp.Fp0, ln);
-    copy9(mp.S, mp.S0, ln);
+    double T[9];
+    m_load_start(q->Fp0, q->sub + SUB_FP0 * ln.sN, started, ln, T);
+    m_store(q->Fp, ln, T);
+    m_load(q->S0, ln, T);
+    m_store(q->S, ln, T);
 #pragma unroll 1
-    for (int r = 0; r < NSL; r++) st(mp.gam, ln, r, ld(started ? mp.st0s + NSL * ln.sN : mp.gam0, ln, r));
+    for (int r = 0; r < NSL; r++) {
+      st(q->xi, ln, r, ld_start(q->xi0, q->st0s, started, ln, r));
+      st(q->gam, ln, r, ld_start(q->gam0, q->st0s + NSL * ln.sN, started, ln, r));
+    }
   }
-#pragma unroll 1
-  for (int r = 0; r < NSL; r++) st(mp.xi, ln, r, xs[r * SWG]);
-  mp.status[e] = status;
-  mp.n_newton[e] = newton;
-  mp.n_fpi[e] = sh.fpi[lane];
-  mp.n_sub[e] = sh.nsub[lane];
+  MpPtr q4 = fresh(m);
+  q4->status[e] = status;
+  q4->n_newton[e] = newton;
+  q4->n_fpi[e] = sh.fpi[lane];
+  q4->n_sub[e] = sh.nsub[lane];
 }
 
-template <int NSL, bool QP>
-__global__ void __launch_bounds__(SWG) __attribute__((amdgpu_waves_per_eu(DMK_STRESS_WAVES)))
-stress_kernel(DmkMPDev mp, const double* __restrict__ Ftarget, const DmkPhaseDev* __restrict__ ph, int phase_id,
-              DmkNumMech num, double dt) {
+// the arguments of stress_kernel, read through its kernel-argument segment
+struct StressArgs {
+  DmkMPDev mp;
+  const double* F;
+  const DmkPhaseDev* ph;
+  DmkNumMech num;
+  double dt;
+  int phase_id;
+};
+
+template <int NSL, bool QP, bool NS>
+__global__ void __launch_bounds__(SWG) __attribute__((amdgpu_waves_per_eu(stress_waves(NSL))))
+stress_kernel(StressArgs a) {
   __shared__ SlipLds<NSL> sh;
-  stress_body<NSL, QP>(mp, Ftarget, ph, phase_id, num, dt, blockIdx.x, sh);
+  MpPtr m = (MpPtr)__builtin_amdgcn_kernarg_segment_ptr();   // a.mp, the first argument's first member
+  stress_body<NSL, QP, NS>(m, a.F, (PhPtr)a.ph, a.phase_id, a.num, a.dt, blockIdx.x, sh);
 }
 
 // The stress integration of several RVEs (and phases) in one launch: item i
 // owns blocks [block0_i, block0_{i+1}) and runs them on its own material
 // point, phase tables, load and time step, exactly as stress_kernel would.
-template <int NSL, bool QP>
-__global__ void __launch_bounds__(SWG) __attribute__((amdgpu_waves_per_eu(DMK_STRESS_WAVES)))
+template <int NSL, bool QP, bool NS>
+__global__ void __launch_bounds__(SWG) __attribute__((amdgpu_waves_per_eu(stress_waves(NSL))))
 stress_kernel_batch(const DmkStressItem* __restrict__ items, int n_items) {
   __shared__ SlipLds<NSL> sh;
   const int b = blockIdx.x;
@@ -576,9 +904,9 @@ stress_kernel_batch(const DmkStressItem* __restrict__ items, int n_items) {
     if (items[mid].block0 <= b) lo = mid; else hi = mid - 1;
   }
   const DmkStressItem* it = items + lo;
-  const DmkMPDev mp = it->mp;
   const DmkNumMech num = it->num;
-  stress_body<NSL, QP>(mp, it->F, it->ph, it->phase_id, num, it->dt, b - it->block0, sh);
+  stress_body<NSL, QP, NS>((MpPtr)&it->mp, it->F, (PhPtr)it->ph,
+                           it->phase_id, num, it->dt, b - it->block0, sh);
 }
 
 // math_rotationalPart (src/math.f90:1004-1043)
@@ -655,19 +983,25 @@ DI void row3(const double* M, int r, double* v) {
 // v = 1) for a response in which every cell converged (flag[0] == ST_OK).
 // Also writes the squared Frobenius norm of each cell's dPdF, summed in
 // Fortran element order (the C_minMaxAvg selection works on it).
-template <int NSL, bool QP>
-__global__ void __launch_bounds__(SWG) tangent_kernel(DmkMPDev mp, const DmkPhaseDev* __restrict__ ph,
+//
+// Column (k, l): dS = dS/dF_kl solves dS + dt sum_a dg_a C:sym(G2 P_a) (P_nS_a : dS)
+// = C:sym(X), X = F_e(k,:) (x) F_p^-1(l,:), G2 = F_e^T A2.  As in the stress
+// integration the sum acts through the E coordinates z of dS alone: N z = E:X with
+// N_kl = delta_kl / C_k + dt E_k : (G2 W_l), one 5x5 (6x6) factorisation for the
+// nine columns; then t = sum_a dg_a P_a (P_nS_a : dS) = sum_l z_l W_l and
+// dS = C:sym(X - dt G2 t), without a loop over the slip systems per column.
+template <int NSL, bool QP, bool NS>
+__global__ void __launch_bounds__(SWG) tangent_kernel(DmkMPDev mp, const DmkPhaseDev* __restrict__ ph_,
                                                       int phase_id, double dt, const int* __restrict__ flag,
                                                       double* __restrict__ dPdF, double* __restrict__ nrm) {
-  __shared__ SlipLds<NSL> sh;
+  constexpr int RK = sym_rank<NS>();
+  PhPtr ph = (PhPtr)ph_;
+  __shared__ double ixi[NSL][SWG], gl[NSL][SWG];
   const int lane = threadIdx.x;
   const int e = blockIdx.x * SWG + lane;
   if (e >= mp.N || flag[0] != ST_OK) return;
   if (mp.phase[e] != phase_id) return;
   const Lane ln = make_lane(mp.N, e);
-  double* xs = &sh.xi[0][lane];
-  double* gs = &sh.g[0][lane];
-  double* ws = &sh.w[0][lane];
   double Fe[9];
   m_load(mp.Fe, ln, Fe);
   {
@@ -678,131 +1012,93 @@ __global__ void __launch_bounds__(SWG) tangent_kernel(DmkMPDev mp, const DmkPhas
 #pragma unroll
     for (int k = 0; k < 4; k++) st(mp.O, ln, k, q[k]);
   }
-#pragma unroll 1
-  for (int r = 0; r < NSL; r++) xs[r * SWG] = ld(mp.xi, ln, r);
+  double H[5][RK], K[3][RK];
   {
-    double S[9];
+    double S[9], s[6], l[5], k3[3];
+    unsigned posm;
+#pragma unroll 4
+    for (int r = 0; r < NSL; r++) ixi[r][lane] = 1.0 / ld(mp.xi, ln, r);
     m_load(mp.S, ln, S);
-    kinetics<NSL, QP, true, false>(ph, S, xs, gs, ws, nullptr);
+    sym_proj<RK>(S, s);
+    kinetics<NSL, QP, NS, true>(ph, s, &ixi[0][lane], &gl[0][lane], l, k3, posm);
+    slip_moments<NSL, NS>(ph, &gl[0][lane], 1.0, posm, H, K);
   }
-  const bool nonschmid = ph->nonschmid;
-
-  double invFp[9], invSubFp0[9], A2[9];
+  double invFp[9], invSubFp0[9], F[9], G2[9];
   {
-    double Fp[9], Fp0[9], F[9];
+    double Fp[9], Fp0[9], A2[9];
     m_load(mp.Fp, ln, Fp);
     m_load(mp.Fp0, ln, Fp0);
     m_load(mp.Fphase, ln, F);
     m_invert(Fp, invFp);
     m_invert(Fp0, invSubFp0);
     m_mul(F, invSubFp0, A2);
-  }
-  // K = I9 + dt sum_a dg_a vec(C:sym(G2 P_a)) vec(Pn_a)^T,  G2 = F_e^T A2
-  double K[81];
-  {
-    double G2[9];
     m_mul_tn(Fe, A2, G2);
 #pragma unroll
-    for (int r = 0; r < 81; r++) K[r] = (r % 10 == 0) ? 1.0 : 0.0;
-#pragma unroll 1
-    for (int a = 0; a < NSL; a++) {
-      double X[9], Xs[9], W[9];
-      m_mul(G2, ph->P[a], X);
-#pragma unroll
-      for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) Xs[3 * i + j] = 0.5 * (X[3 * i + j] + X[3 * j + i]);
-      hooke_sym(ph->C11, ph->C12, ph->C44, Xs, W);
-      const bool pos = gs[a * SWG] > 0.0;
-      double u = dt * ws[a * SWG];
-      if (nonschmid) {
-        double Pn[9];
-#pragma unroll
-        for (int c = 0; c < 9; c++) Pn[c] = pos ? ph->Pp[a][c] : ph->Pm[a][c];
-#pragma unroll
-        for (int r = 0; r < 9; r++) {
-          double wr = u * W[r];
-#pragma unroll
-          for (int c = 0; c < 9; c++) K[9 * r + c] = fma(wr, Pn[c], K[9 * r + c]);
-        }
-      } else {
-        u = pos ? u : -u;            // Schmid law: P_nS,neg = -P_nS,pos exactly
-#pragma unroll
-        for (int r = 0; r < 9; r++) {
-          double wr = u * W[r];
-#pragma unroll
-          for (int c = 0; c < 9; c++) K[9 * r + c] = fma(wr, ph->Pp[a][c], K[9 * r + c]);
-        }
-      }
-    }
+    for (int q = 0; q < 9; q++) G2[q] *= dt;
   }
-  double v0[9], tau[9];
-  const bool sing = dmk_qr_factor<9>(K, v0, tau);
+  double N[RK * RK], rd[RK], v0[RK], tau[RK];
+  reduced_matrix<RK>(ph, G2, H, K, N);
+  const bool sing = dmk_qr_factor<RK>(N, rd, v0, tau);
 
-  double M1[9], M2[9], M3[9], Mid[9];
-  {
-    double S[9], F[9];
-    m_load(mp.S, ln, S);
-    m_load(mp.Fphase, ln, F);
-    m_mul_nt(S, invFp, M1);        // S invFp^T
-    m_mul(F, invFp, M2);           // F invFp
-    m_mul(M2, S, M3);              // F invFp S
-    m_mul(invFp, M1, Mid);         // invFp S invFp^T
-  }
+  double S[9], M1[9], Mid[9];
+  m_load(mp.S, ln, S);
+  m_mul_nt(S, invFp, M1);          // S invFp^T
+  m_mul(invFp, M1, Mid);           // invFp S invFp^T
   double n2 = 0.0;
 #pragma unroll 1
   for (int l = 0; l < 3; l++) {
 #pragma unroll 1
     for (int k = 0; k < 3; k++) {
-      // rhs column: C : sym(Fe(k,:) (x) invFp(l,:))
       double fk[3], pl[3], ml[3];
       row3(Fe, k, fk);
       row3(invFp, l, pl);
       row3(Mid, l, ml);
-      double X[9], y[9];
+      double X[9], z[6], t[9], y[9], D[9];
 #pragma unroll
       for (int n = 0; n < 3; n++)
 #pragma unroll
-        for (int m = 0; m < 3; m++) X[3 * n + m] = 0.5 * (fk[n] * pl[m] + fk[m] * pl[n]);
-      hooke_sym(ph->C11, ph->C12, ph->C44, X, y);
-      if (!sing) dmk_qr_apply_solve<9>(K, v0, tau, y);
-      // t = sum_a dg_a P_a (Pn_a : dSdF)
-      double t[9];
+        for (int m = 0; m < 3; m++) X[3 * n + m] = fk[n] * pl[m];
+      sym_proj<RK>(X, z);
+      if (!sing) {
+        dmk_qr_apply_solve<RK>(N, rd, v0, tau, z);
+      } else {                     // as after a failed solve: dS = C:sym(X)
 #pragma unroll
-      for (int q = 0; q < 9; q++) t[q] = 0.0;
-#pragma unroll 1
-      for (int a = 0; a < NSL; a++) {
-        const bool pos = gs[a * SWG] > 0.0;
-        double c = 0.0;
-        if (nonschmid) {
-#pragma unroll
-          for (int q = 0; q < 9; q++) c = fma(pos ? ph->Pp[a][q] : ph->Pm[a][q], y[q], c);
-        } else {
-#pragma unroll
-          for (int q = 0; q < 9; q++) c = fma(ph->Pp[a][q], y[q], c);
-          c = pos ? c : -c;
-        }
-        c *= ws[a * SWG];
-#pragma unroll
-        for (int q = 0; q < 9; q++) t[q] = fma(c, ph->P[a][q], t[q]);
+        for (int q = 0; q < RK; q++) z[q] *= modulus<RK>(ph, q);
       }
-      // dFpinv = -dt invSubFp0 t;  F dFpinv = -dt A2 t
-      double D[9], AD[9];
-      m_mul(invSubFp0, t, D);
-      m_mul(A2, t, AD);
+      moments_apply<RK>(H, K, z, t);
+      {
+        double Gt[9], Xs[9];
+        m_mul(G2, t, Gt);
+        if (!sing) {
 #pragma unroll
-      for (int q = 0; q < 9; q++) { D[q] = -D[q] * dt; AD[q] = -AD[q] * dt; }
-      double R2[9], R3[9], R4[9], R1[9], col[9];
-      m_mul(AD, M1, R2);            // F dFpinv S invFp^T
-      m_mul(M2, y, R3);
-      m_mul_nt(R3, invFp, R4);      // F invFp dSdF invFp^T
-      m_mul_nt(M3, D, R1);          // F invFp S dFpinv^T
+          for (int q = 0; q < 9; q++) X[q] -= Gt[q];
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+          for (int j = 0; j < 3; j++) Xs[3 * i + j] = 0.5 * (X[3 * i + j] + X[3 * j + i]);
+        hooke_sym(ph->C11, ph->C12, ph->C44, Xs, y);
+      }
+      // d(F_p^-1) = D = -dt invSubFp0 t and
+      // dP = e_k (x) Mid(l,:) + F (D S F_p^-T + F_p^-1 (dS F_p^-T + S D^T))
+      m_mul(invSubFp0, t, D);
+#pragma unroll
+      for (int q = 0; q < 9; q++) D[q] *= -dt;
+      double T1[9], T2[9], col[9];
+      m_mul_nt(y, invFp, T1);
+      m_mul_nt(S, D, T2);
+#pragma unroll
+      for (int q = 0; q < 9; q++) T1[q] += T2[q];
+      m_mul(invFp, T1, T2);
+      m_mul(D, M1, T1);
+#pragma unroll
+      for (int q = 0; q < 9; q++) T1[q] += T2[q];
+      m_mul(F, T1, col);
 #pragma unroll
       for (int i = 0; i < 3; i++)
+        if (i == k) {
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-          double base = (i == k) ? ml[j] : 0.0;
-          col[3 * i + j] = base + R2[3 * i + j] + R4[3 * i + j] + R1[3 * i + j];
+          for (int j = 0; j < 3; j++) col[3 * i + j] += ml[j];
         }
 #pragma unroll
       for (int j = 0; j < 3; j++)
@@ -820,62 +1116,64 @@ __global__ void __launch_bounds__(SWG) tangent_kernel(DmkMPDev mp, const DmkPhas
 }  // namespace
 
 // ---------------------------------------------------------------------------- launchers
-template <int NSL, bool QP>
-static void launch_stress(const DmkMPDev* mp, const double* Ftarget, const DmkPhaseDev* ph, int phase_id,
-                          const DmkNumMech* num, double dt, hipStream_t s) {
-  dim3 blk(SWG), grd((mp->N + SWG - 1) / SWG);
-  hipLaunchKernelGGL((stress_kernel<NSL, QP>), grd, blk, 0, s, *mp, Ftarget, ph, phase_id, *num, dt);
+namespace {
+
+// f(slip systems, quarter powers, non-Schmid terms) with compile-time arguments
+// for a variant = nsl (+ DMK_SYS_NONSCHMID); false when there is no such kernel
+template <bool B>
+struct Flag { static constexpr bool value = B; };
+template <int N>
+struct Count { static constexpr int value = N; };
+
+template <class Fn>
+bool for_variant(int variant, bool qp, Fn&& f) {
+  auto pick = [&](auto n) {
+    const bool ns = variant >= DMK_SYS_NONSCHMID;
+    if (qp) ns ? f(n, Flag<true>{}, Flag<true>{}) : f(n, Flag<true>{}, Flag<false>{});
+    else ns ? f(n, Flag<false>{}, Flag<true>{}) : f(n, Flag<false>{}, Flag<false>{});
+  };
+  switch (variant % DMK_SYS_NONSCHMID) {
+    case 12: pick(Count<12>{}); return true;
+    case 24: pick(Count<24>{}); return true;
+    default: return false;
+  }
 }
 
-template <int NSL, bool QP>
-static void launch_tangent(const DmkMPDev* mp, const DmkPhaseDev* ph, int phase_id, double dt, const int* flag,
-                           double* dPdF, double* nrm, hipStream_t s) {
-  dim3 blk(SWG), grd((mp->N + SWG - 1) / SWG);
-  hipLaunchKernelGGL((tangent_kernel<NSL, QP>), grd, blk, 0, s, *mp, ph, phase_id, dt, flag, dPdF, nrm);
-}
+}  // namespace
 
 extern "C" int dmk_launch_stress(const DmkMPDev* mp, const double* Ftarget, const DmkPhaseDev* ph,
                                  const DmkPhaseDev* ph_host, int phase_id, const DmkNumMech* num, double dt,
                                  hipStream_t s) {
-  const bool qp = ph_host->quarter_pow != 0;
-  switch (ph_host->nsl) {
-    case 12: qp ? launch_stress<12, true>(mp, Ftarget, ph, phase_id, num, dt, s)
-                : launch_stress<12, false>(mp, Ftarget, ph, phase_id, num, dt, s); break;
-    case 24: qp ? launch_stress<24, true>(mp, Ftarget, ph, phase_id, num, dt, s)
-                : launch_stress<24, false>(mp, Ftarget, ph, phase_id, num, dt, s); break;
-    default: return 1;
-  }
+  const dim3 blk(SWG), grd((mp->N + SWG - 1) / SWG);
+  const bool known = for_variant(dmk_sys_variant(ph_host), ph_host->quarter_pow != 0, [&](auto n, auto qp, auto ns) {
+    hipLaunchKernelGGL((stress_kernel<decltype(n)::value, decltype(qp)::value, decltype(ns)::value>), grd, blk, 0, s,
+                       StressArgs{*mp, Ftarget, ph, *num, dt, phase_id});
+  });
+  if (!known) return 1;
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
-extern "C" int dmk_launch_stress_batch(const DmkStressItem* items_dev, int n_items, int n_blocks, int nsl,
+extern "C" int dmk_launch_stress_batch(const DmkStressItem* items_dev, int n_items, int n_blocks, int variant,
                                        int quarter_pow, hipStream_t s) {
   if (n_items < 1 || n_blocks < 1) return 0;
-  dim3 blk(SWG), grd(n_blocks);
-  if (nsl == 12 && quarter_pow)
-    hipLaunchKernelGGL((stress_kernel_batch<12, true>), grd, blk, 0, s, items_dev, n_items);
-  else if (nsl == 12)
-    hipLaunchKernelGGL((stress_kernel_batch<12, false>), grd, blk, 0, s, items_dev, n_items);
-  else if (nsl == 24 && quarter_pow)
-    hipLaunchKernelGGL((stress_kernel_batch<24, true>), grd, blk, 0, s, items_dev, n_items);
-  else if (nsl == 24)
-    hipLaunchKernelGGL((stress_kernel_batch<24, false>), grd, blk, 0, s, items_dev, n_items);
-  else
-    return 1;
+  const dim3 blk(SWG), grd(n_blocks);
+  const bool known = for_variant(variant, quarter_pow != 0, [&](auto n, auto qp, auto ns) {
+    hipLaunchKernelGGL((stress_kernel_batch<decltype(n)::value, decltype(qp)::value, decltype(ns)::value>), grd, blk,
+                       0, s, items_dev, n_items);
+  });
+  if (!known) return 1;
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
 extern "C" int dmk_launch_tangent(const DmkMPDev* mp, const DmkPhaseDev* ph, const DmkPhaseDev* ph_host,
                                   int phase_id, double dt, const int* flag, double* dPdF, double* nrm,
                                   hipStream_t s) {
-  const bool qp = ph_host->quarter_pow != 0;
-  switch (ph_host->nsl) {
-    case 12: qp ? launch_tangent<12, true>(mp, ph, phase_id, dt, flag, dPdF, nrm, s)
-                : launch_tangent<12, false>(mp, ph, phase_id, dt, flag, dPdF, nrm, s); break;
-    case 24: qp ? launch_tangent<24, true>(mp, ph, phase_id, dt, flag, dPdF, nrm, s)
-                : launch_tangent<24, false>(mp, ph, phase_id, dt, flag, dPdF, nrm, s); break;
-    default: return 1;
-  }
+  const dim3 blk(SWG), grd((mp->N + SWG - 1) / SWG);
+  const bool known = for_variant(dmk_sys_variant(ph_host), ph_host->quarter_pow != 0, [&](auto n, auto qp, auto ns) {
+    hipLaunchKernelGGL((tangent_kernel<decltype(n)::value, decltype(qp)::value, decltype(ns)::value>), grd, blk, 0, s,
+                       *mp, ph, phase_id, dt, flag, dPdF, nrm);
+  });
+  if (!known) return 1;
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 

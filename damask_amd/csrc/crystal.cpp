@@ -178,12 +178,34 @@ int dmk_build_phase(const dmk_phase_desc* d, DmkPhaseDev* p) {
         }
     }
   }
+  // traceless basis of the per-cell kernels: E_1 = diag(1,-1,0)/sqrt2,
+  // E_2 = diag(1,1,-2)/sqrt6, then symmetric and skew pairs (12), (02), (01)
+  // over sqrt2; E_6 = I/sqrt3
+  const double r2 = std::sqrt(0.5), r3 = std::sqrt(1.0 / 3.0), r6 = std::sqrt(1.0 / 6.0);
+  auto sym6 = [&](const double* X, double* o) {
+    o[0] = (X[0] - X[4]) * r2;
+    o[1] = (X[0] + X[4] - 2.0 * X[8]) * r6;
+    o[2] = (X[5] + X[7]) * r2;
+    o[3] = (X[2] + X[6]) * r2;
+    o[4] = (X[1] + X[3]) * r2;
+    o[5] = (X[0] + X[4] + X[8]) * r3;
+  };
+  for (int a = 0; a < nsl; a++) {
+    double o[6];
+    sym6(p->P[a], o);
+    for (int k = 0; k < 5; k++) p->sp[a][k] = o[k];
+    p->sp[a][5] = (p->P[a][5] - p->P[a][7]) * r2;
+    p->sp[a][6] = (p->P[a][2] - p->P[a][6]) * r2;
+    p->sp[a][7] = (p->P[a][1] - p->P[a][3]) * r2;
+    sym6(p->Pp[a], p->qp[a]);
+    sym6(p->Pm[a], p->qm[a]);
+  }
   // interaction (reacting r, acting a)
   for (int r = 0; r < nsl; r++)
     for (int a = 0; a < nsl; a++) {
       int t = d->lattice == 0 ? CF_INT[used[r]][used[a]] : CI_INT[used[r]][used[a]];
       if (t > d->n_h) return 5;
-      p->H[r][a] = d->h_sl_sl[t - 1];
+      p->H[r][a] = p->Hc[a][r] = d->h_sl_sl[t - 1];
       p->Ht[r][a] = t - 1;
     }
   p->n_h = d->n_h;
@@ -192,6 +214,7 @@ int dmk_build_phase(const dmk_phase_desc* d, DmkPhaseDev* p) {
     for (int s = 0; s < d->N_sl[f]; s++, a++) {
       p->g0[a] = d->dot_gamma_0[f];
       p->n[a] = d->n[f];
+      p->inv_n[a] = 1.0 / d->n[f];
       p->a[a] = d->a[f];
       p->h0[a] = d->h_0[f];
       p->xi_inf[a] = d->xi_inf[f];
@@ -199,12 +222,19 @@ int dmk_build_phase(const dmk_phase_desc* d, DmkPhaseDev* p) {
       p->c2[a] = d->c_2[f];
       p->fsat[a] = d->f_sat[f];
       p->xi_sat[a] = d->xi_inf[f] + d->f_sat[f] * std::sqrt(0.0);
+      p->inv_xi_sat[a] = 1.0 / p->xi_sat[a];
       p->hf[a] = d->h_0[f] * (1.0 + d->c_1[f] * std::pow(0.0, d->c_2[f]));
     }
   p->quarter_pow = 1;
   for (int b = 0; b < nsl; b++)
     for (double y : {p->n[b], p->a[b]})
       if (!(y > 0.0 && y <= 64.0 && y * 4.0 == std::rint(y * 4.0))) p->quarter_pow = 0;
+  p->n_k = p->quarter_pow && p->n[0] >= 1.0 ? (int)(4.0 * p->n[0]) : 0;
+  p->a_k = p->quarter_pow ? (int)(4.0 * p->a[0]) : 0;
+  for (int b = 1; b < nsl; b++) {
+    if (p->n[b] != p->n[0]) p->n_k = 0;
+    if (p->a[b] != p->a[0]) p->a_k = 0;
+  }
   p->atol_xi = d->atol_xi;
   p->atol_gamma = d->atol_gamma;
   return 0;

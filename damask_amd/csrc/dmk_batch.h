@@ -9,7 +9,7 @@ struct DmkStressItem;
 struct dmk_handle;
 
 // Hand the stress integration of one residual evaluation (its items: one per
-// phase, key = 2 nsl + quarter_pow) to the batch.  Called from the RVE's own
+// phase, key = 2 dmk_sys_variant + quarter_pow) to the batch.  Called from the RVE's own
 // host thread after its input F has been enqueued on `st`; returns once the
 // batched launch holding these items is enqueued, with `st` made to wait for
 // it.  Blocks until every RVE of the batch still running has submitted.

@@ -13,7 +13,7 @@
 #define DMK_NSL_MAX 24
 #define DMK_MAX_PHASES 8
 #define DMK_STRESS_WG 64       // work-group (one wavefront) of the per-cell kernels
-#define DMK_SUB_ROWS 54        // rows of the per-cell stress-integration scratch (DmkMPDev::sub)
+#define DMK_SUB_ROWS 27        // rows of the per-cell stress-integration scratch (DmkMPDev::sub)
 
 #define DMK_CHECK(x)                                                                   \
   do {                                                                                 \
@@ -53,23 +53,35 @@ struct DmkPhaseDev {
   int nsl;
   int nonschmid;                    // P_nS_neg differs from -P_nS_pos
   int quarter_pow;                  // every n_sl and a_sl is a positive multiple of 1/4, <= 64
+  int n_k;                          // 4 n where quarter_pow and all systems share one n >= 1, else 0
+  int a_k;                          // 4 a where quarter_pow and all systems share one a, else 0
   double C11, C12, C44;             // cubic stiffness (Voigt constants), lattice frame
   double P[DMK_NSL_MAX][9];         // Schmid tensor d (x) n
   double Pp[DMK_NSL_MAX][9];        // non-Schmid projection, positive sense
   double Pm[DMK_NSL_MAX][9];        // non-Schmid projection, negative sense
   double Qp[DMK_NSL_MAX][9];        // C : Pp
   double Qm[DMK_NSL_MAX][9];        // C : Pm
+  // coordinates in the traceless basis of the per-cell kernels: E_1..E_5 and
+  // R_1..R_3 of P; E_1..E_6 of Pp and Pm
+  double sp[DMK_NSL_MAX][8];
+  double qp[DMK_NSL_MAX][6], qm[DMK_NSL_MAX][6];
   double H[DMK_NSL_MAX][DMK_NSL_MAX];  // H[reacting][acting]
-  double g0[DMK_NSL_MAX], n[DMK_NSL_MAX], a[DMK_NSL_MAX], h0[DMK_NSL_MAX];
+  double Hc[DMK_NSL_MAX][DMK_NSL_MAX]; // the same by [acting][reacting]
+  double g0[DMK_NSL_MAX], n[DMK_NSL_MAX], inv_n[DMK_NSL_MAX], a[DMK_NSL_MAX], h0[DMK_NSL_MAX];
   double xi_inf[DMK_NSL_MAX], c1[DMK_NSL_MAX], c2[DMK_NSL_MAX], fsat[DMK_NSL_MAX];
   // without twins (sum F_tw = 0): xi_inf + f_sat sqrt(0) and h_0 (1 + c_1 0^c_2)
-  double xi_sat[DMK_NSL_MAX], hf[DMK_NSL_MAX];
+  double xi_sat[DMK_NSL_MAX], inv_xi_sat[DMK_NSL_MAX], hf[DMK_NSL_MAX];
   double atol_xi, atol_gamma;
   // interaction type (index into h_sl_sl) of H[reacting][acting]: parameter
   // cotangents of the adjoint
   int n_h;
   int32_t Ht[DMK_NSL_MAX][DMK_NSL_MAX];
 };
+
+// kernel variant of a phase in the batched stress launches: its slip systems,
+// plus this when non-Schmid terms act
+#define DMK_SYS_NONSCHMID 64
+inline int dmk_sys_variant(const DmkPhaseDev* ph) { return ph->nsl + (ph->nonschmid ? DMK_SYS_NONSCHMID : 0); }
 
 struct DmkNumMech {
   double r_cutback_min, r_cutback, r_increase, eps_rel_state;
@@ -107,7 +119,7 @@ struct DmkMPDev {
   double* st0s;                  // state at the start of the sub-step (after the first sub-step)
   double* last1;                 // state-rate history, ping-pong pair
   double* last2;
-  double* sub;                   // [DMK_SUB_ROWS][N]: sub-step F_0, F, F_p0, L_p0, line-search state
+  double* sub;                   // [DMK_SUB_ROWS][N]: F, F_p, L_p of the last completed sub-step
 };
 
 // one (RVE, phase) of a batched stress launch (stress_kernel_batch)

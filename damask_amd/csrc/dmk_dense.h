@@ -10,110 +10,75 @@
 // gives the same solution to rounding; that is what is used here.
 //
 // Singularity: a column whose remaining part is exactly zero makes R
-// singular; the functions then report failure, as dgesv reports info > 0
+// singular; the factorisation then reports failure, as dgesv reports info > 0
 // for an exactly zero pivot.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
-#define DMK_HD __host__ __device__ __forceinline__
+#define DMK_DENSE __device__ __forceinline__
 
-// Reflector for column k: H = I - tau v v^T with v = (v0, x_{k+1..n-1}),
-// H x = beta e_k.  Returns (beta, v0, tau); nrm == 0 flags a zero column.
-struct DmkHouse {
-  double beta, v0, tau;
-  bool zero;
-};
-
-template <int n>
-DMK_HD DmkHouse dmk_house(const double* J, int k) {
-  double alpha = J[n * k + k];
-  double sigma = 0.0;
-#pragma unroll
-  for (int i = k + 1; i < n; i++) sigma = fma(J[n * i + k], J[n * i + k], sigma);
-  double nrm = sqrt(fma(alpha, alpha, sigma));
-  DmkHouse h;
-  h.beta = alpha >= 0.0 ? -nrm : nrm;
-  h.v0 = alpha - h.beta;                 // |v0| = |alpha| + nrm: no cancellation
-  h.tau = -1.0 / (h.beta * h.v0);        // 2 / (v^T v)
-  h.zero = !(nrm > 0.0);
-  return h;
+// 1/x and 1/sqrt(x): the hardware approximation and two Newton steps each
+// (within 1 and 2 ulp for normal results), without the scaling and fix-up
+// sequences of a division and a square root.  An n = 5 factorisation has 5 of
+// each in one dependent chain.
+DMK_DENSE double dmk_rcp(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
 }
 
-// Solve J x = b in place (J destroyed, x returned in b).  Returns true when
-// J is singular (the contents of b are then undefined).
+DMK_DENSE double dmk_rsq(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  const double h = 0.5 * x;
+  y = fma(y, fma(-h * y, y, 0.5), y);
+  return fma(y, fma(-h * y, y, 0.5), y);
+}
+
+// Factorisation J = Q R in place: R in the upper triangle without its diagonal,
+// reflector tails below it; per column k the inverse diagonal of R in rd and
+// the reflector I - tau v v^T with v = (v0, tail).  Returns true when J is
+// singular.
 template <int n>
-DMK_HD bool dmk_qr_solve(double* J, double* b) {
+DMK_DENSE bool dmk_qr_factor(double* J, double* rd, double* v0, double* tau) {
   bool sing = false;
 #pragma unroll
   for (int k = 0; k < n; k++) {
-    DmkHouse h = dmk_house<n>(J, k);
-    sing |= h.zero;
+    const double alpha = J[n * k + k];
+    double s2 = alpha * alpha;
+#pragma unroll
+    for (int i = k + 1; i < n; i++) s2 = fma(J[n * i + k], J[n * i + k], s2);
+    sing |= !(s2 > 0.0);
+    const double rn = dmk_rsq(s2), nrm = s2 * rn;
+    // beta = -sign(alpha) |column|, v0 = alpha - beta (no cancellation),
+    // tau = 2 / (v^T v) = -1 / (beta v0)
+    const double av = fabs(alpha) + nrm;
+    v0[k] = copysign(av, alpha);
+    tau[k] = rn * dmk_rcp(av);
+    rd[k] = -copysign(rn, alpha);
 #pragma unroll
     for (int j = k + 1; j < n; j++) {
-      double w = h.v0 * J[n * k + j];
+      double w = v0[k] * J[n * k + j];
 #pragma unroll
       for (int i = k + 1; i < n; i++) w = fma(J[n * i + k], J[n * i + j], w);
-      double s = h.tau * w;
-      J[n * k + j] = fma(-s, h.v0, J[n * k + j]);
+      const double s = tau[k] * w;
+      J[n * k + j] = fma(-s, v0[k], J[n * k + j]);
 #pragma unroll
       for (int i = k + 1; i < n; i++) J[n * i + j] = fma(-s, J[n * i + k], J[n * i + j]);
     }
-    {
-      double w = h.v0 * b[k];
-#pragma unroll
-      for (int i = k + 1; i < n; i++) w = fma(J[n * i + k], b[i], w);
-      double s = h.tau * w;
-      b[k] = fma(-s, h.v0, b[k]);
-#pragma unroll
-      for (int i = k + 1; i < n; i++) b[i] = fma(-s, J[n * i + k], b[i]);
-    }
-    J[n * k + k] = h.beta;
-  }
-#pragma unroll
-  for (int k = n - 1; k >= 0; k--) {
-    double s = b[k];
-#pragma unroll
-    for (int j = k + 1; j < n; j++) s = fma(-J[n * k + j], b[j], s);
-    b[k] = s / J[n * k + k];
   }
   return sing;
 }
 
-// Factorisation kept for several right-hand sides: R in the upper triangle
-// (diagonal = beta), reflector tails below it, v0 and tau per column.
+// J x = b for a factorised J, x returned in b
 template <int n>
-DMK_HD bool dmk_qr_factor(double* J, double* v0, double* tau) {
-  bool sing = false;
-#pragma unroll
-  for (int k = 0; k < n; k++) {
-    DmkHouse h = dmk_house<n>(J, k);
-    sing |= h.zero;
-#pragma unroll
-    for (int j = k + 1; j < n; j++) {
-      double w = h.v0 * J[n * k + j];
-#pragma unroll
-      for (int i = k + 1; i < n; i++) w = fma(J[n * i + k], J[n * i + j], w);
-      double s = h.tau * w;
-      J[n * k + j] = fma(-s, h.v0, J[n * k + j]);
-#pragma unroll
-      for (int i = k + 1; i < n; i++) J[n * i + j] = fma(-s, J[n * i + k], J[n * i + j]);
-    }
-    J[n * k + k] = h.beta;
-    v0[k] = h.v0;
-    tau[k] = h.tau;
-  }
-  return sing;
-}
-
-template <int n>
-DMK_HD void dmk_qr_apply_solve(const double* J, const double* v0, const double* tau, double* b) {
+DMK_DENSE void dmk_qr_apply_solve(const double* J, const double* rd, const double* v0, const double* tau, double* b) {
 #pragma unroll
   for (int k = 0; k < n; k++) {
     double w = v0[k] * b[k];
 #pragma unroll
     for (int i = k + 1; i < n; i++) w = fma(J[n * i + k], b[i], w);
-    double s = tau[k] * w;
+    const double s = tau[k] * w;
     b[k] = fma(-s, v0[k], b[k]);
 #pragma unroll
     for (int i = k + 1; i < n; i++) b[i] = fma(-s, J[n * i + k], b[i]);
@@ -123,6 +88,6 @@ DMK_HD void dmk_qr_apply_solve(const double* J, const double* v0, const double* 
     double s = b[k];
 #pragma unroll
     for (int j = k + 1; j < n; j++) s = fma(-J[n * k + j], b[j], s);
-    b[k] = s / J[n * k + k];
+    b[k] = s * rd[k];
   }
 }

@@ -149,11 +149,12 @@ DHI bool m_invert(const double* A, double* inv) {
   return false;
 }
 
-DHI double m_norm(const double* A) {
+// squared Frobenius norm
+DHI double m_norm2(const double* A) {
   double s = 0.0;
 #pragma unroll
   for (int k = 0; k < 9; k++) s = fma(A[k], A[k], s);
-  return sqrt(s);
+  return s;
 }
 
 // C : X for cubic stiffness in the lattice frame, X symmetric, through the

@@ -364,7 +364,7 @@ static int response_enqueue(dmk_handle* h, const double* F, double dt, const Aim
     int key[DMK_MAX_PHASES];
     for (int p = 0; p < h->n_phases; p++) {
       items[p] = DmkStressItem{h->mp, F, h->ph_dev + p, h->nm, dt, p, 0};
-      key[p] = 2 * h->ph[p].nsl + (h->ph[p].quarter_pow ? 1 : 0);
+      key[p] = 2 * dmk_sys_variant(&h->ph[p]) + (h->ph[p].quarter_pow ? 1 : 0);
     }
     int rc = dmk_stress_batch_submit(h->batch, h->batch_slot, items, key, h->n_phases, h->st);
     if (rc) return rc;
@@ -638,7 +638,7 @@ static int residual_lockstep(dmk_handle* h, const DotJobs* jobs, double* dots_ou
   int key[DMK_MAX_PHASES];
   for (int p = 0; p < h->n_phases; p++) {
     items[p] = DmkStressItem{h->mp, h->lk_X, h->ph_dev + p, h->nm, h->dt, p, 0};
-    key[p] = 2 * h->ph[p].nsl + (h->ph[p].quarter_pow ? 1 : 0);
+    key[p] = 2 * dmk_sys_variant(&h->ph[p]) + (h->ph[p].quarter_pow ? 1 : 0);
   }
   DmkResidDev q{};
   q.st = h->mp.status;
