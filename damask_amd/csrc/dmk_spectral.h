@@ -4,10 +4,27 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+// Division of an index below 2^14 by a run-time constant d: (i m) >> s with
+// s = 14 + ceil(log2 d), m = floor(2^s / d) + 1.  0 < m d - 2^s <= d, so
+// i (m d - 2^s) <= i d < 2^s for i < 2^14 and the quotient is exact (the product
+// is below 2^30, both factors below 2^24).  One 24-bit multiplication and a shift, where a division by an unknown
+// is some 40 instructions; the transforms divide several times per value moved.
+struct FftDiv {
+  uint32_t m = 0;
+  int s = 0, d = 1;
+};
+FftDiv dmk_fft_div(int d);
+
+// 1-D transform of length L: the stages' radices, with nb[i] = L / radix[i]
+// butterflies each and ns[i] = product of the radices before.  In LDS, position p
+// of a line is stored at p + (p >> ps) and lines are ldl apart.
 struct FftPlan {
   int L;
   int nstages;
   int radix[16];
+  FftDiv nb[16], ns[16];
+  FftDiv len, half;        // L and h = L / 2 + 1
+  int ps, ldl;
 };
 
 // tile shapes: gx[0] = line pairs per block of the x pass, gx[1], gx[2] =

@@ -28,11 +28,18 @@ __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_doub
 __device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
 
-// twiddle w^m, w = exp(sign 2 pi i / L); table holds the forward (sign -1) values
-__device__ __forceinline__ double2 twid(const double2* __restrict__ tw, int m, int sign) {
+// twiddle w^m, w = exp(SIGN 2 pi i / L); the table holds the forward (-1) values
+template <int SIGN>
+__device__ __forceinline__ double2 twid(const double2* __restrict__ tw, int m) {
   double2 t = tw[m];
-  return sign < 0 ? t : cconj(t);
+  return SIGN < 0 ? t : cconj(t);
 }
+
+// quotient of an index below 2^14 (FftDiv)
+__device__ __forceinline__ int fdiv(int i, const FftDiv& d) { return (int)(__umul24((unsigned)i, d.m) >> d.s); }
+
+// LDS position of entry p of a line
+__device__ __forceinline__ int lpos(int p, int ps) { return p + (p >> ps); }
 
 // Work-groups of a launch are dispatched round-robin over the eight XCDs of
 // the MI355X, each with its own L2.  Kernels whose neighbouring blocks read
@@ -44,8 +51,28 @@ __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + s;
 }
 
+// cos and sin of 2 pi m / R for the odd radices
 template <int R>
-__device__ __forceinline__ void butterfly(double2* v, const double2* __restrict__ tw, int L, int sign) {
+struct OddRoots;
+template <>
+struct OddRoots<3> {
+  static constexpr double c[2] = {1.0, -0.5};
+  static constexpr double s[2] = {0.0, 0.86602540378443864676};
+};
+template <>
+struct OddRoots<5> {
+  static constexpr double c[3] = {1.0, 0.30901699437494742410, -0.80901699437494742410};
+  static constexpr double s[3] = {0.0, 0.95105651629515357212, 0.58778525229247312917};
+};
+template <>
+struct OddRoots<7> {
+  static constexpr double c[4] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624};
+  static constexpr double s[4] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
+};
+
+// DFT of R values in place, sign SIGN
+template <int R, int SIGN>
+__device__ __forceinline__ void butterfly(double2* v) {
   if constexpr (R == 2) {
     double2 a = v[0], b = v[1];
     v[0] = cadd(a, b);
@@ -54,7 +81,7 @@ __device__ __forceinline__ void butterfly(double2* v, const double2* __restrict_
     double2 a = v[0], b = v[1], c = v[2], d = v[3];
     double2 s0 = cadd(a, c), s1 = csub(a, c), s2 = cadd(b, d), s3 = csub(b, d);
     // multiply s3 by -i (forward) or +i (inverse)
-    double2 r3 = sign < 0 ? make_double2(s3.y, -s3.x) : make_double2(-s3.y, s3.x);
+    double2 r3 = SIGN < 0 ? make_double2(s3.y, -s3.x) : make_double2(-s3.y, s3.x);
     v[0] = cadd(s0, s2);
     v[2] = csub(s0, s2);
     v[1] = cadd(s1, r3);
@@ -65,7 +92,7 @@ __device__ __forceinline__ void butterfly(double2* v, const double2* __restrict_
     double2 a[4], b[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) { a[j] = cadd(v[j], v[j + 4]); b[j] = csub(v[j], v[j + 4]); }
-    if (sign < 0) {
+    if (SIGN < 0) {
       b[1] = make_double2((b[1].x + b[1].y) * c, (b[1].y - b[1].x) * c);
       b[2] = make_double2(b[2].y, -b[2].x);
       b[3] = make_double2((b[3].y - b[3].x) * c, -(b[3].x + b[3].y) * c);
@@ -74,94 +101,124 @@ __device__ __forceinline__ void butterfly(double2* v, const double2* __restrict_
       b[2] = make_double2(-b[2].y, b[2].x);
       b[3] = make_double2(-(b[3].x + b[3].y) * c, (b[3].x - b[3].y) * c);
     }
-    butterfly<4>(a, tw, L, sign);
-    butterfly<4>(b, tw, L, sign);
+    butterfly<4, SIGN>(a);
+    butterfly<4, SIGN>(b);
 #pragma unroll
     for (int j = 0; j < 4; j++) { v[2 * j] = a[j]; v[2 * j + 1] = b[j]; }
   } else {
-    double2 w[R];
-    const int st = L / R;
+    // odd R: the pairs x_m +- x_{R-m} share their cosine and sine sums between
+    // the outputs p and R - p
+    constexpr int H = (R - 1) / 2;
+    double2 t[H], d[H];
 #pragma unroll
-    for (int m = 0; m < R; m++) w[m] = twid(tw, m * st, sign);
-    double2 o[R];
+    for (int m = 0; m < H; m++) { t[m] = cadd(v[m + 1], v[R - 1 - m]); d[m] = csub(v[m + 1], v[R - 1 - m]); }
+    const double2 v0 = v[0];
+    double2 sum = v0;
 #pragma unroll
-    for (int p = 0; p < R; p++) {
-      double2 acc = v[0];
+    for (int m = 0; m < H; m++) sum = cadd(sum, t[m]);
+    v[0] = sum;
 #pragma unroll
-      for (int q = 1; q < R; q++) acc = cadd(acc, cmul(v[q], w[(p * q) % R]));
-      o[p] = acc;
+    for (int p = 1; p <= H; p++) {
+      double2 a = v0, b = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int m = 1; m <= H; m++) {
+        const int q = (p * m) % R, k = q <= H ? q : R - q;
+        const double c = OddRoots<R>::c[k], s = q <= H ? OddRoots<R>::s[k] : -OddRoots<R>::s[k];
+        a.x = fma(c, t[m - 1].x, a.x);
+        a.y = fma(c, t[m - 1].y, a.y);
+        b.x = fma(s, d[m - 1].x, b.x);
+        b.y = fma(s, d[m - 1].y, b.y);
+      }
+      // a + SIGN i b and its mirror
+      const double2 f = make_double2(a.x + b.y, a.y - b.x), g = make_double2(a.x - b.y, a.y + b.x);
+      v[p] = SIGN < 0 ? f : g;
+      v[R - p] = SIGN < 0 ? g : f;
     }
-#pragma unroll
-    for (int p = 0; p < R; p++) v[p] = o[p];
   }
 }
 
-// one Stockham stage of radix R over `nlines` lines of length L held in LDS
+// One Stockham stage of radix R, stage i of the plan: butterfly j of a line
+// takes entries j + r nb and leaves them at o + r Ns, o = (j / Ns) Ns R + j mod Ns.
+// Strides of both in LDS positions (lpos): lines are padded where 64 divides L,
+// and then 8 divides nb and every Ns but the first, so they are constant.
+template <int R, int SIGN>
+__device__ __forceinline__ int stage_load(const double2* in, const FftPlan& pl, int i, int Ns,
+                                          const double2* __restrict__ tw, int idx, double2* v) {
+  const int nb = pl.nb[i].d, line = fdiv(idx, pl.nb[i]), j = idx - line * nb;
+  const int ist = lpos(nb, pl.ps);
+  const double2* src = in + line * pl.ldl + lpos(j, pl.ps);
+#pragma unroll
+  for (int r = 0; r < R; r++) v[r] = src[r * ist];
+  int o = R * j;
+  if (Ns > 1) {
+    const int jn = fdiv(j, pl.ns[i]), k = j - jn * Ns, kt = k * fdiv(nb, pl.ns[i]);   // k L / (Ns R)
+    o = jn * Ns * R + k;
+#pragma unroll
+    for (int r = 1; r < R; r++) v[r] = cmul(v[r], twid<SIGN>(tw, r * kt));
+  }
+  butterfly<R, SIGN>(v);
+  return line * pl.ldl + lpos(o, pl.ps);
+}
+
 template <int R>
-__device__ void stockham_stage(const double2* in, double2* out, int nlines, int L, int ldl, int Ns,
-                               const double2* __restrict__ tw, int sign) {
-  const int nb = L / R;
-  const int tot = nlines * nb;
-  const int tstep = L / (Ns * R);
+__device__ __forceinline__ void stage_store(double2* out, const FftPlan& pl, int Ns, int at, const double2* v) {
+  const int ost = Ns > 1 ? lpos(Ns, pl.ps) : 1;
+#pragma unroll
+  for (int r = 0; r < R; r++) out[at + r * ost] = v[r];
+}
+
+template <int R, int SIGN>
+__device__ __forceinline__ void stockham_stage(const double2* in, double2* out, int nlines, const FftPlan& pl, int i,
+                                               int Ns, const double2* __restrict__ tw) {
+  const int tot = nlines * pl.nb[i].d;
   for (int idx = threadIdx.x; idx < tot; idx += blockDim.x) {
-    int line = idx / nb, j = idx - line * nb;
-    const double2* src = in + line * ldl;
-    double2* dst = out + line * ldl;
     double2 v[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) v[r] = src[j + r * nb];
-    int k = j % Ns;
-    if (Ns > 1) {
-#pragma unroll
-      for (int r = 1; r < R; r++) v[r] = cmul(v[r], twid(tw, (r * k * tstep) % L, sign));
-    }
-    butterfly<R>(v, tw, L, sign);
-    int o = (j / Ns) * Ns * R + k;
-#pragma unroll
-    for (int r = 0; r < R; r++) dst[o + r * Ns] = v[r];
+    const int at = stage_load<R, SIGN>(in, pl, i, Ns, tw, idx, v);
+    stage_store<R>(out, pl, Ns, at, v);
   }
 }
 
 // generic prime radix (rare sizes): O(R^2) DFT
-__device__ void stockham_stage_generic(const double2* in, double2* out, int nlines, int L, int ldl, int Ns, int R,
-                                       const double2* __restrict__ tw, int sign) {
-  const int nb = L / R;
+template <int SIGN>
+__device__ void stockham_stage_generic(const double2* in, double2* out, int nlines, const FftPlan& pl, int i, int Ns,
+                                       const double2* __restrict__ tw) {
+  const int L = pl.L, R = pl.radix[i], nb = L / R;
   const int tot = nlines * nb;
   const int tstep = L / (Ns * R);
-  const int st = L / R;
   for (int idx = threadIdx.x; idx < tot; idx += blockDim.x) {
     int line = idx / nb, j = idx - line * nb;
-    const double2* src = in + line * ldl;
-    double2* dst = out + line * ldl;
+    const double2* src = in + line * pl.ldl;
+    double2* dst = out + line * pl.ldl;
     int k = j % Ns;
     int o = (j / Ns) * Ns * R + k;
     for (int p = 0; p < R; p++) {
       double2 acc = make_double2(0.0, 0.0);
       for (int q = 0; q < R; q++) {
-        double2 x = src[j + q * nb];
-        if (Ns > 1 && q > 0) x = cmul(x, twid(tw, (q * k * tstep) % L, sign));
-        acc = cadd(acc, q == 0 ? x : cmul(x, twid(tw, ((p * q) % R) * st, sign)));
+        double2 x = src[lpos(j + q * nb, pl.ps)];
+        if (Ns > 1 && q > 0) x = cmul(x, twid<SIGN>(tw, q * k * tstep));
+        acc = cadd(acc, q == 0 ? x : cmul(x, twid<SIGN>(tw, ((p * q) % R) * nb)));
       }
-      dst[o + p * Ns] = acc;
+      dst[lpos(o + p * Ns, pl.ps)] = acc;
     }
   }
 }
 
 // full 1-D FFT of nlines LDS lines; returns the buffer holding the result
-__device__ double2* lds_fft(double2* b0, double2* b1, int nlines, int L, int ldl, const FftPlan& pl,
-                            const double2* __restrict__ tw, int sign) {
+template <int SIGN>
+__device__ __forceinline__ double2* lds_fft(double2* b0, double2* b1, int nlines, const FftPlan& pl,
+                                            const double2* __restrict__ tw) {
   double2 *in = b0, *out = b1;
   int Ns = 1;
   for (int s = 0; s < pl.nstages; s++) {
-    int R = pl.radix[s];
+    const int R = pl.radix[s];
     switch (R) {
-      case 2: stockham_stage<2>(in, out, nlines, L, ldl, Ns, tw, sign); break;
-      case 3: stockham_stage<3>(in, out, nlines, L, ldl, Ns, tw, sign); break;
-      case 4: stockham_stage<4>(in, out, nlines, L, ldl, Ns, tw, sign); break;
-      case 5: stockham_stage<5>(in, out, nlines, L, ldl, Ns, tw, sign); break;
-      case 7: stockham_stage<7>(in, out, nlines, L, ldl, Ns, tw, sign); break;
-      case 8: stockham_stage<8>(in, out, nlines, L, ldl, Ns, tw, sign); break;
-      default: stockham_stage_generic(in, out, nlines, L, ldl, Ns, R, tw, sign); break;
+      case 2: stockham_stage<2, SIGN>(in, out, nlines, pl, s, Ns, tw); break;
+      case 3: stockham_stage<3, SIGN>(in, out, nlines, pl, s, Ns, tw); break;
+      case 4: stockham_stage<4, SIGN>(in, out, nlines, pl, s, Ns, tw); break;
+      case 5: stockham_stage<5, SIGN>(in, out, nlines, pl, s, Ns, tw); break;
+      case 7: stockham_stage<7, SIGN>(in, out, nlines, pl, s, Ns, tw); break;
+      case 8: stockham_stage<8, SIGN>(in, out, nlines, pl, s, Ns, tw); break;
+      default: stockham_stage_generic<SIGN>(in, out, nlines, pl, s, Ns, tw); break;
     }
     __syncthreads();
     double2* t = in; in = out; out = t;
@@ -175,35 +232,28 @@ __device__ double2* lds_fft(double2* b0, double2* b1, int nlines, int L, int ldl
 __global__ void __launch_bounds__(256) fft_x_r2c(const double* __restrict__ in, double2* __restrict__ out,
                                                  int nl, FftPlan pl, const double2* __restrict__ tw, int pairs_per_block) {
   extern __shared__ double2 lds[];
-  const int L = pl.L, h = L / 2 + 1, ldl = L + 1;
+  const int L = pl.L, h = pl.half.d, ldl = pl.ldl, ps = pl.ps;
   double2* b0 = lds;
   double2* b1 = lds + pairs_per_block * ldl;
   const int p0 = blockIdx.x * pairs_per_block;
   const long l0 = 2L * p0;
   const int nlines_here = min(2 * pairs_per_block, nl - (int)l0);
   const int npairs = (nlines_here + 1) / 2;
-  for (int i = threadIdx.x; i < 2 * pairs_per_block * L; i += blockDim.x) {
-    int line = i / L, pos = i - line * L;
-    double v = line < nlines_here ? in[(l0 + line) * L + pos] : 0.0;
-    double2* c = &b0[(line >> 1) * ldl + pos];
-    if (line & 1) c->y = v; else c->x = v;
+  for (int i = threadIdx.x; i < npairs * L; i += blockDim.x) {
+    const int p = fdiv(i, pl.len), pos = i - p * L;
+    const double* src = in + (l0 + 2 * p) * L + pos;
+    b0[p * ldl + lpos(pos, ps)] = make_double2(src[0], 2 * p + 1 < nlines_here ? src[L] : 0.0);
   }
   __syncthreads();
-  double2* r = lds_fft(b0, b1, npairs, L, ldl, pl, tw, -1);
-  for (int i = threadIdx.x; i < 2 * pairs_per_block * h; i += blockDim.x) {
-    int line = i / h, k = i - line * h;
-    if (line >= nlines_here) continue;
-    const double2* z = r + (line >> 1) * ldl;
-    double2 a = z[k], b = cconj(z[(L - k) % L]);
-    double2 v;
-    if (line & 1) {            // (Z[k] - conj Z[L-k]) / (2i)
-      double2 d = csub(a, b);
-      v = make_double2(0.5 * d.y, -0.5 * d.x);
-    } else {
-      double2 s = cadd(a, b);
-      v = make_double2(0.5 * s.x, 0.5 * s.y);
-    }
-    out[(l0 + line) * h + k] = v;
+  const double2* r = lds_fft<-1>(b0, b1, npairs, pl, tw);
+  // the pair's spectra: (Z[k] + conj Z[L-k]) / 2 and (Z[k] - conj Z[L-k]) / (2i)
+  for (int i = threadIdx.x; i < npairs * h; i += blockDim.x) {
+    const int p = fdiv(i, pl.half), k = i - p * h;
+    const double2* z = r + p * ldl;
+    const double2 a = z[lpos(k, ps)], b = cconj(z[lpos(k ? L - k : 0, ps)]), s = cadd(a, b), d = csub(a, b);
+    double2* dst = out + (l0 + 2 * p) * h + k;
+    dst[0] = make_double2(0.5 * s.x, 0.5 * s.y);
+    if (2 * p + 1 < nlines_here) dst[h] = make_double2(0.5 * d.y, -0.5 * d.x);
   }
 }
 
@@ -212,7 +262,7 @@ __global__ void __launch_bounds__(256) fft_x_r2c(const double* __restrict__ in, 
 __global__ void __launch_bounds__(256) fft_x_c2r(const double2* __restrict__ in, double* __restrict__ out,
                                                  int nl, FftPlan pl, const double2* __restrict__ tw, int pairs_per_block) {
   extern __shared__ double2 lds[];
-  const int L = pl.L, h = L / 2 + 1, ldl = L + 1;
+  const int L = pl.L, h = pl.half.d, ldl = pl.ldl, ps = pl.ps;
   double2* b0 = lds;
   double2* b1 = lds + pairs_per_block * ldl;
   const int p0 = blockIdx.x * pairs_per_block;
@@ -221,205 +271,65 @@ __global__ void __launch_bounds__(256) fft_x_c2r(const double2* __restrict__ in,
   const int npairs = (nlines_here + 1) / 2;
   // Z[k] = A[k] + i B[k] with A, B extended by Hermitian symmetry; the
   // imaginary parts of the DC and Nyquist bins do not enter
-  for (int i = threadIdx.x; i < pairs_per_block * L; i += blockDim.x) {
-    int p = i / L, k = i - p * L;
-    double2 z = make_double2(0.0, 0.0);
-    if (p < npairs) {
-      int kk = (k < h) ? k : L - k;
-      bool cj = k >= h;
-      long la = l0 + 2 * p, lb = la + 1;
-      double2 a = in[la * h + kk];
-      if (kk == 0 || 2 * kk == L) a.y = 0.0;
-      if (cj) a.y = -a.y;
-      double2 b = make_double2(0.0, 0.0);
-      if (2 * p + 1 < nlines_here) {
-        b = in[lb * h + kk];
-        if (kk == 0 || 2 * kk == L) b.y = 0.0;
-        if (cj) b.y = -b.y;
-      }
-      z = make_double2(a.x - b.y, a.y + b.x);
-    }
-    b0[p * ldl + k] = z;
+  for (int i = threadIdx.x; i < npairs * h; i += blockDim.x) {
+    const int p = fdiv(i, pl.half), k = i - p * h;
+    const double2* src = in + (l0 + 2 * p) * h + k;
+    const bool real = k == 0 || 2 * k == L;
+    double2 a = src[0], b = 2 * p + 1 < nlines_here ? src[h] : make_double2(0.0, 0.0);
+    if (real) a.y = b.y = 0.0;
+    double2* dst = b0 + p * ldl;
+    dst[lpos(k, ps)] = make_double2(a.x - b.y, a.y + b.x);
+    if (!real) dst[lpos(L - k, ps)] = make_double2(a.x + b.y, b.x - a.y);
   }
   __syncthreads();
-  double2* r = lds_fft(b0, b1, npairs, L, ldl, pl, tw, +1);
-  for (int i = threadIdx.x; i < 2 * pairs_per_block * L; i += blockDim.x) {
-    int line = i / L, pos = i - line * L;
-    if (line >= nlines_here) continue;
-    double2 z = r[(line >> 1) * ldl + pos];
-    out[(l0 + line) * L + pos] = (line & 1) ? z.y : z.x;
+  const double2* r = lds_fft<+1>(b0, b1, npairs, pl, tw);
+  for (int i = threadIdx.x; i < npairs * L; i += blockDim.x) {
+    const int p = fdiv(i, pl.len), pos = i - p * L;
+    const double2 z = r[p * ldl + lpos(pos, ps)];
+    double* dst = out + (l0 + 2 * p) * L + pos;
+    dst[0] = z.x;
+    if (2 * p + 1 < nlines_here) dst[L] = z.y;
   }
 }
 
 // In-place variants for radix 2, 4 and 8 plans: each thread keeps its
-// butterflies (at most KMAX) in registers across a barrier and writes them
-// back into the same LDS buffer, so one buffer suffices and more blocks fit on
-// a CU.  Same arithmetic as stockham_stage / lds_fft.
-constexpr int IP_KMAX = 2;     // butterflies per thread and stage
-constexpr int IP_KU = 12;      // unpacked values per thread
+// butterflies (IP_VALS values of a stage) in registers across a barrier and
+// writes them back into the same LDS buffer, so one buffer suffices and more
+// blocks fit on a CU, or planes that two buffers do not (up to 128x128).  Same
+// arithmetic as stockham_stage / lds_fft.
+constexpr int IP_VALS = 16;
+constexpr int IP_THREADS = 640;   // largest block
 
-template <int R>
-__device__ void stockham_stage_ip(double2* buf, int nlines, int L, int ldl, int Ns, const double2* __restrict__ tw,
-                                  int sign) {
-  const int nb = L / R;
-  const int tot = nlines * nb;
-  const int tstep = L / (Ns * R);
-  double2 v[IP_KMAX][R];
-  int dst[IP_KMAX];
+template <int R, int SIGN>
+__device__ __forceinline__ void stockham_stage_ip(double2* buf, int nlines, const FftPlan& pl, int i, int Ns,
+                                                  const double2* __restrict__ tw) {
+  constexpr int KMAX = IP_VALS / R;
+  const int tot = nlines * pl.nb[i].d;
+  double2 v[KMAX][R];
+  int dst[KMAX];
 #pragma unroll
-  for (int q = 0; q < IP_KMAX; q++) {
+  for (int q = 0; q < KMAX; q++) {
     const int idx = threadIdx.x + q * blockDim.x;
-    dst[q] = -1;
-    if (idx < tot) {
-      const int line = idx / nb, j = idx - line * nb;
-      const double2* src = buf + line * ldl;
-#pragma unroll
-      for (int r = 0; r < R; r++) v[q][r] = src[j + r * nb];
-      const int k = j % Ns;
-      if (Ns > 1) {
-#pragma unroll
-        for (int r = 1; r < R; r++) v[q][r] = cmul(v[q][r], twid(tw, (r * k * tstep) % L, sign));
-      }
-      butterfly<R>(v[q], tw, L, sign);
-      dst[q] = line * ldl + (j / Ns) * Ns * R + k;
-    }
+    if (idx < tot) dst[q] = stage_load<R, SIGN>(buf, pl, i, Ns, tw, idx, v[q]);
   }
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < IP_KMAX; q++)
-    if (dst[q] >= 0) {
-#pragma unroll
-      for (int r = 0; r < R; r++) buf[dst[q] + r * Ns] = v[q][r];
-    }
+  for (int q = 0; q < KMAX; q++)
+    if ((int)(threadIdx.x + q * blockDim.x) < tot) stage_store<R>(buf, pl, Ns, dst[q], v[q]);
   __syncthreads();
 }
 
-__device__ void lds_fft_ip(double2* buf, int nlines, int L, int ldl, const FftPlan& pl, const double2* __restrict__ tw,
-                           int sign) {
+template <int SIGN>
+__device__ __forceinline__ void lds_fft_ip(double2* buf, int nlines, const FftPlan& pl,
+                                           const double2* __restrict__ tw) {
   int Ns = 1;
   for (int s = 0; s < pl.nstages; s++) {
     const int R = pl.radix[s];
-    if (R == 8) stockham_stage_ip<8>(buf, nlines, L, ldl, Ns, tw, sign);
-    else if (R == 4) stockham_stage_ip<4>(buf, nlines, L, ldl, Ns, tw, sign);
-    else stockham_stage_ip<2>(buf, nlines, L, ldl, Ns, tw, sign);
+    if (R == 8) stockham_stage_ip<8, SIGN>(buf, nlines, pl, s, Ns, tw);
+    else if (R == 4) stockham_stage_ip<4, SIGN>(buf, nlines, pl, s, Ns, tw);
+    else stockham_stage_ip<2, SIGN>(buf, nlines, pl, s, Ns, tw);
     Ns *= R;
   }
-}
-
-__device__ __forceinline__ void xy_r2c_ip_body(const double* __restrict__ in, double2* __restrict__ out, int N1,
-                                               int N2, int N3, const FftPlan& px, const double2* __restrict__ twx,
-                                               const FftPlan& py, const double2* __restrict__ twy, unsigned plane) {
-  extern __shared__ double2 lds[];
-  const int h = N1 / 2 + 1, np = (N2 + 1) / 2, lx = N1 + 1, ly = N2 + 1;
-  double2* A = lds;
-  const double* src = in + (long)plane * N1 * N2;
-  for (int i = threadIdx.x; i < 2 * np * N1; i += blockDim.x) {
-    int line = i / N1, pos = i - line * N1;
-    double v = line < N2 ? src[(long)line * N1 + pos] : 0.0;
-    double2* c = &A[(line >> 1) * lx + pos];
-    if (line & 1) c->y = v; else c->x = v;
-  }
-  __syncthreads();
-  lds_fft_ip(A, np, N1, lx, px, twx, -1);
-  // unpack the pairs into y lines (in registers across the barrier)
-  double2 u[IP_KU];
-#pragma unroll
-  for (int q = 0; q < IP_KU; q++) {
-    const int i = threadIdx.x + q * blockDim.x;
-    if (i < N2 * h) {
-      int line = i / h, k = i - line * h;
-      const double2* z = A + (line >> 1) * lx;
-      double2 a = z[k], b = cconj(z[(N1 - k) % N1]);
-      if (line & 1) {
-        double2 d = csub(a, b);
-        u[q] = make_double2(0.5 * d.y, -0.5 * d.x);
-      } else {
-        double2 s = cadd(a, b);
-        u[q] = make_double2(0.5 * s.x, 0.5 * s.y);
-      }
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < IP_KU; q++) {
-    const int i = threadIdx.x + q * blockDim.x;
-    if (i < N2 * h) {
-      int line = i / h, k = i - line * h;
-      A[k * ly + line] = u[q];
-    }
-  }
-  __syncthreads();
-  lds_fft_ip(A, h, N2, ly, py, twy, -1);
-  double2* dst = out + (plane / N3) * ((long)h * N2 * N3) + (long)(plane % N3) * h * N2;
-  for (int i = threadIdx.x; i < N2 * h; i += blockDim.x) {
-    int ky = i / h, kx = i - ky * h;
-    dst[i] = A[kx * ly + ky];
-  }
-}
-
-__global__ __launch_bounds__(512) void fft_xy_r2c_ip(const double* __restrict__ in, double2* __restrict__ out, int N1, int N2, int N3,
-                              FftPlan px, const double2* __restrict__ twx, FftPlan py,
-                              const double2* __restrict__ twy) {
-  xy_r2c_ip_body(in, out, N1, N2, N3, px, twx, py, twy, blockIdx.x);
-}
-
-__device__ __forceinline__ void yx_c2r_ip_body(const double2* __restrict__ in, double* __restrict__ out, int N1,
-                                               int N2, int N3, const FftPlan& px, const double2* __restrict__ twx,
-                                               const FftPlan& py, const double2* __restrict__ twy, unsigned plane) {
-  extern __shared__ double2 lds[];
-  const int h = N1 / 2 + 1, np = (N2 + 1) / 2, lx = N1 + 1, ly = N2 + 1;
-  double2* A = lds;
-  const double2* src = in + (plane / N3) * ((long)h * N2 * N3) + (long)(plane % N3) * h * N2;
-  for (int i = threadIdx.x; i < N2 * h; i += blockDim.x) {
-    int ky = i / h, kx = i - ky * h;
-    A[kx * ly + ky] = src[i];
-  }
-  __syncthreads();
-  lds_fft_ip(A, h, N2, ly, py, twy, +1);
-  // pack pairs of y lines into complex x lines (registers across the barrier)
-  double2 u[IP_KU];
-#pragma unroll
-  for (int q = 0; q < IP_KU; q++) {
-    const int i = threadIdx.x + q * blockDim.x;
-    if (i < np * N1) {
-      int p = i / N1, k = i - p * N1;
-      int kk = (k < h) ? k : N1 - k;
-      bool cj = k >= h;
-      double2 a = A[kk * ly + 2 * p];
-      if (kk == 0 || 2 * kk == N1) a.y = 0.0;
-      if (cj) a.y = -a.y;
-      double2 b = make_double2(0.0, 0.0);
-      if (2 * p + 1 < N2) {
-        b = A[kk * ly + 2 * p + 1];
-        if (kk == 0 || 2 * kk == N1) b.y = 0.0;
-        if (cj) b.y = -b.y;
-      }
-      u[q] = make_double2(a.x - b.y, a.y + b.x);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < IP_KU; q++) {
-    const int i = threadIdx.x + q * blockDim.x;
-    if (i < np * N1) {
-      int p = i / N1, k = i - p * N1;
-      A[p * lx + k] = u[q];
-    }
-  }
-  __syncthreads();
-  lds_fft_ip(A, np, N1, lx, px, twx, +1);
-  double* dst = out + (long)plane * N1 * N2;
-  for (int i = threadIdx.x; i < N1 * N2; i += blockDim.x) {
-    int line = i / N1, pos = i - line * N1;
-    double2 z = A[(line >> 1) * lx + pos];
-    dst[i] = (line & 1) ? z.y : z.x;
-  }
-}
-
-__global__ __launch_bounds__(512) void fft_yx_c2r_ip(const double2* __restrict__ in, double* __restrict__ out, int N1, int N2, int N3,
-                              FftPlan px, const double2* __restrict__ twx, FftPlan py,
-                              const double2* __restrict__ twy) {
-  yx_c2r_ip_body(in, out, N1, N2, N3, px, twx, py, twy, blockIdx.x);
 }
 
 // Fused x and y passes, one block per (field, z) plane: the real plane and its
@@ -429,117 +339,178 @@ __global__ __launch_bounds__(512) void fft_yx_c2r_ip(const double2* __restrict__
 // y (same line packing, same Stockham stages), so for even N2 results are
 // bitwise those of the separate passes (for odd N2 the x pass pairs the last
 // line of a plane with zeros instead of the next plane's first line: equal to
-// rounding).  LDS: two buffers of max(ceil(N2/2) (N1+1), h (N2+1)) complex
-// values.
-__device__ __forceinline__ int xy_buf(int N1, int N2) {
-  const int h = N1 / 2 + 1, np = (N2 + 1) / 2;
-  int a = np * (N1 + 1), b = h * (N2 + 1);
+// rounding).  LDS: one (IP) or two buffers of xy_buf complex values.
+// Between the passes the plane changes from pairs of x lines to y lines: through
+// registers across a barrier with one buffer (KU values a thread), from one
+// buffer to the other with two.
+__host__ __device__ __forceinline__ int xy_buf(const FftPlan& px, const FftPlan& py) {
+  const int a = ((py.L + 1) / 2) * px.ldl, b = (px.L / 2 + 1) * py.ldl;
   return a > b ? a : b;
 }
 
-__device__ __forceinline__ void xy_r2c_body(const double* __restrict__ in, double2* __restrict__ out, int N1, int N2,
-                                            int N3, const FftPlan& px, const double2* __restrict__ twx,
-                                            const FftPlan& py, const double2* __restrict__ twy, unsigned plane) {
+template <bool IP, int KU>
+__device__ __forceinline__ void xy_r2c_body(const double* __restrict__ in, double2* __restrict__ out, int N3,
+                                            const FftPlan& px, const double2* __restrict__ twx, const FftPlan& py,
+                                            const double2* __restrict__ twy, unsigned plane) {
   extern __shared__ double2 lds[];
-  const int h = N1 / 2 + 1, np = (N2 + 1) / 2, lx = N1 + 1, ly = N2 + 1;
-  double2* A = lds;
-  double2* B = lds + xy_buf(N1, N2);
+  const int N1 = px.L, N2 = py.L, h = px.half.d, np = (N2 + 1) / 2, lx = px.ldl, ly = py.ldl;
+  double2 *A = lds, *B = lds + (IP ? 0 : xy_buf(px, py));
   const double* src = in + (long)plane * N1 * N2;   // plane = field * N3 + z
-  for (int i = threadIdx.x; i < 2 * np * N1; i += blockDim.x) {
-    int line = i / N1, pos = i - line * N1;
-    double v = line < N2 ? src[(long)line * N1 + pos] : 0.0;
-    double2* c = &A[(line >> 1) * lx + pos];
-    if (line & 1) c->y = v; else c->x = v;
+  for (int i = threadIdx.x; i < np * N1; i += blockDim.x) {
+    const int p = fdiv(i, px.len), pos = i - p * N1;
+    const double* s = src + 2 * p * N1 + pos;
+    A[p * lx + lpos(pos, px.ps)] = make_double2(s[0], 2 * p + 1 < N2 ? s[N1] : 0.0);
   }
   __syncthreads();
-  double2* r = lds_fft(A, B, np, N1, lx, px, twx, -1);
-  double2* t = r == A ? B : A;
-  for (int i = threadIdx.x; i < N2 * h; i += blockDim.x) {
-    int line = i / h, k = i - line * h;
-    const double2* z = r + (line >> 1) * lx;
-    double2 a = z[k], b = cconj(z[(N1 - k) % N1]);
-    double2 v;
-    if (line & 1) {
-      double2 d = csub(a, b);
-      v = make_double2(0.5 * d.y, -0.5 * d.x);
-    } else {
-      double2 s = cadd(a, b);
-      v = make_double2(0.5 * s.x, 0.5 * s.y);
+  const double2* z = A;
+  if (IP) lds_fft_ip<-1>(A, np, px, twx);
+  else z = lds_fft<-1>(A, B, np, px, twx);
+  double2* t = IP || z == B ? A : B;
+  // the pairs' spectra: (Z[k] + conj Z[N1-k]) / 2 and (Z[k] - conj Z[N1-k]) / (2i)
+  auto unpack = [&](int i, double2& s, double2& d) {
+    const int p = fdiv(i, px.half), k = i - p * h;
+    const double2* y = z + p * lx;
+    const double2 a = y[lpos(k, px.ps)], b = cconj(y[lpos(k ? N1 - k : 0, px.ps)]);
+    s = cadd(a, b);
+    d = csub(a, b);
+    s = make_double2(0.5 * s.x, 0.5 * s.y);
+    d = make_double2(0.5 * d.y, -0.5 * d.x);
+  };
+  auto put = [&](int i, const double2& s, const double2& d) {
+    const int p = fdiv(i, px.half), k = i - p * h;
+    t[k * ly + lpos(2 * p, py.ps)] = s;
+    if (2 * p + 1 < N2) t[k * ly + lpos(2 * p + 1, py.ps)] = d;
+  };
+  if (IP) {
+    double2 u[KU], w[KU];
+#pragma unroll
+    for (int q = 0; q < KU; q++) {
+      const int i = threadIdx.x + q * blockDim.x;
+      if (i < np * h) unpack(i, u[q], w[q]);
     }
-    t[k * ly + line] = v;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < KU; q++) {
+      const int i = threadIdx.x + q * blockDim.x;
+      if (i < np * h) put(i, u[q], w[q]);
+    }
+  } else {
+    for (int i = threadIdx.x; i < np * h; i += blockDim.x) {
+      double2 s, d;
+      unpack(i, s, d);
+      put(i, s, d);
+    }
   }
   __syncthreads();
-  double2* q = lds_fft(t, r, h, N2, ly, py, twy, -1);
+  const double2* q = t;
+  if (IP) lds_fft_ip<-1>(A, h, py, twy);
+  else q = lds_fft<-1>(t, t == A ? B : A, h, py, twy);
   double2* dst = out + (plane / N3) * ((long)h * N2 * N3) + (long)(plane % N3) * h * N2;
   for (int i = threadIdx.x; i < N2 * h; i += blockDim.x) {
-    int ky = i / h, kx = i - ky * h;
-    dst[i] = q[kx * ly + ky];
+    const int ky = fdiv(i, px.half), kx = i - ky * h;
+    dst[i] = q[kx * ly + lpos(ky, py.ps)];
   }
 }
 
-__global__ void fft_xy_r2c(const double* __restrict__ in, double2* __restrict__ out, int N1, int N2, int N3,
-                           FftPlan px, const double2* __restrict__ twx, FftPlan py,
-                           const double2* __restrict__ twy) {
-  xy_r2c_body(in, out, N1, N2, N3, px, twx, py, twy, blockIdx.x);
-}
-
-__device__ __forceinline__ void yx_c2r_body(const double2* __restrict__ in, double* __restrict__ out, int N1, int N2,
-                                            int N3, const FftPlan& px, const double2* __restrict__ twx,
-                                            const FftPlan& py, const double2* __restrict__ twy, unsigned plane) {
+template <bool IP, int KU>
+__device__ __forceinline__ void yx_c2r_body(const double2* __restrict__ in, double* __restrict__ out, int N3,
+                                            const FftPlan& px, const double2* __restrict__ twx, const FftPlan& py,
+                                            const double2* __restrict__ twy, unsigned plane) {
   extern __shared__ double2 lds[];
-  const int h = N1 / 2 + 1, np = (N2 + 1) / 2, lx = N1 + 1, ly = N2 + 1;
-  double2* A = lds;
-  double2* B = lds + xy_buf(N1, N2);
+  const int N1 = px.L, N2 = py.L, h = px.half.d, np = (N2 + 1) / 2, lx = px.ldl, ly = py.ldl;
+  double2 *A = lds, *B = lds + (IP ? 0 : xy_buf(px, py));
   const double2* src = in + (plane / N3) * ((long)h * N2 * N3) + (long)(plane % N3) * h * N2;
   for (int i = threadIdx.x; i < N2 * h; i += blockDim.x) {
-    int ky = i / h, kx = i - ky * h;
-    A[kx * ly + ky] = src[i];
+    const int ky = fdiv(i, px.half), kx = i - ky * h;
+    A[kx * ly + lpos(ky, py.ps)] = src[i];
   }
   __syncthreads();
-  double2* r = lds_fft(A, B, h, N2, ly, py, twy, +1);
-  double2* t = r == A ? B : A;
-  // pairs of y lines into one complex line, Hermitian-extended in x; the
-  // imaginary parts of the DC and Nyquist bins do not enter
-  for (int i = threadIdx.x; i < np * N1; i += blockDim.x) {
-    int p = i / N1, k = i - p * N1;
-    int kk = (k < h) ? k : N1 - k;
-    bool cj = k >= h;
-    double2 a = r[kk * ly + 2 * p];
-    if (kk == 0 || 2 * kk == N1) a.y = 0.0;
-    if (cj) a.y = -a.y;
-    double2 b = make_double2(0.0, 0.0);
-    if (2 * p + 1 < N2) {
-      b = r[kk * ly + 2 * p + 1];
-      if (kk == 0 || 2 * kk == N1) b.y = 0.0;
-      if (cj) b.y = -b.y;
+  const double2* z = A;
+  if (IP) lds_fft_ip<+1>(A, h, py, twy);
+  else z = lds_fft<+1>(A, B, h, py, twy);
+  double2* t = IP || z == B ? A : B;
+  // pairs of y lines into one complex line, Hermitian-extended in x (entries k
+  // and N1 - k); the imaginary parts of the DC and Nyquist bins do not enter
+  auto pack = [&](int i, double2& a, double2& b) {
+    const int p = fdiv(i, px.half), k = i - p * h;
+    a = z[k * ly + lpos(2 * p, py.ps)];
+    b = 2 * p + 1 < N2 ? z[k * ly + lpos(2 * p + 1, py.ps)] : make_double2(0.0, 0.0);
+    if (k == 0 || 2 * k == N1) a.y = b.y = 0.0;
+  };
+  auto put = [&](int i, const double2& a, const double2& b) {
+    const int p = fdiv(i, px.half), k = i - p * h;
+    t[p * lx + lpos(k, px.ps)] = make_double2(a.x - b.y, a.y + b.x);
+    if (k != 0 && 2 * k != N1) t[p * lx + lpos(N1 - k, px.ps)] = make_double2(a.x + b.y, b.x - a.y);
+  };
+  if (IP) {
+    double2 u[KU], w[KU];
+#pragma unroll
+    for (int q = 0; q < KU; q++) {
+      const int i = threadIdx.x + q * blockDim.x;
+      if (i < np * h) pack(i, u[q], w[q]);
     }
-    t[p * lx + k] = make_double2(a.x - b.y, a.y + b.x);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < KU; q++) {
+      const int i = threadIdx.x + q * blockDim.x;
+      if (i < np * h) put(i, u[q], w[q]);
+    }
+  } else {
+    for (int i = threadIdx.x; i < np * h; i += blockDim.x) {
+      double2 a, b;
+      pack(i, a, b);
+      put(i, a, b);
+    }
   }
   __syncthreads();
-  double2* q = lds_fft(t, r, np, N1, lx, px, twx, +1);
+  const double2* q = t;
+  if (IP) lds_fft_ip<+1>(A, np, px, twx);
+  else q = lds_fft<+1>(t, t == A ? B : A, np, px, twx);
   double* dst = out + (long)plane * N1 * N2;
-  for (int i = threadIdx.x; i < N1 * N2; i += blockDim.x) {
-    int line = i / N1, pos = i - line * N1;
-    double2 z = q[(line >> 1) * lx + pos];
-    dst[i] = (line & 1) ? z.y : z.x;
+  for (int i = threadIdx.x; i < np * N1; i += blockDim.x) {
+    const int p = fdiv(i, px.len), pos = i - p * N1;
+    const double2 v = q[p * lx + lpos(pos, px.ps)];
+    double* d = dst + 2 * p * N1 + pos;
+    d[0] = v.x;
+    if (2 * p + 1 < N2) d[N1] = v.y;
   }
 }
 
-__global__ void fft_yx_c2r(const double2* __restrict__ in, double* __restrict__ out, int N1, int N2, int N3,
-                           FftPlan px, const double2* __restrict__ twx, FftPlan py,
-                           const double2* __restrict__ twy) {
-  yx_c2r_body(in, out, N1, N2, N3, px, twx, py, twy, blockIdx.x);
+// pair entries a thread of the in-place kernels carries across the barrier
+constexpr int IP_KU = 8;
+
+__global__ void __launch_bounds__(IP_THREADS) fft_xy_r2c_ip(const double* __restrict__ in, double2* __restrict__ out,
+                                                            int N3, FftPlan px, const double2* __restrict__ twx,
+                                                            FftPlan py, const double2* __restrict__ twy) {
+  xy_r2c_body<true, IP_KU>(in, out, N3, px, twx, py, twy, blockIdx.x);
+}
+
+__global__ void __launch_bounds__(IP_THREADS) fft_yx_c2r_ip(const double2* __restrict__ in, double* __restrict__ out,
+                                                            int N3, FftPlan px, const double2* __restrict__ twx,
+                                                            FftPlan py, const double2* __restrict__ twy) {
+  yx_c2r_body<true, IP_KU>(in, out, N3, px, twx, py, twy, blockIdx.x);
+}
+
+__global__ void fft_xy_r2c(const double* __restrict__ in, double2* __restrict__ out, int N3, FftPlan px,
+                           const double2* __restrict__ twx, FftPlan py, const double2* __restrict__ twy) {
+  xy_r2c_body<false, 1>(in, out, N3, px, twx, py, twy, blockIdx.x);
+}
+
+__global__ void fft_yx_c2r(const double2* __restrict__ in, double* __restrict__ out, int N3, FftPlan px,
+                           const double2* __restrict__ twx, FftPlan py, const double2* __restrict__ twy) {
+  yx_c2r_body<false, 1>(in, out, N3, px, twx, py, twy, blockIdx.x);
 }
 
 // c2c pass along a strided axis.  A line group is `gx` lines adjacent in x
 // (unit stride) starting at x0, of length L with element stride `stride`;
 // groups are enumerated over (outer index, x chunk); outer o has base offset
 // (o / M) * comp_stride + (o % M) * outer_stride.
-__global__ void __launch_bounds__(256) fft_strided(double2* __restrict__ data, int nx, int gx, int M, long comp_stride,
-                                                   long outer_stride, long stride, FftPlan pl,
-                                                   const double2* __restrict__ tw, int sign) {
+template <int SIGN>
+__global__ void __launch_bounds__(256) fft_strided(double2* __restrict__ data, int nx, FftDiv gxd, int M,
+                                                   long comp_stride, long outer_stride, long stride, FftPlan pl,
+                                                   const double2* __restrict__ tw) {
   extern __shared__ double2 lds[];
-  const int L = pl.L, ldl = L + 1;
+  const int L = pl.L, ldl = pl.ldl, gx = gxd.d;
   double2* b0 = lds;
   double2* b1 = lds + gx * ldl;
   const int nchunk = (nx + gx - 1) / gx;
@@ -549,18 +520,26 @@ __global__ void __launch_bounds__(256) fft_strided(double2* __restrict__ data, i
   const int nlx = min(gx, nx - x0);
   double2* base = data + (long)(o / M) * comp_stride + (long)(o % M) * outer_stride + x0;
   for (int i = threadIdx.x; i < gx * L; i += blockDim.x) {
-    int j = i / gx, x = i - j * gx;
-    b0[x * ldl + j] = x < nlx ? base[(long)j * stride + x] : make_double2(0.0, 0.0);
+    const int j = fdiv(i, gxd), x = i - j * gx;
+    b0[x * ldl + lpos(j, pl.ps)] = x < nlx ? base[(long)j * stride + x] : make_double2(0.0, 0.0);
   }
   __syncthreads();
-  double2* r = lds_fft(b0, b1, gx, L, ldl, pl, tw, sign);
+  const double2* r = lds_fft<SIGN>(b0, b1, gx, pl, tw);
   for (int i = threadIdx.x; i < gx * L; i += blockDim.x) {
-    int j = i / gx, x = i - j * gx;
-    if (x < nlx) base[(long)j * stride + x] = r[x * ldl + j];
+    const int j = fdiv(i, gxd), x = i - j * gx;
+    if (x < nlx) base[(long)j * stride + x] = r[x * ldl + lpos(j, pl.ps)];
   }
 }
 
 // ---------------------------------------------------------------- Gamma + div
+// kx, ky, kz of frequency f (fewer than 2^32: N < 2^29 cells)
+__device__ __forceinline__ void freq_of(unsigned f, const GammaArgs& g, int& kx, int& ky, int& kz) {
+  const unsigned r = f / (unsigned)g.h, z = r / (unsigned)g.n[1];
+  kx = (int)(f - r * (unsigned)g.h);
+  ky = (int)(r - z * (unsigned)g.n[1]);
+  kz = (int)z;
+}
+
 __device__ __forceinline__ double wrap_freq(int k, int n) { return (double)(k > n / 2 ? k - n : k); }
 
 // divergence contribution and (with do_gamma) the Gamma convolution of one
@@ -662,10 +641,8 @@ __global__ void __launch_bounds__(256) gamma_div_kernel(double2* __restrict__ Z,
   const long f = (long)blockIdx.x * blockDim.x + threadIdx.x;
   double contrib = 0.0;
   if (f < Nk) {
-    int kx = (int)(f % g.h);
-    long r = f / g.h;
-    int ky = (int)(r % g.n[1]);
-    int kz = (int)(r / g.n[1]);
+    int kx, ky, kz;
+    freq_of((unsigned)f, g, kx, ky, kz);
     double2 P[9];
 #pragma unroll
     for (int c = 0; c < 9; c++) P[c] = Z[c * Nk + f];
@@ -691,159 +668,106 @@ __global__ void __launch_bounds__(256) gamma_div_kernel(double2* __restrict__ Z,
 // the nine fields in one kernel.  A block holds gz consecutive columns
 // m = kx + h ky (all z) of the nine fields in LDS, as lines (field, column)
 // of length N3: each frequency then has its nine components at hand, and the
-// spectrum makes one round trip through HBM instead of three.
+// spectrum makes one round trip through HBM instead of three.  IP: one LDS
+// buffer (z plans of radix 2, 4 and 8: the in-place Stockham stages of the fused
+// x-y kernels), so twice the columns fit per block and a block reads 16 gz
+// contiguous bytes per (field, z) row; same arithmetic.
+template <bool IP>
 __device__ __forceinline__ void zgz_body(double2* __restrict__ Z, const GammaArgs& g, const FftPlan& pz,
-                                         const double2* __restrict__ twz, int gz, double* __restrict__ div_partial,
-                                         unsigned blk) {
+                                         const double2* __restrict__ twz, const FftDiv& gzd,
+                                         double* __restrict__ div_partial, unsigned blk) {
   extern __shared__ double2 lds[];
-  __shared__ double red[1024];
-  const int h = g.h, N3 = g.n[2], ldl = N3 + 1;
+  __shared__ double red[IP ? IP_THREADS / 64 : 1024 / 64];
+  const int h = g.h, N3 = pz.L, ldl = pz.ldl, ps = pz.ps, gz = gzd.d;
   const long M = (long)h * g.n[1], Nk = M * N3;
   const long m0 = (long)blk * gz;
   const int nl = (int)min((long)gz, M - m0);
   const int nlines = 9 * gz;
-  double2* b0 = lds;
-  double2* b1 = lds + nlines * ldl;
-  for (int i = threadIdx.x; i < 9 * N3 * gz; i += blockDim.x) {
-    int j = i % gz, t = i / gz, kz = t % N3, c = t / N3;
-    b0[(c * gz + j) * ldl + kz] = j < nl ? Z[c * Nk + (long)kz * M + m0 + j] : make_double2(0.0, 0.0);
+  double2 *A = lds, *B = lds + (IP ? 0 : nlines * ldl);
+  for (int i = threadIdx.x; i < nlines * N3; i += blockDim.x) {
+    const int t = fdiv(i, gzd), j = i - t * gz, c = fdiv(t, pz.len), kz = t - c * N3;
+    A[(c * gz + j) * ldl + lpos(kz, ps)] = j < nl ? Z[c * Nk + (long)kz * M + m0 + j] : make_double2(0.0, 0.0);
   }
   __syncthreads();
-  double2* r = lds_fft(b0, b1, nlines, N3, ldl, pz, twz, -1);
-  double2* o = r == b0 ? b1 : b0;
+  double2* r = A;
+  if (IP) lds_fft_ip<-1>(A, nlines, pz, twz);
+  else r = lds_fft<-1>(A, B, nlines, pz, twz);
+  const int ky0 = (int)(m0 / h), kx0 = (int)(m0 - (long)ky0 * h);
   double contrib = 0.0;
   for (int i = threadIdx.x; i < gz * N3; i += blockDim.x) {
-    int j = i % gz, kz = i / gz;
+    const int kz = fdiv(i, gzd), j = i - kz * gz;
     if (j >= nl) continue;
-    const long m = m0 + j;
+    int kx = kx0 + j, ky = ky0;
+    while (kx >= h) { kx -= h; ky++; }
+    double2* p = r + j * ldl + lpos(kz, ps);
     double2 P[9];
 #pragma unroll
-    for (int c = 0; c < 9; c++) P[c] = r[(c * gz + j) * ldl + kz];
-    contrib += gamma_div_point(P, (int)(m % h), (int)(m / h), kz, m == 0 && kz == 0, g);
+    for (int c = 0; c < 9; c++) P[c] = p[c * gz * ldl];
+    contrib += gamma_div_point(P, kx, ky, kz, kx == 0 && ky == 0 && kz == 0, g);
     if (g.do_gamma) {
 #pragma unroll
-      for (int c = 0; c < 9; c++) r[(c * gz + j) * ldl + kz] = P[c];
+      for (int c = 0; c < 9; c++) p[c * gz * ldl] = P[c];
     }
   }
   if (g.do_div) {
-    red[threadIdx.x] = contrib;
+    // sums of the wavefronts, then of the block
+#pragma unroll
+    for (int k = 32; k > 0; k >>= 1) contrib += __shfl_xor(contrib, k, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = contrib;
     __syncthreads();
-    for (int k = blockDim.x / 2; k > 0; k >>= 1) {
-      if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
-      __syncthreads();
+    if (threadIdx.x == 0) {
+      double s = 0.0;
+      for (unsigned w = 0; w < blockDim.x >> 6; w++) s += red[w];
+      div_partial[blk] = s;
     }
-    if (threadIdx.x == 0) div_partial[blk] = red[0];
   }
   __syncthreads();
-  double2* q = lds_fft(r, o, nlines, N3, ldl, pz, twz, +1);
-  for (int i = threadIdx.x; i < 9 * N3 * gz; i += blockDim.x) {
-    int j = i % gz, t = i / gz, kz = t % N3, c = t / N3;
-    if (j < nl) Z[c * Nk + (long)kz * M + m0 + j] = q[(c * gz + j) * ldl + kz];
+  const double2* q = r;
+  if (IP) lds_fft_ip<+1>(A, nlines, pz, twz);
+  else q = lds_fft<+1>(r, r == A ? B : A, nlines, pz, twz);
+  for (int i = threadIdx.x; i < nlines * N3; i += blockDim.x) {
+    const int t = fdiv(i, gzd), j = i - t * gz, c = fdiv(t, pz.len), kz = t - c * N3;
+    if (j < nl) Z[c * Nk + (long)kz * M + m0 + j] = q[(c * gz + j) * ldl + lpos(kz, ps)];
   }
 }
 
-__global__ void fft_zgz(double2* __restrict__ Z, GammaArgs g, FftPlan pz, const double2* __restrict__ twz, int gz,
+__global__ void fft_zgz(double2* __restrict__ Z, GammaArgs g, FftPlan pz, const double2* __restrict__ twz, FftDiv gz,
                         double* __restrict__ div_partial) {
-  zgz_body(Z, g, pz, twz, gz, div_partial, xcd_block(blockIdx.x, gridDim.x));
+  zgz_body<false>(Z, g, pz, twz, gz, div_partial, xcd_block(blockIdx.x, gridDim.x));
 }
 
-// fft_zgz with one LDS buffer (z plans of radix 2, 4 and 8: the in-place
-// Stockham stages of the fused x-y kernels), so twice the columns fit per block
-// and a block reads 16 gz contiguous bytes per (field, z) row.  Same arithmetic
-// as fft_zgz.
-__device__ __forceinline__ void zgz_ip_body(double2* __restrict__ Z, const GammaArgs& g, const FftPlan& pz,
-                                            const double2* __restrict__ twz, int gz, double* __restrict__ div_partial,
-                                            unsigned blk) {
-  extern __shared__ double2 lds[];
-  __shared__ double red[512];
-  const int h = g.h, N3 = g.n[2], ldl = N3 + 1;
-  const long M = (long)h * g.n[1], Nk = M * N3;
-  const long m0 = (long)blk * gz;
-  const int nl = (int)min((long)gz, M - m0);
-  const int nlines = 9 * gz;
-  double2* A = lds;
-  for (int i = threadIdx.x; i < 9 * N3 * gz; i += blockDim.x) {
-    int j = i % gz, t = i / gz, kz = t % N3, c = t / N3;
-    A[(c * gz + j) * ldl + kz] = j < nl ? Z[c * Nk + (long)kz * M + m0 + j] : make_double2(0.0, 0.0);
-  }
-  __syncthreads();
-  lds_fft_ip(A, nlines, N3, ldl, pz, twz, -1);
-  double contrib = 0.0;
-  for (int i = threadIdx.x; i < gz * N3; i += blockDim.x) {
-    int j = i % gz, kz = i / gz;
-    if (j >= nl) continue;
-    const long m = m0 + j;
-    double2 P[9];
-#pragma unroll
-    for (int c = 0; c < 9; c++) P[c] = A[(c * gz + j) * ldl + kz];
-    contrib += gamma_div_point(P, (int)(m % h), (int)(m / h), kz, m == 0 && kz == 0, g);
-    if (g.do_gamma) {
-#pragma unroll
-      for (int c = 0; c < 9; c++) A[(c * gz + j) * ldl + kz] = P[c];
-    }
-  }
-  if (g.do_div) {
-    red[threadIdx.x] = contrib;
-    __syncthreads();
-    for (int k = blockDim.x / 2; k > 0; k >>= 1) {
-      if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) div_partial[blk] = red[0];
-  }
-  __syncthreads();
-  lds_fft_ip(A, nlines, N3, ldl, pz, twz, +1);
-  for (int i = threadIdx.x; i < 9 * N3 * gz; i += blockDim.x) {
-    int j = i % gz, t = i / gz, kz = t % N3, c = t / N3;
-    if (j < nl) Z[c * Nk + (long)kz * M + m0 + j] = A[(c * gz + j) * ldl + kz];
-  }
-}
-
-__global__ void __launch_bounds__(512) fft_zgz_ip(double2* __restrict__ Z, GammaArgs g, FftPlan pz,
-                                                  const double2* __restrict__ twz, int gz,
-                                                  double* __restrict__ div_partial) {
-  zgz_ip_body(Z, g, pz, twz, gz, div_partial, xcd_block(blockIdx.x, gridDim.x));
+__global__ void __launch_bounds__(IP_THREADS) fft_zgz_ip(double2* __restrict__ Z, GammaArgs g, FftPlan pz,
+                                                         const double2* __restrict__ twz, FftDiv gz,
+                                                         double* __restrict__ div_partial) {
+  zgz_body<true>(Z, g, pz, twz, gz, div_partial, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // The transforms of a lockstep round: the fused kernels above over the RVEs
 // of one FFT configuration (blockIdx.y = RVE), each with its own fields and
 // Gamma arguments
-__global__ __launch_bounds__(512) void fft_xy_r2c_ip_batch(const DmkResidDev* __restrict__ R, int N1, int N2, int N3,
-                                                            FftPlan px, const double2* __restrict__ twx, FftPlan py,
-                                                            const double2* __restrict__ twy) {
+template <bool IP>
+__global__ void __launch_bounds__(IP ? IP_THREADS : 1024) fft_xy_r2c_batch(const DmkResidDev* __restrict__ R, int N3,
+                                                                          FftPlan px, const double2* __restrict__ twx,
+                                                                          FftPlan py,
+                                                                          const double2* __restrict__ twy) {
   const DmkResidDev& q = R[blockIdx.y];
-  xy_r2c_ip_body(q.Pnew, q.Z, N1, N2, N3, px, twx, py, twy, blockIdx.x);
+  xy_r2c_body<IP, IP ? IP_KU : 1>(q.Pnew, q.Z, N3, px, twx, py, twy, blockIdx.x);
 }
 
-__global__ void fft_xy_r2c_batch(const DmkResidDev* __restrict__ R, int N1, int N2, int N3, FftPlan px,
-                                 const double2* __restrict__ twx, FftPlan py, const double2* __restrict__ twy) {
+template <bool IP>
+__global__ void __launch_bounds__(IP ? IP_THREADS : 1024) fft_yx_c2r_batch(const DmkResidDev* __restrict__ R, int N3,
+                                                                          FftPlan px, const double2* __restrict__ twx,
+                                                                          FftPlan py,
+                                                                          const double2* __restrict__ twy) {
   const DmkResidDev& q = R[blockIdx.y];
-  xy_r2c_body(q.Pnew, q.Z, N1, N2, N3, px, twx, py, twy, blockIdx.x);
+  yx_c2r_body<IP, IP ? IP_KU : 1>(q.Z, q.r, N3, px, twx, py, twy, blockIdx.x);
 }
 
-__global__ __launch_bounds__(512) void fft_yx_c2r_ip_batch(const DmkResidDev* __restrict__ R, int N1, int N2, int N3,
-                                                            FftPlan px, const double2* __restrict__ twx, FftPlan py,
-                                                            const double2* __restrict__ twy) {
+template <bool IP>
+__global__ void __launch_bounds__(IP ? IP_THREADS : 1024) fft_zgz_batch(const DmkResidDev* __restrict__ R, FftPlan pz,
+                                                                       const double2* __restrict__ twz, FftDiv gz) {
   const DmkResidDev& q = R[blockIdx.y];
-  yx_c2r_ip_body(q.Z, q.r, N1, N2, N3, px, twx, py, twy, blockIdx.x);
-}
-
-__global__ void fft_yx_c2r_batch(const DmkResidDev* __restrict__ R, int N1, int N2, int N3, FftPlan px,
-                                 const double2* __restrict__ twx, FftPlan py, const double2* __restrict__ twy) {
-  const DmkResidDev& q = R[blockIdx.y];
-  yx_c2r_body(q.Z, q.r, N1, N2, N3, px, twx, py, twy, blockIdx.x);
-}
-
-__global__ void __launch_bounds__(512) fft_zgz_ip_batch(const DmkResidDev* __restrict__ R, FftPlan pz,
-                                                        const double2* __restrict__ twz, int gz) {
-  const DmkResidDev& q = R[blockIdx.y];
-  zgz_ip_body(q.Z, q.g, pz, twz, gz, q.divp, xcd_block(blockIdx.x, gridDim.x));
-}
-
-__global__ void fft_zgz_batch(const DmkResidDev* __restrict__ R, FftPlan pz, const double2* __restrict__ twz,
-                              int gz) {
-  const DmkResidDev& q = R[blockIdx.y];
-  zgz_body(q.Z, q.g, pz, twz, gz, q.divp, xcd_block(blockIdx.x, gridDim.x));
+  zgz_body<IP>(q.Z, q.g, pz, twz, gz, q.divp, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // utilities_curlRMS (spectral_utilities.f90:697-757): per frequency the
@@ -858,10 +782,8 @@ __global__ void __launch_bounds__(256) curl_kernel(const double2* __restrict__ Z
   const long f = (long)blockIdx.x * blockDim.x + threadIdx.x;
   double contrib = 0.0;
   if (f < Nk) {
-    int kx = (int)(f % g.h);
-    long r = f / g.h;
-    int ky = (int)(r % g.n[1]);
-    int kz = (int)(r / g.n[1]);
+    int kx, ky, kz;
+    freq_of((unsigned)f, g, kx, ky, kz);
     const double TAU = 6.283185307179586;
     double w[3];
     w[0] = TAU * (double)kx / g.size[0];
@@ -913,10 +835,8 @@ __global__ void __launch_bounds__(256) galerkin_kernel(double2* __restrict__ Z, 
   const long f = (long)blockIdx.x * blockDim.x + threadIdx.x;
   double contrib = 0.0;
   if (f < Nk) {
-    int kx = (int)(f % g.h);
-    long r = f / g.h;
-    int ky = (int)(r % g.n[1]);
-    int kz = (int)(r / g.n[1]);
+    int kx, ky, kz;
+    freq_of((unsigned)f, g, kx, ky, kz);
     const double TAU = 6.283185307179586;
     double a[3];
     a[0] = TAU * (double)kx / g.size[0];
@@ -992,10 +912,8 @@ __global__ void coords_freq_kernel(const double2* __restrict__ Fh, double2* __re
   const long Nk = (long)g.h * g.n[1] * g.n[2];
   const long f = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= Nk) return;
-  int kx = (int)(f % g.h);
-  long r = f / g.h;
-  int ky = (int)(r % g.n[1]);
-  int kz = (int)(r / g.n[1]);
+  int kx, ky, kz;
+  freq_of((unsigned)f, g, kx, ky, kz);
   const double TAU = 6.283185307179586;
   double a[3] = {TAU * (double)kx / g.size[0], TAU * wrap_freq(ky, g.n[1]) / g.size[1],
                  TAU * wrap_freq(kz, g.n[2]) / g.size[2]};
@@ -1056,6 +974,16 @@ __global__ void coords_nodes_kernel(const double* __restrict__ u, CoordsArgs c, 
 }  // namespace
 
 // ---------------------------------------------------------------------------- host
+FftDiv dmk_fft_div(int d) {
+  FftDiv v;
+  int lg = 0;
+  while ((1 << lg) < d) lg++;
+  v.d = d;
+  v.s = 14 + lg;
+  v.m = (uint32_t)((1ull << v.s) / (unsigned)d) + 1;
+  return v;
+}
+
 static FftPlan make_plan(int L) {
   FftPlan p{};
   p.L = L;
@@ -1065,6 +993,17 @@ static FftPlan make_plan(int L) {
   while (n % 2 == 0) { p.radix[p.nstages++] = 2; n /= 2; }
   for (int f = 3; n > 1; f += 2)
     while (n % f == 0) { p.radix[p.nstages++] = f; n /= f; }
+  for (int s = 0, ns = 1; s < p.nstages; ns *= p.radix[s++]) {
+    p.nb[s] = dmk_fft_div(L / p.radix[s]);
+    p.ns[s] = dmk_fft_div(ns);
+  }
+  p.len = dmk_fft_div(L);
+  p.half = dmk_fft_div(L / 2 + 1);
+  // the first radix-8 stage writes every eighth entry: one pad per eight spreads
+  // them over the banks.  64 | L keeps the other stages' strides constant; long
+  // lines are left dense for their LDS.  An odd line distance spreads the columns.
+  p.ps = L % 64 == 0 && L <= 1024 ? 3 : 31;
+  p.ldl = (L + (p.ps < 31 ? L >> p.ps : 0)) | 1;
   return p;
 }
 
@@ -1157,108 +1096,85 @@ void dmk_fft_free(DmkFFT* fft) {
 }
 
 static const size_t FFT_LDS_MAX = 64 * 1024;
-// the fused x-y kernels may take more (the MI355X allows 160 KB per block)
+// the fused kernels may take more (the MI355X allows 160 KB per block)
 static const size_t FFT_XY_LDS_MAX = 160 * 1024;
 
-static size_t xy_lds(const DmkFFT* fft) {
-  const int N1 = fft->n[0], N2 = fft->n[1], h = fft->h, np = (N2 + 1) / 2;
-  size_t a = (size_t)np * (N1 + 1), b = (size_t)h * (N2 + 1);
-  return 2 * sizeof(double2) * (a > b ? a : b);
+// LDS of `lines` lines of axis d in two buffers
+static size_t lines_lds(const DmkFFT* fft, int d, int lines) {
+  return 2 * sizeof(double2) * (size_t)lines * fft->plan[d].ldl;
+}
+
+static size_t xy_lds(const DmkFFT* fft, int ip) {
+  return (ip ? 1 : 2) * sizeof(double2) * (size_t)xy_buf(fft->plan[0], fft->plan[1]);
 }
 
 static void launch_xy_r2c(const DmkFFT* fft, int howmany, const double* in, double2* out, int threads, int ip,
                           hipStream_t s) {
-  if (ip)
-    hipLaunchKernelGGL(fft_xy_r2c_ip, dim3(howmany * fft->n[2]), dim3(threads), xy_lds(fft) / 2, s, in, out,
-                       fft->n[0], fft->n[1], fft->n[2], fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
-  else
-    hipLaunchKernelGGL(fft_xy_r2c, dim3(howmany * fft->n[2]), dim3(threads), xy_lds(fft), s, in, out, fft->n[0],
-                       fft->n[1], fft->n[2], fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
+  hipLaunchKernelGGL(ip ? fft_xy_r2c_ip : fft_xy_r2c, dim3(howmany * fft->n[2]), dim3(threads), xy_lds(fft, ip), s, in,
+                     out, fft->n[2], fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
 }
 
 static void launch_yx_c2r(const DmkFFT* fft, int howmany, const double2* in, double* out, int threads, int ip,
                           hipStream_t s) {
-  if (ip)
-    hipLaunchKernelGGL(fft_yx_c2r_ip, dim3(howmany * fft->n[2]), dim3(threads), xy_lds(fft) / 2, s, in, out,
-                       fft->n[0], fft->n[1], fft->n[2], fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
-  else
-    hipLaunchKernelGGL(fft_yx_c2r, dim3(howmany * fft->n[2]), dim3(threads), xy_lds(fft), s, in, out, fft->n[0],
-                       fft->n[1], fft->n[2], fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
+  hipLaunchKernelGGL(ip ? fft_yx_c2r_ip : fft_yx_c2r, dim3(howmany * fft->n[2]), dim3(threads), xy_lds(fft, ip), s, in,
+                     out, fft->n[2], fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
 }
 
-// the in-place x-y kernels need radix 2/4/8 plans and every stage, unpack and
-// pack to fit the per-thread register slots at this block size
-static bool xy_ip_fits(const DmkFFT* fft, int threads) {
-  const int N1 = fft->n[0], N2 = fft->n[1], h = fft->h, np = (N2 + 1) / 2;
-  for (int d = 0; d < 2; d++) {
-    const FftPlan& p = fft->plan[d];
-    const int lines = d == 0 ? np : h, L = fft->n[d];
-    for (int st = 0; st < p.nstages; st++) {
-      const int R = p.radix[st];
-      if (R != 2 && R != 4 && R != 8) return false;
-      if ((long)lines * (L / R) > (long)IP_KMAX * threads) return false;
-    }
+// the in-place kernels need radix 2/4/8 plans and every stage of `lines` lines
+// of axis d to fit the per-thread butterfly slots at this block size
+static bool ip_fits(const DmkFFT* fft, int d, int lines, int threads) {
+  const FftPlan& p = fft->plan[d];
+  for (int st = 0; st < p.nstages; st++) {
+    const int R = p.radix[st];
+    if (R != 2 && R != 4 && R != 8) return false;
+    if ((long)lines * (p.L / R) > (long)(IP_VALS / R) * threads) return false;
   }
-  return (long)N2 * h <= (long)IP_KU * threads && (long)np * N1 <= (long)IP_KU * threads;
+  return threads <= IP_THREADS;
+}
+
+// ... and the x-y kernels the pairs carried between the passes
+static bool xy_ip_fits(const DmkFFT* fft, int threads) {
+  const int h = fft->h, np = (fft->n[1] + 1) / 2;
+  return ip_fits(fft, 0, np, threads) && ip_fits(fft, 1, h, threads) && (long)np * h <= (long)IP_KU * threads;
 }
 
 static void launch_x_r2c(const DmkFFT* fft, int howmany, const double* in, double2* out, int ppb, hipStream_t s) {
-  const int N1 = fft->n[0];
   int nl = howmany * fft->n[1] * fft->n[2];
   int nblk = (nl + 2 * ppb - 1) / (2 * ppb);
-  size_t lds = sizeof(double2) * 2 * ppb * (N1 + 1);
-  hipLaunchKernelGGL(fft_x_r2c, dim3(nblk), dim3(256), lds, s, in, out, nl, fft->plan[0], fft->tw[0], ppb);
+  hipLaunchKernelGGL(fft_x_r2c, dim3(nblk), dim3(256), lines_lds(fft, 0, ppb), s, in, out, nl, fft->plan[0],
+                     fft->tw[0], ppb);
 }
 
 static void launch_x_c2r(const DmkFFT* fft, int howmany, const double2* in, double* out, int ppb, hipStream_t s) {
-  const int N1 = fft->n[0];
   int nl = howmany * fft->n[1] * fft->n[2];
   int nblk = (nl + 2 * ppb - 1) / (2 * ppb);
-  size_t lds = sizeof(double2) * 2 * ppb * (N1 + 1);
-  hipLaunchKernelGGL(fft_x_c2r, dim3(nblk), dim3(256), lds, s, in, out, nl, fft->plan[0], fft->tw[0], ppb);
+  hipLaunchKernelGGL(fft_x_c2r, dim3(nblk), dim3(256), lines_lds(fft, 0, ppb), s, in, out, nl, fft->plan[0],
+                     fft->tw[0], ppb);
 }
 
 // y (axis 1) or z (axis 2) pass over the half spectra, in place
 static void launch_strided(const DmkFFT* fft, int howmany, double2* data, int axis, int gx, int sign, hipStream_t s) {
   const int N2 = fft->n[1], N3 = fft->n[2], h = fft->h;
   const long Nk = (long)h * N2 * N3;
-  const int L = fft->n[axis];
-  int nch = (h + gx - 1) / gx;
-  size_t lds = sizeof(double2) * 2 * gx * (L + 1);
-  if (axis == 1)
-    hipLaunchKernelGGL(fft_strided, dim3(howmany * N3 * nch), dim3(256), lds, s, data, h, gx, N3, Nk, (long)h * N2,
-                       (long)h, fft->plan[1], fft->tw[1], sign);
-  else
-    hipLaunchKernelGGL(fft_strided, dim3(howmany * N2 * nch), dim3(256), lds, s, data, h, gx, N2, Nk, (long)h,
-                       (long)h * N2, fft->plan[2], fft->tw[2], sign);
+  const int nch = (h + gx - 1) / gx, M = axis == 1 ? N3 : N2;
+  const long outer = axis == 1 ? (long)h * N2 : h, stride = axis == 1 ? h : (long)h * N2;
+  hipLaunchKernelGGL(sign < 0 ? fft_strided<-1> : fft_strided<+1>, dim3(howmany * M * nch), dim3(256),
+                     lines_lds(fft, axis, gx), s, data, h, dmk_fft_div(gx), M, Nk, outer, stride, fft->plan[axis],
+                     fft->tw[axis]);
 }
 
+// (beside a few static sums)
+static const size_t FFT_ZGZ_LDS_MAX = FFT_XY_LDS_MAX - 256;
 static size_t zgz_lds(const DmkFFT* fft, int gz, int ip) {
-  return (ip ? 1 : 2) * sizeof(double2) * 9 * gz * (fft->n[2] + 1);
-}
-
-// the single-buffer z kernel needs a radix 2/4/8 z plan whose every stage fits
-// the per-thread butterfly slots at this block size
-static bool zgz_ip_fits(const DmkFFT* fft, int gz, int threads) {
-  const FftPlan& p = fft->plan[2];
-  for (int st = 0; st < p.nstages; st++) {
-    const int R = p.radix[st];
-    if (R != 2 && R != 4 && R != 8) return false;
-    if ((long)9 * gz * (fft->n[2] / R) > (long)IP_KMAX * threads) return false;
-  }
-  return true;
+  return (ip ? 1 : 2) * sizeof(double2) * 9 * gz * (size_t)fft->plan[2].ldl;
 }
 
 static void launch_zgz(const DmkFFT* fft, double2* Z, const GammaArgs* g, int gz, int threads, int ip,
                        double* div_partial, hipStream_t s) {
   const long M = (long)fft->h * fft->n[1];
   unsigned nb = (unsigned)((M + gz - 1) / gz);
-  if (ip)
-    hipLaunchKernelGGL(fft_zgz_ip, dim3(nb), dim3(threads), zgz_lds(fft, gz, 1), s, Z, *g, fft->plan[2],
-                       fft->tw[2], gz, div_partial);
-  else
-    hipLaunchKernelGGL(fft_zgz, dim3(nb), dim3(threads), zgz_lds(fft, gz, 0), s, Z, *g, fft->plan[2], fft->tw[2],
-                       gz, div_partial);
+  hipLaunchKernelGGL(ip ? fft_zgz_ip : fft_zgz, dim3(nb), dim3(threads), zgz_lds(fft, gz, ip), s, Z, *g, fft->plan[2],
+                     fft->tw[2], dmk_fft_div(gz), div_partial);
 }
 
 int dmk_fft_tune(DmkFFT* fft, double2* cscratch, double* rscratch, hipStream_t s) {
@@ -1283,7 +1199,7 @@ int dmk_fft_tune(DmkFFT* fft, double2* cscratch, double* rscratch, hipStream_t s
     const int L = fft->n[0];
     float best = 1e30f;
     for (int ppb : {1024 / L, 512 / L, 256 / L, 2048 / L}) {
-      if (ppb < 1 || sizeof(double2) * 2 * ppb * (L + 1) > FFT_LDS_MAX) continue;
+      if (ppb < 1 || lines_lds(fft, 0, ppb) > FFT_LDS_MAX) continue;
       float t = timed([&] { launch_x_r2c(fft, howmany, rscratch, cscratch, ppb, s); });
       if (t < best) { best = t; fft->gx[0] = ppb; }
     }
@@ -1297,7 +1213,7 @@ int dmk_fft_tune(DmkFFT* fft, double2* cscratch, double* rscratch, hipStream_t s
     int last = -1;
     for (int nch = 1; nch <= fft->h && nch <= 16; nch++) {
       int gx = (fft->h + nch - 1) / nch;
-      if (gx == last || sizeof(double2) * 2 * gx * (L + 1) > FFT_LDS_MAX) continue;
+      if (gx == last || lines_lds(fft, axis, gx) > FFT_LDS_MAX) continue;
       last = gx;
       float t = timed([&] { launch_strided(fft, howmany, cscratch, axis, gx, -1, s); });
       if (t < best) { best = t; fft->gx[axis] = gx; }
@@ -1309,17 +1225,19 @@ int dmk_fft_tune(DmkFFT* fft, double2* cscratch, double* rscratch, hipStream_t s
   fft->xy_threads = 0;
   fft->xy_ip = 0;
   const char* force = getenv("DMK_FFT_XY");
-  if (fft->n[0] >= 2 && fft->n[1] >= 2 && xy_lds(fft) <= FFT_XY_LDS_MAX && !(force && force[0] == '0')) {
+  if (fft->n[0] >= 2 && fft->n[1] >= 2 && !(force && force[0] == '0')) {
     float sep = timed([&] { launch_x_r2c(fft, howmany, rscratch, cscratch, fft->gx[0], s); }) + t_y;
     if (force && (force[0] == '1' || force[0] == '2')) sep = 1e30f;
-    for (int ip = 0; ip <= 1; ip++)
-      for (int th : {256, 512, 1024}) {
-        if (ip && (th > 512 || !xy_ip_fits(fft, th))) continue;   // launch bounds of the in-place kernels
+    for (int ip = 0; ip <= 1; ip++) {
+      if (xy_lds(fft, ip) > FFT_XY_LDS_MAX) continue;
+      for (int th : {256, 384, 512, 576, 640, 1024}) {
+        if (ip ? !xy_ip_fits(fft, th) : th % 256 != 0) continue;
         if (force && force[0] == '1' && ip) continue;       // DMK_FFT_XY=1: the two-buffer variant
         if (force && force[0] == '2' && !ip) continue;      // DMK_FFT_XY=2: the in-place variant
         float t = timed([&] { launch_xy_r2c(fft, howmany, rscratch, cscratch, th, ip, s); });
         if (t < sep) { sep = t; fft->xy_threads = th; fft->xy_ip = ip; }
       }
+    }
   }
   // fused z passes and Gamma against the separate kernels (a reference medium
   // with an invertible acoustic tensor; DMK_FFT_ZGZ=0 / 1 / 2 forces separate /
@@ -1343,14 +1261,14 @@ int dmk_fft_tune(DmkFFT* fft, double2* cscratch, double* rscratch, hipStream_t s
     if (fz && (fz[0] == '1' || fz[0] == '2')) sep = 1e30f;
     bool any_ip = false;
     for (int gz : {2, 4, 8, 16})
-      for (int th : {256, 512}) any_ip |= zgz_lds(fft, gz, 1) <= FFT_XY_LDS_MAX && zgz_ip_fits(fft, gz, th);
+      for (int th : {256, 512}) any_ip |= zgz_lds(fft, gz, 1) <= FFT_ZGZ_LDS_MAX && ip_fits(fft, 2, 9 * gz, th);
     for (int ip = 0; ip <= 1; ip++)
-      for (int gz : {1, 2, 4, 8, 16}) {
-        if (zgz_lds(fft, gz, ip) > FFT_XY_LDS_MAX) continue;
+      for (int gz : {1, 2, 4, 7, 8, 16}) {
+        if (zgz_lds(fft, gz, ip) > FFT_ZGZ_LDS_MAX) continue;
         if (fz && fz[0] == '1' && ip) continue;                 // DMK_FFT_ZGZ=1: the two-buffer kernel
         if (fz && fz[0] == '2' && any_ip && !ip) continue;      // DMK_FFT_ZGZ=2: the single-buffer kernel
-        for (int th : {256, 512}) {
-          if (ip && !zgz_ip_fits(fft, gz, th)) continue;
+        for (int th : {256, 512, 576}) {
+          if (ip ? !ip_fits(fft, 2, 9 * gz, th) : th % 256 != 0) continue;
           float t = timed([&] { launch_zgz(fft, cscratch, &g, gz, th, ip, part, s); });
           if (t < sep) { sep = t; fft->zgz_g = gz; fft->zgz_threads = th; fft->zgz_ip = ip; }
         }
@@ -1384,28 +1302,18 @@ int dmk_fft_c2r_xy(const DmkFFT* fft, int howmany, double2* in, double* out, hip
 int dmk_transform_batch(const DmkFFT* fft, const DmkResidDev* R, int nr, hipStream_t s) {
   if (nr < 1) return 0;
   if (!fft->xy_threads || !fft->zgz_g) return 1;
-  const int N1 = fft->n[0], N2 = fft->n[1], N3 = fft->n[2];
+  const int N2 = fft->n[1], N3 = fft->n[2];
   const dim3 gxy(9 * N3, nr);
   const long M = (long)fft->h * N2;
   const dim3 gzz((unsigned)((M + fft->zgz_g - 1) / fft->zgz_g), nr);
-  if (fft->xy_ip)
-    hipLaunchKernelGGL(fft_xy_r2c_ip_batch, gxy, dim3(fft->xy_threads), xy_lds(fft) / 2, s, R, N1, N2, N3,
-                       fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
-  else
-    hipLaunchKernelGGL(fft_xy_r2c_batch, gxy, dim3(fft->xy_threads), xy_lds(fft), s, R, N1, N2, N3, fft->plan[0],
-                       fft->tw[0], fft->plan[1], fft->tw[1]);
-  if (fft->zgz_ip)
-    hipLaunchKernelGGL(fft_zgz_ip_batch, gzz, dim3(fft->zgz_threads), zgz_lds(fft, fft->zgz_g, 1), s, R,
-                       fft->plan[2], fft->tw[2], fft->zgz_g);
-  else
-    hipLaunchKernelGGL(fft_zgz_batch, gzz, dim3(fft->zgz_threads), zgz_lds(fft, fft->zgz_g, 0), s, R, fft->plan[2],
-                       fft->tw[2], fft->zgz_g);
-  if (fft->xy_ip)
-    hipLaunchKernelGGL(fft_yx_c2r_ip_batch, gxy, dim3(fft->xy_threads), xy_lds(fft) / 2, s, R, N1, N2, N3,
-                       fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
-  else
-    hipLaunchKernelGGL(fft_yx_c2r_batch, gxy, dim3(fft->xy_threads), xy_lds(fft), s, R, N1, N2, N3, fft->plan[0],
-                       fft->tw[0], fft->plan[1], fft->tw[1]);
+  const FftPlan &px = fft->plan[0], &py = fft->plan[1], &pz = fft->plan[2];
+  const dim3 txy(fft->xy_threads), tz(fft->zgz_threads);
+  hipLaunchKernelGGL(fft->xy_ip ? fft_xy_r2c_batch<true> : fft_xy_r2c_batch<false>, gxy, txy, xy_lds(fft, fft->xy_ip),
+                     s, R, N3, px, fft->tw[0], py, fft->tw[1]);
+  hipLaunchKernelGGL(fft->zgz_ip ? fft_zgz_batch<true> : fft_zgz_batch<false>, gzz, tz,
+                     zgz_lds(fft, fft->zgz_g, fft->zgz_ip), s, R, pz, fft->tw[2], dmk_fft_div(fft->zgz_g));
+  hipLaunchKernelGGL(fft->xy_ip ? fft_yx_c2r_batch<true> : fft_yx_c2r_batch<false>, gxy, txy, xy_lds(fft, fft->xy_ip),
+                     s, R, N3, px, fft->tw[0], py, fft->tw[1]);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
