@@ -909,69 +909,56 @@ stress_kernel_batch(const DmkStressItem* __restrict__ items, int n_items) {
                            it->phase_id, num, it->dt, b - it->block0, sh);
 }
 
-// math_rotationalPart (src/math.f90:1004-1043)
+// The rotation R of F = R U (math_rotationalPart, src/math.f90:1004-1043) as the
+// limit of R <- (R + R^-T)/2 from F (Higham, SIAM J. Sci. Stat. Comput. 7(4) 1986),
+// which converges quadratically: a step below 1e-8 leaves an error below 1e-16.
+// An elastic F takes three steps.
 DI void rotational_part(const double* F, double* R) {
-  const double TAU = 6.283185307179586;
-  double C[9], FF[9], FC[9];
-  m_mul_tn(F, F, C);
-  double I1 = C[0] + C[4] + C[8];
-  double I2 = C[0] * C[4] + C[0] * C[8] + C[4] * C[8] - (C[1] * C[1] + C[2] * C[2] + C[5] * C[5]);
-  double I3 = -(C[0] * C[5] * C[5] + C[4] * C[2] * C[2] + C[8] * C[1] * C[1]) + C[0] * C[4] * C[8]
-            + 2.0 * C[1] * C[2] * C[5];
-  m_mul(F, F, FF);
-  double trF = F[0] + F[4] + F[8];
-  double IF2 = 0.5 * (trF * trF - (FF[0] + FF[4] + FF[8]));
-  double l[3];
-  double q = fmax(I1 * I1 - 3.0 * I2, 0.0);
-  double x = pow(q, 1.5);
-  if (!dEq0(x)) {
-    double arg = fmin(fmax((I1 * I1 * I1 - 4.5 * I1 * I2 + 13.5 * I3) / x, -1.0), 1.0);
-    double Phi = acos(arg);
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      double lam = I1 + (2.0 * sqrt(q)) * cos((Phi - TAU * (double)(k + 1)) / 3.0);
-      l[k] = sqrt(fmax(lam, 0.0) / 3.0);
+  for (int k = 0; k < 9; k++) R[k] = F[k];
+#pragma unroll 1
+  for (int it = 0; it < 64; it++) {
+    double c[9];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        const int i1 = (i + 1) % 3, i2 = (i + 2) % 3, j1 = (j + 1) % 3, j2 = (j + 2) % 3;
+        c[3 * i + j] = R[3 * i1 + j1] * R[3 * i2 + j2] - R[3 * i1 + j2] * R[3 * i2 + j1];
+      }
+    const double g = 0.5 * dmk_rcp(R[0] * c[0] + R[1] * c[1] + R[2] * c[2]);
+    double d2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      const double d = fma(g, c[k], -0.5 * R[k]);
+      d2 = fma(d, d, d2);
+      R[k] += d;
     }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 3; k++) l[k] = sqrt(I1 / 3.0);
+    if (!(d2 > 1.0e-16)) break;
   }
-  double U1 = l[0] + l[1] + l[2], U2 = l[0] * l[1] + l[1] * l[2] + l[2] * l[0];
-  m_mul(F, C, FC);
-#pragma unroll
-  for (int i = 0; i < 3; i++)
-#pragma unroll
-    for (int j = 0; j < 3; j++)
-      R[3 * i + j] = U1 * IF2 * (i == j ? 1.0 : 0.0) + (U1 * U1 - U2) * F[3 * i + j] - U1 * trF * F[3 * j + i]
-                   + U1 * FF[3 * j + i] - FC[3 * i + j];
-  double d = pow(m_det(R), -1.0 / 3.0);
-#pragma unroll
-  for (int k = 0; k < 9; k++) R[k] *= d;
 }
 
-// om2qu (src/rotations.f90:486-514), P = -1
+// om2qu (src/rotations.f90:486-514), P = -1: the largest of 4 q_k^2 (by the
+// reference's comparisons) gives its component, which divides the others; the
+// four cases share one root
 DI void om2qu(const double* om, double* qu) {
-  double tr = om[0] + om[4] + om[8];
-  double s;
-  if (tr > 0.0) {
-    s = 0.5 / sqrt(tr + 1.0);
-    qu[0] = 0.25 / s; qu[1] = (om[7] - om[5]) * s; qu[2] = (om[2] - om[6]) * s; qu[3] = (om[3] - om[1]) * s;
-  } else if (om[0] > om[4] && om[0] > om[8]) {
-    s = 2.0 * sqrt(1.0 + om[0] - om[4] - om[8]);
-    qu[0] = (om[7] - om[5]) / s; qu[1] = 0.25 * s; qu[2] = (om[1] + om[3]) / s; qu[3] = (om[2] + om[6]) / s;
-  } else if (om[4] > om[8]) {
-    s = 2.0 * sqrt(1.0 + om[4] - om[0] - om[8]);
-    qu[0] = (om[2] - om[6]) / s; qu[1] = (om[1] + om[3]) / s; qu[2] = 0.25 * s; qu[3] = (om[5] + om[7]) / s;
-  } else {
-    s = 2.0 * sqrt(1.0 + om[8] - om[0] - om[4]);
-    qu[0] = (om[3] - om[1]) / s; qu[1] = (om[2] + om[6]) / s; qu[2] = (om[5] + om[7]) / s; qu[3] = 0.25 * s;
-  }
+  const double tr = om[0] + om[4] + om[8];
+  const bool c0 = tr > 0.0, c1 = om[0] > om[4] && om[0] > om[8], c2 = om[4] > om[8];
+  const double t = c0 ? tr + 1.0
+                      : (c1 ? 1.0 + om[0] - om[4] - om[8]
+                            : (c2 ? 1.0 + om[4] - om[0] - om[8] : 1.0 + om[8] - om[0] - om[4]));
+  const double h = 0.5 * dmk_rsq(t), big = t * h;
+  const double m0 = (om[7] - om[5]) * h, m1 = (om[2] - om[6]) * h, m2 = (om[3] - om[1]) * h;
+  const double p0 = (om[5] + om[7]) * h, p1 = (om[2] + om[6]) * h, p2 = (om[1] + om[3]) * h;
+  qu[0] = c0 ? big : (c1 ? m0 : (c2 ? m1 : m2));
+  qu[1] = c0 ? m0 : (c1 ? big : (c2 ? p2 : p1));
+  qu[2] = c0 ? m1 : (c1 ? p2 : (c2 ? big : p0));
+  qu[3] = c0 ? m2 : (c1 ? p1 : (c2 ? p0 : big));
   if (signbit(qu[0])) for (int k = 0; k < 4; k++) qu[k] = -qu[k];
   for (int k = 1; k < 4; k++) if (!dEq0(qu[k])) qu[k] = -qu[k];
-  double n = sqrt(qu[0] * qu[0] + qu[1] * qu[1] + qu[2] * qu[2] + qu[3] * qu[3]);
-  for (int k = 0; k < 4; k++) qu[k] /= n;
+  const double n = dmk_rsq(qu[0] * qu[0] + qu[1] * qu[1] + qu[2] * qu[2] + qu[3] * qu[3]);
+  for (int k = 0; k < 4; k++) qu[k] *= n;
 }
-
 
 // row r (runtime, uniform) of a register 3x3 without dynamic register indexing
 DI void row3(const double* M, int r, double* v) {
@@ -979,138 +966,268 @@ DI void row3(const double* M, int r, double* v) {
   for (int j = 0; j < 3; j++) v[j] = r == 0 ? M[j] : (r == 1 ? M[3 + j] : M[6 + j]);
 }
 
+// A E_k B^T for the symmetric basis tensor E_k (k a compile-time constant)
+DI void basis_between(const double* A, int k, const double* B, double* T) {
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+      const double* a = A + 3 * i;
+      const double* b = B + 3 * m;
+      double v;
+      switch (k) {
+        case 0: v = R2 * (a[0] * b[0] - a[1] * b[1]); break;
+        case 1: v = R6 * (a[0] * b[0] + a[1] * b[1] - 2.0 * (a[2] * b[2])); break;
+        case 2: v = R2 * (a[1] * b[2] + a[2] * b[1]); break;
+        case 3: v = R2 * (a[0] * b[2] + a[2] * b[0]); break;
+        case 4: v = R2 * (a[0] * b[1] + a[1] * b[0]); break;
+        default: v = R3 * (a[0] * b[0] + a[1] * b[1] + a[2] * b[2]); break;
+      }
+      T[3 * i + m] = v;
+    }
+}
+
+// a, b, c, d summed over the wavefront: every lane of the k-th row of 16 lanes
+// holds the sum of the k-th.  Two swaps of half-waves and rows fold four values
+// into one register, four rotations within the rows finish them: 21 instructions
+// for four sums instead of 18 for each.
+DI void swap_halves(double& a, double& b) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  a = __hiloint2double(hi[0], lo[0]);
+  b = __hiloint2double(hi[1], lo[1]);
+}
+DI void swap_rows(double& a, double& b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  a = __hiloint2double(hi[0], lo[0]);
+  b = __hiloint2double(hi[1], lo[1]);
+}
+template <int ROR>
+DI double row_ror(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x120 + ROR, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x120 + ROR, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+DI double wave_rows(double a, double b, double c, double d) {
+  swap_halves(a, c);
+  double s = a + c;       // lower half: a, upper half: c
+  swap_halves(b, d);
+  double t = b + d;
+  swap_rows(s, t);
+  s += t;                 // rows: a, b, c, d
+  s += row_ror<8>(s);
+  s += row_ror<4>(s);
+  s += row_ror<2>(s);
+  s += row_ror<1>(s);
+  return s;
+}
+
 // Orientation and consistent tangent of the homogenization (one constituent,
 // v = 1) for a response in which every cell converged (flag[0] == ST_OK).
-// Also writes the squared Frobenius norm of each cell's dPdF, summed in
-// Fortran element order (the C_minMaxAvg selection works on it).
+// Also writes the squared Frobenius norm of each cell's dPdF and, with part, per
+// work-group its 81 sums and the extrema of the norms (dmk_stiffness_averages),
+// to which every phase adds its cells; reading dPdF again for the sums took 38 us
+// at 64^3.
 //
 // Column (k, l): dS = dS/dF_kl solves dS + dt sum_a dg_a C:sym(G2 P_a) (P_nS_a : dS)
 // = C:sym(X), X = F_e(k,:) (x) F_p^-1(l,:), G2 = F_e^T A2.  As in the stress
 // integration the sum acts through the E coordinates z of dS alone: N z = E:X with
 // N_kl = delta_kl / C_k + dt E_k : (G2 W_l), one 5x5 (6x6) factorisation for the
-// nine columns; then t = sum_a dg_a P_a (P_nS_a : dS) = sum_l z_l W_l and
-// dS = C:sym(X - dt G2 t), without a loop over the slip systems per column.
+// nine columns; then t = sum_a dg_a P_a (P_nS_a : dS) = sum_l z_l W_l,
+// dS = sum_k z_k E_k with z_6 = C_6 E_6 : (X - dt G2 t), and with
+// D = -dt F_p0^-1 t the derivative of F_p^-1
+//   dP = e_k (x) (F_p^-1 S F_p^-T)(l,:) + F (D S F_p^-T + F_p^-1 (dS F_p^-T + S D^T))
+//      = e_k (x) (F_p^-1 S F_p^-T)(l,:) + sum_l z_l T_l,
+// T_l = F F_p^-1 E_l F_p^-T - dt (F F_p0^-1 W_l S F_p^-T + F F_p^-1 S W_l^T F_p0^-T):
+// the six T_l are formed once, a column is then a 5x5 solve and 54 products.
+// The traffic (57 values a cell in, 86 out: 60 us at 64^3 at copy rate) and the
+// latency of a wavefront's chain bound it: one wavefront a SIMD, all inputs loaded
+// at once.  64^3 cells of the cF tension 116 us, with stiffness_averages 128; a
+// column at a time, with the averages from dPdF, took 155 + 58 us.  Two
+// wavefronts a SIMD, with spills: 134 us without the sums, against 98 us.
 template <int NSL, bool QP, bool NS>
-__global__ void __launch_bounds__(SWG) tangent_kernel(DmkMPDev mp, const DmkPhaseDev* __restrict__ ph_,
-                                                      int phase_id, double dt, const int* __restrict__ flag,
-                                                      double* __restrict__ dPdF, double* __restrict__ nrm) {
+__global__ void __launch_bounds__(SWG) __attribute__((amdgpu_waves_per_eu(1)))
+tangent_kernel(DmkMPDev mp, const DmkPhaseDev* __restrict__ ph_, int phase_id, double dt,
+               const int* __restrict__ flag, double* __restrict__ dPdF, double* __restrict__ nrm,
+               double* __restrict__ part, double* __restrict__ pmax, double* __restrict__ pmin) {
   constexpr int RK = sym_rank<NS>();
   PhPtr ph = (PhPtr)ph_;
-  __shared__ double ixi[NSL][SWG], gl[NSL][SWG];
+  // [row][lane]: 1/xi and the rate derivatives per system; then W_l in rows 8 l to
+  // 8 l + 7, where T_l (but its last entry) takes its place
+  __shared__ double sh[(2 * NSL > 8 * RK ? 2 * NSL : 8 * RK)][SWG];
+  __shared__ double sums[81];
   const int lane = threadIdx.x;
-  const int e = blockIdx.x * SWG + lane;
-  if (e >= mp.N || flag[0] != ST_OK) return;
-  if (mp.phase[e] != phase_id) return;
+  if (flag[0] != ST_OK) return;
+  // lanes without a cell of this phase go along, for the sums over the wavefront
+  const int e = min((int)(blockIdx.x * SWG) + lane, mp.N - 1);
+  const bool act = (int)(blockIdx.x * SWG) + lane < mp.N && mp.phase[e] == phase_id;
+  const bool first = phase_id == 0;
+  if (!__any(act)) {
+    if (part && first) {
+      for (int c = lane; c < 81; c += SWG) part[81l * blockIdx.x + c] = 0.0;
+      if (lane == 0) { pmax[blockIdx.x] = 0.0; pmin[blockIdx.x] = DBL_MAX; }
+    }
+    return;
+  }
   const Lane ln = make_lane(mp.N, e);
-  double Fe[9];
-  m_load(mp.Fe, ln, Fe);
-  {
-    double R[9], Rt[9], q[4];
-    rotational_part(Fe, R);
-    m_transpose(R, Rt);
-    om2qu(Rt, q);
+  double N[RK * RK], rd[RK], v0[RK], tau[RK], g6[RK];
+  double T6[9], T8[RK];       // T_6 (Schmid law) and the last entries of T_1..T_RK
+  // every input at once: one trip to memory
+  double xi[NSL], S[9], Fp[9], Fp0[9], F[9], Fe[9];
 #pragma unroll
-    for (int k = 0; k < 4; k++) st(mp.O, ln, k, q[k]);
-  }
-  double H[5][RK], K[3][RK];
-  {
-    double S[9], s[6], l[5], k3[3];
-    unsigned posm;
-#pragma unroll 4
-    for (int r = 0; r < NSL; r++) ixi[r][lane] = 1.0 / ld(mp.xi, ln, r);
-    m_load(mp.S, ln, S);
-    sym_proj<RK>(S, s);
-    kinetics<NSL, QP, NS, true>(ph, s, &ixi[0][lane], &gl[0][lane], l, k3, posm);
-    slip_moments<NSL, NS>(ph, &gl[0][lane], 1.0, posm, H, K);
-  }
-  double invFp[9], invSubFp0[9], F[9], G2[9];
-  {
-    double Fp[9], Fp0[9], A2[9];
-    m_load(mp.Fp, ln, Fp);
-    m_load(mp.Fp0, ln, Fp0);
-    m_load(mp.Fphase, ln, F);
-    m_invert(Fp, invFp);
-    m_invert(Fp0, invSubFp0);
-    m_mul(F, invSubFp0, A2);
-    m_mul_tn(Fe, A2, G2);
-#pragma unroll
-    for (int q = 0; q < 9; q++) G2[q] *= dt;
-  }
-  double N[RK * RK], rd[RK], v0[RK], tau[RK];
-  reduced_matrix<RK>(ph, G2, H, K, N);
-  const bool sing = dmk_qr_factor<RK>(N, rd, v0, tau);
-
-  double S[9], M1[9], Mid[9];
+  for (int r = 0; r < NSL; r++) xi[r] = ld(mp.xi, ln, r);
   m_load(mp.S, ln, S);
-  m_mul_nt(S, invFp, M1);          // S invFp^T
-  m_mul(invFp, M1, Mid);           // invFp S invFp^T
+  m_load(mp.Fp, ln, Fp);
+  m_load(mp.Fp0, ln, Fp0);
+  m_load(mp.Fphase, ln, F);
+  m_load(mp.Fe, ln, Fe);
+  batch_end();
+  double invFp[9], Mid[9];
+  {
+    double A2[9], invFp0[9], B[9], M1[9], BS[9];
+    {
+      double H[5][RK], K[3][RK], s[6], l5[5], k3[3];
+      unsigned posm;
+#pragma unroll
+      for (int r = 0; r < NSL; r++) sh[r][lane] = dmk_rcp(xi[r]);
+      sym_proj<RK>(S, s);
+      kinetics<NSL, QP, NS, true>(ph, s, &sh[0][lane], &sh[NSL][lane], l5, k3, posm);
+      slip_moments<NSL, NS>(ph, &sh[NSL][lane], 1.0, posm, H, K);
+      m_invert(Fp, invFp);
+      m_invert(Fp0, invFp0);
+      m_mul(F, invFp0, A2);
+#pragma unroll
+      for (int q = 0; q < 9; q++) { A2[q] *= dt; invFp0[q] *= -dt; }
+      m_mul(F, invFp, B);
+      m_mul_nt(S, invFp, M1);          // S F_p^-T
+      m_mul(invFp, M1, Mid);           // F_p^-1 S F_p^-T
+      m_mul(B, S, BS);
+      double G2[9];
+      m_mul_tn(Fe, A2, G2);            // dt F_e^T A2
+      reduced_matrix<RK>(ph, G2, H, K, N);
+#pragma unroll
+      for (int l = 0; l < RK; l++) {
+        // W_l to LDS; tr(G2 W_l)/sqrt3
+        double h[5], q3[3], W[9], v = 0.0;
+#pragma unroll
+        for (int k = 0; k < 5; k++) { h[k] = H[k][l]; sh[8 * l + k][lane] = h[k]; }
+#pragma unroll
+        for (int m = 0; m < 3; m++) { q3[m] = K[m][l]; sh[8 * l + 5 + m][lane] = q3[m]; }
+        if (RK == 5) {
+          from_basis(h, q3, W);
+#pragma unroll
+          for (int q = 0; q < 9; q++) v = fma(G2[(q % 3) * 3 + q / 3], W[q], v);
+        }
+        g6[l] = v * R3;
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < RK; l++) {
+      double h[5], k3[3], W[9], V[9], U[9], T[9];
+#pragma unroll
+      for (int k = 0; k < 5; k++) h[k] = sh[8 * l + k][lane];
+#pragma unroll
+      for (int m = 0; m < 3; m++) k3[m] = sh[8 * l + 5 + m][lane];
+      from_basis(h, k3, W);
+      basis_between(B, l, invFp, T);
+      m_mul(W, M1, V);
+      m_mul(A2, V, U);
+#pragma unroll
+      for (int q = 0; q < 9; q++) T[q] -= U[q];
+      m_mul_nt(BS, W, V);
+      m_mul_nt(V, invFp0, U);
+#pragma unroll
+      for (int q = 0; q < 9; q++) T[q] += U[q];
+#pragma unroll
+      for (int q = 0; q < 8; q++) sh[8 * l + q][lane] = T[q];
+      T8[l] = T[8];
+    }
+    if (RK == 5) basis_between(B, 5, invFp, T6);
+  }
+  const bool sing = dmk_qr_factor<RK>(N, rd, v0, tau);
+  const double C6 = ph->C11 + 2.0 * ph->C12;
   double n2 = 0.0;
 #pragma unroll 1
   for (int l = 0; l < 3; l++) {
-#pragma unroll 1
+    double pl[3], ml[3], z[3][6];
+    row3(invFp, l, pl);
+    row3(Mid, l, ml);
+#pragma unroll
     for (int k = 0; k < 3; k++) {
-      double fk[3], pl[3], ml[3];
-      row3(Fe, k, fk);
-      row3(invFp, l, pl);
-      row3(Mid, l, ml);
-      double X[9], z[6], t[9], y[9], D[9];
+      const double* fk = Fe + 3 * k;
+      double X[9];
 #pragma unroll
       for (int n = 0; n < 3; n++)
 #pragma unroll
         for (int m = 0; m < 3; m++) X[3 * n + m] = fk[n] * pl[m];
-      sym_proj<RK>(X, z);
+      sym_proj<RK>(X, z[k]);
       if (!sing) {
-        dmk_qr_apply_solve<RK>(N, rd, v0, tau, z);
+        dmk_qr_apply_solve<RK>(N, rd, v0, tau, z[k]);
       } else {                     // as after a failed solve: dS = C:sym(X)
 #pragma unroll
-        for (int q = 0; q < RK; q++) z[q] *= modulus<RK>(ph, q);
+        for (int q = 0; q < RK; q++) z[k][q] *= modulus<RK>(ph, q);
       }
-      moments_apply<RK>(H, K, z, t);
-      {
-        double Gt[9], Xs[9];
-        m_mul(G2, t, Gt);
+      if (RK == 5) {
+        double v = (X[0] + X[4] + X[8]) * R3;
         if (!sing) {
 #pragma unroll
-          for (int q = 0; q < 9; q++) X[q] -= Gt[q];
+          for (int q = 0; q < RK; q++) v = fma(-g6[q], z[k][q], v);
         }
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-          for (int j = 0; j < 3; j++) Xs[3 * i + j] = 0.5 * (X[3 * i + j] + X[3 * j + i]);
-        hooke_sym(ph->C11, ph->C12, ph->C44, Xs, y);
+        z[k][5] = C6 * v;
       }
-      // d(F_p^-1) = D = -dt invSubFp0 t and
-      // dP = e_k (x) Mid(l,:) + F (D S F_p^-T + F_p^-1 (dS F_p^-T + S D^T))
-      m_mul(invSubFp0, t, D);
+    }
 #pragma unroll
-      for (int q = 0; q < 9; q++) D[q] *= -dt;
-      double T1[9], T2[9], col[9];
-      m_mul_nt(y, invFp, T1);
-      m_mul_nt(S, D, T2);
+    for (int j = 0; j < 3; j++)
 #pragma unroll
-      for (int q = 0; q < 9; q++) T1[q] += T2[q];
-      m_mul(invFp, T1, T2);
-      m_mul(D, M1, T1);
+      for (int i = 0; i < 3; i++) {
+        const int c = 3 * i + j;
+        double v[3];
 #pragma unroll
-      for (int q = 0; q < 9; q++) T1[q] += T2[q];
-      m_mul(F, T1, col);
+        for (int q = 0; q < 6; q++) {
+          const double t = q >= RK ? T6[c] : (c == 8 ? T8[q < RK ? q : 0] : sh[8 * q + (c & 7)][lane]);
 #pragma unroll
-      for (int i = 0; i < 3; i++)
-        if (i == k) {
-#pragma unroll
-          for (int j = 0; j < 3; j++) col[3 * i + j] += ml[j];
+          for (int k = 0; k < 3; k++) v[k] = q ? fma(z[k][q], t, v[k]) : z[k][0] * t;
         }
 #pragma unroll
-      for (int j = 0; j < 3; j++)
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-          double v = col[3 * i + j];
-          st(dPdF, ln, i + 3 * j + 9 * k + 27 * l, v);
-          n2 = fma(v, v, n2);
+        for (int k = 0; k < 3; k++) {
+          if (i == k) v[k] += ml[j];
+          if (act) st(dPdF, ln, i + 3 * j + 9 * k + 27 * l, v[k]);
+          n2 = fma(v[k], v[k], n2);
+          if (!act) v[k] = 0.0;
         }
+        if (part) {
+          // row k of 16 lanes: the sum of v[k]
+          const double sum = wave_rows(v[0], v[1], v[2], 0.0);
+          const int k = lane >> 4;
+          if ((lane & 15) == 0 && k < 3) sums[i + 3 * j + 9 * k + 27 * l] = sum;
+        }
+      }
+  }
+  if (part) {
+    double mx = act && n2 > 0.0 ? n2 : 0.0, mn = act && n2 < DBL_MAX ? n2 : DBL_MAX;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      mx = fmax(mx, __shfl_xor(mx, o, 64));
+      mn = fmin(mn, __shfl_xor(mn, o, 64));
+    }
+    for (int c = lane; c < 81; c += SWG) {
+      double* d = part + 81l * blockIdx.x + c;
+      *d = first ? sums[c] : *d + sums[c];
+    }
+    if (lane == 0) {
+      pmax[blockIdx.x] = first ? mx : fmax(mx, pmax[blockIdx.x]);
+      pmin[blockIdx.x] = first ? mn : fmin(mn, pmin[blockIdx.x]);
     }
   }
+  double R[9], Rt[9], q[4];
+  rotational_part(Fe, R);
+  m_transpose(R, Rt);
+  om2qu(Rt, q);
+  if (!act) return;
   nrm[e] = n2;
+#pragma unroll
+  for (int k = 0; k < 4; k++) st(mp.O, ln, k, q[k]);
 }
 
 }  // namespace
@@ -1167,11 +1284,11 @@ extern "C" int dmk_launch_stress_batch(const DmkStressItem* items_dev, int n_ite
 
 extern "C" int dmk_launch_tangent(const DmkMPDev* mp, const DmkPhaseDev* ph, const DmkPhaseDev* ph_host,
                                   int phase_id, double dt, const int* flag, double* dPdF, double* nrm,
-                                  hipStream_t s) {
+                                  double* part, double* pmax, double* pmin, hipStream_t s) {
   const dim3 blk(SWG), grd((mp->N + SWG - 1) / SWG);
   const bool known = for_variant(dmk_sys_variant(ph_host), ph_host->quarter_pow != 0, [&](auto n, auto qp, auto ns) {
     hipLaunchKernelGGL((tangent_kernel<decltype(n)::value, decltype(qp)::value, decltype(ns)::value>), grd, blk, 0, s,
-                       *mp, ph, phase_id, dt, flag, dPdF, nrm);
+                       *mp, ph, phase_id, dt, flag, dPdF, nrm, part, pmax, pmin);
   });
   if (!known) return 1;
   return hipGetLastError() == hipSuccess ? 0 : 2;

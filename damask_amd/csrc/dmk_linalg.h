@@ -80,10 +80,11 @@ int dmk_mdot(const double* x, const double* Y, long ldY, int l, int mode, long n
              hipStream_t s);
 int dmk_axpby(long n, double a, const double* x, double b, const double* y, double* z, hipStream_t s);
 int dmk_combine(long n, const double* XM, const CombineArgs* c, double* XA, hipStream_t s);
-// C_minMaxAvg from the per-cell norms nrm (written by the tangent kernel):
-// partial extrema, global extrema, per-chunk first qualifying cell, first overall, gather
-int dmk_cminmax(const double* dPdF, long N, double band, const double* nrm, double* pmax, double* pmin,
-                long* csel, long* sel, double* ext, double* out, hipStream_t s);
+// C_volAvg (wgt times the sums) and C_minMaxAvg from what the tangent kernel left
+// per work-group: nb sums of each of the 81 columns, nb extrema of the norms nrm
+int dmk_stiffness_averages(const double* part, const double* pmax, const double* pmin, int nb, const double* nrm,
+                           const double* dPdF, long N, double band, double wgt, double* avg, double* cmm,
+                           hipStream_t s);
 // convergence flag and iteration counters; partial needs 3 * dmk_nchunk(N) doubles
 int dmk_status(const int32_t* st, const int32_t* nn, const int32_t* nf, long N, double* partial, int* flag,
                unsigned long long* cnt, hipStream_t s);
@@ -107,6 +108,10 @@ struct DmkStressItem;
 // block0 ascending)
 extern "C" int dmk_launch_stress_batch(const DmkStressItem* items_dev, int n_items, int n_blocks, int variant,
                                        int quarter_pow, hipStream_t s);
+// orientation and dPdF of one phase's cells; the phases are launched in order,
+// 0 first.  part (81 per block), pmax and pmin (blocks each), one block per
+// DMK_STRESS_WG cells, or all null: sums and norm extrema for
+// dmk_stiffness_averages
 extern "C" int dmk_launch_tangent(const DmkMPDev* mp, const DmkPhaseDev* ph, const DmkPhaseDev* ph_host,
                                   int phase_id, double dt, const int* flag, double* dPdF, double* nrm,
-                                  hipStream_t s);
+                                  double* part, double* pmax, double* pmin, hipStream_t s);

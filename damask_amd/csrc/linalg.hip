@@ -351,100 +351,72 @@ __global__ void combine_kernel(long n, const double* __restrict__ XM, CombineArg
   XA[i] = v;
 }
 
-__global__ void __launch_bounds__(RB) minmax_partial(const double* __restrict__ nrm, long N, double* __restrict__ pmax,
-                                                     double* __restrict__ pmin) {
-  __shared__ double smax[RB], smin[RB];
-  long s = (long)blockIdx.x * PER_BLOCK, e = min(s + PER_BLOCK, N);
+// C_volAvg and C_minMaxAvg from the tangent kernel's per-work-group sums and
+// extrema of the squared norms (nb of each).  Blocks 0..80: one column each.
+// Block 81: the first cells whose norm is the largest / smallest within band,
+// norm (1 + band) >= max, norm (1 - band) <= min, hence in the first work-group
+// whose extremum is; none when no norm is comparable.
+constexpr int AB = 1024;
+__global__ void __launch_bounds__(AB) stiffness_averages(const double* __restrict__ part, const double* __restrict__ pmax,
+                                                         const double* __restrict__ pmin, int nb,
+                                                         const double* __restrict__ nrm, const double* __restrict__ dPdF,
+                                                         long N, double band, double wgt, double* __restrict__ avg,
+                                                         double* __restrict__ cmm) {
+  const int t = threadIdx.x;
+  __shared__ double smax[AB], smin[AB];
+  __shared__ int imax[AB], imin[AB];
+  if (blockIdx.x < 81) {
+    const double* p = part + blockIdx.x;
+    double acc = 0.0;
+#pragma unroll 4
+    for (int i = t; i < nb; i += AB) acc += p[81l * i];
+    smax[t] = acc;
+    __syncthreads();
+    for (int k = AB / 2; k > 0; k >>= 1) {
+      if (t < k) smax[t] += smax[t + k];
+      __syncthreads();
+    }
+    if (t == 0) avg[blockIdx.x] = smax[0] * wgt;
+    return;
+  }
   double mx = 0.0, mn = DBL_MAX;
-  for (long i = s + threadIdx.x; i < e; i += RB) {
-    double v = nrm[i];
-    if (v > mx) mx = v;
-    if (v < mn) mn = v;
-  }
-  smax[threadIdx.x] = mx; smin[threadIdx.x] = mn;
+  for (int i = t; i < nb; i += AB) { mx = fmax(mx, pmax[i]); mn = fmin(mn, pmin[i]); }
+  smax[t] = mx; smin[t] = mn;
   __syncthreads();
-  for (int k = RB / 2; k > 0; k >>= 1) {
-    if (threadIdx.x < k) {
-      smax[threadIdx.x] = fmax(smax[threadIdx.x], smax[threadIdx.x + k]);
-      smin[threadIdx.x] = fmin(smin[threadIdx.x], smin[threadIdx.x + k]);
-    }
+  for (int k = AB / 2; k > 0; k >>= 1) {
+    if (t < k) { smax[t] = fmax(smax[t], smax[t + k]); smin[t] = fmin(smin[t], smin[t + k]); }
     __syncthreads();
   }
-  if (threadIdx.x == 0) { pmax[blockIdx.x] = smax[0]; pmin[blockIdx.x] = smin[0]; }
-}
-
-// global extrema of the per-cell norms from the chunk partials (one block)
-__global__ void __launch_bounds__(RB) extrema_finalize(const double* __restrict__ pmax, const double* __restrict__ pmin,
-                                                       int nchunk, double* __restrict__ ext) {
-  __shared__ double smax[RB], smin[RB];
-  double mx = 0.0, mn = DBL_MAX;
-  for (int i = threadIdx.x; i < nchunk; i += RB) { mx = fmax(mx, pmax[i]); mn = fmin(mn, pmin[i]); }
-  smax[threadIdx.x] = mx; smin[threadIdx.x] = mn;
+  const double gmax = smax[0], gmin = smin[0];
+  auto is_max = [&](double v) { return gmax > 0.0 && v * (1.0 + band) >= gmax; };
+  auto is_min = [&](double v) { return gmin < DBL_MAX && v * (1.0 - band) <= gmin; };
+  int bx = nb, bn = nb;
+  for (int i = nb - 1 - t; i >= 0; i -= AB) {
+    if (is_max(pmax[i])) bx = i;
+    if (is_min(pmin[i])) bn = i;
+  }
+  imax[t] = bx; imin[t] = bn;
   __syncthreads();
-  for (int k = RB / 2; k > 0; k >>= 1) {
-    if (threadIdx.x < k) {
-      smax[threadIdx.x] = fmax(smax[threadIdx.x], smax[threadIdx.x + k]);
-      smin[threadIdx.x] = fmin(smin[threadIdx.x], smin[threadIdx.x + k]);
-    }
+  for (int k = AB / 2; k > 0; k >>= 1) {
+    if (t < k) { imax[t] = min(imax[t], imax[t + k]); imin[t] = min(imin[t], imin[t + k]); }
     __syncthreads();
   }
-  if (threadIdx.x == 0) { ext[0] = smax[0]; ext[1] = smin[0]; }
-}
-
-// first cell of each chunk that satisfies the (banded) extremum rule:
-// norm (1 + band) >= max, norm (1 - band) <= min; N when none
-__global__ void __launch_bounds__(RB) select_partial(const double* __restrict__ nrm, long N,
-                                                     const double* __restrict__ ext, double band,
-                                                     long* __restrict__ csel, int nchunk) {
-  __shared__ long simax[RB], simin[RB];
-  const double gmax = ext[0], gmin = ext[1];
-  long s = (long)blockIdx.x * PER_BLOCK, e = min(s + PER_BLOCK, N);
-  long imax = N, imin = N;
-  for (long i = s + threadIdx.x; i < e; i += RB) {
-    double v = nrm[i];
-    if (imax == N && gmax > 0.0 && v * (1.0 + band) >= gmax) imax = i;
-    if (imin == N && gmin < DBL_MAX && v * (1.0 - band) <= gmin) imin = i;
-  }
-  simax[threadIdx.x] = imax; simin[threadIdx.x] = imin;
+  bx = imax[0]; bn = imin[0];
   __syncthreads();
-  for (int k = RB / 2; k > 0; k >>= 1) {
-    if (threadIdx.x < k) {
-      simax[threadIdx.x] = min(simax[threadIdx.x], simax[threadIdx.x + k]);
-      simin[threadIdx.x] = min(simin[threadIdx.x], simin[threadIdx.x + k]);
-    }
-    __syncthreads();
+  // wavefront 0: the cell of the maximum, wavefront 1: of the minimum
+  if (t < 2 * DMK_STRESS_WG) {
+    const int w = t / DMK_STRESS_WG, lane = t % DMK_STRESS_WG, b = w ? bn : bx;
+    const long e = (long)b * DMK_STRESS_WG + lane;
+    const bool hit = b < nb && e < N && (w ? is_min(nrm[e]) : is_max(nrm[e]));
+    const unsigned long long m = __ballot(hit);
+    if (lane == 0) (w ? imin : imax)[0] = m ? b * DMK_STRESS_WG + __ffsll(m) - 1 : -1;
   }
-  if (threadIdx.x == 0) { csel[blockIdx.x] = simax[0]; csel[nchunk + blockIdx.x] = simin[0]; }
-}
-
-// first qualifying cell over all chunks (one block): sel[0] = imax, sel[1] = imin (-1: none)
-__global__ void __launch_bounds__(RB) select_finalize(const long* __restrict__ csel, int nchunk, long N,
-                                                      long* __restrict__ sel) {
-  __shared__ long simax[RB], simin[RB];
-  long imax = N, imin = N;
-  for (int i = threadIdx.x; i < nchunk; i += RB) { imax = min(imax, csel[i]); imin = min(imin, csel[nchunk + i]); }
-  simax[threadIdx.x] = imax; simin[threadIdx.x] = imin;
   __syncthreads();
-  for (int k = RB / 2; k > 0; k >>= 1) {
-    if (threadIdx.x < k) {
-      simax[threadIdx.x] = min(simax[threadIdx.x], simax[threadIdx.x + k]);
-      simin[threadIdx.x] = min(simin[threadIdx.x], simin[threadIdx.x + k]);
-    }
-    __syncthreads();
+  if (t < 81) {
+    const double vx = imax[0] >= 0 ? dPdF[(long)t * N + imax[0]] : 0.0;
+    const double vn = imin[0] >= 0 ? dPdF[(long)t * N + imin[0]] : DBL_MAX;
+    cmm[t] = 0.5 * (vx + vn);
   }
-  if (threadIdx.x == 0) {
-    sel[0] = simax[0] < N ? simax[0] : -1;
-    sel[1] = simin[0] < N ? simin[0] : -1;
-  }
-}
-
-__global__ void gather_cminmax(const double* __restrict__ dPdF, long N, const long* __restrict__ sel,
-                               double* __restrict__ out) {
-  int q = threadIdx.x;
-  if (q >= 81) return;
-  double mx = sel[0] >= 0 ? dPdF[q * N + sel[0]] : 0.0;
-  double mn = sel[1] >= 0 ? dPdF[q * N + sel[1]] : DBL_MAX;
-  out[q] = 0.5 * (mx + mn);
 }
 
 // per chunk: any cell not converged, sums of Newton and state iterations
@@ -667,14 +639,11 @@ int dmk_combine(long n, const double* XM, const CombineArgs* c, double* XA, hipS
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
-int dmk_cminmax(const double* dPdF, long N, double band, const double* nrm, double* pmax, double* pmin,
-                long* csel, long* sel, double* ext, double* out, hipStream_t s) {
-  int nc = dmk_nchunk(N);
-  hipLaunchKernelGGL(minmax_partial, dim3(nc), dim3(RB), 0, s, nrm, N, pmax, pmin);
-  hipLaunchKernelGGL(extrema_finalize, dim3(1), dim3(RB), 0, s, pmax, pmin, nc, ext);
-  hipLaunchKernelGGL(select_partial, dim3(nc), dim3(RB), 0, s, nrm, N, ext, band, csel, nc);
-  hipLaunchKernelGGL(select_finalize, dim3(1), dim3(RB), 0, s, csel, nc, N, sel);
-  hipLaunchKernelGGL(gather_cminmax, dim3(1), dim3(128), 0, s, dPdF, N, sel, out);
+int dmk_stiffness_averages(const double* part, const double* pmax, const double* pmin, int nb, const double* nrm,
+                           const double* dPdF, long N, double band, double wgt, double* avg, double* cmm,
+                           hipStream_t s) {
+  hipLaunchKernelGGL(stiffness_averages, dim3(82), dim3(AB), 0, s, part, pmax, pmin, nb, nrm, dPdF, N, band, wgt, avg,
+                     cmm);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 

@@ -205,7 +205,7 @@ struct dmk_handle {
   double *F, *F_lastinc, *Fdot, *R, *XM, *FM, *XA, *FA, *Xh, *Fh, *Fext, *Pext;
   double2 *Z, *U;
   double *u3, *xn_dev, *xp_dev;
-  double *partial, *small, *nrm, *pmax, *pmin, *ext;
+  double *partial, *small, *nrm, *pmax, *pmin;
   double* divp = nullptr;            // per-block divergence sums of the basic residual
   int div_nb = 0;                    // how many
   bool div_pending = false;          // divp holds sums the next residual_finish adds up
@@ -214,7 +214,6 @@ struct dmk_handle {
   bool lk_pending = false;
   const double* lk_X = nullptr;
   double* lk_r = nullptr;
-  long *sel, *csel;
   int* flag;
   unsigned long long* cnt;
   double* hsmall = nullptr;          // pinned host mirror of small results
@@ -320,6 +319,9 @@ static void gamma_coef(double wgt, const double* C, GammaArgs* g) {
 
 static void set_gamma_coef(dmk_handle* h, const double* C) { gamma_coef(h->wgt, C, &h->ga); }
 
+// work-groups of the per-cell kernels
+static int cell_blocks(long N) { return (int)((N + DMK_STRESS_WG - 1) / DMK_STRESS_WG); }
+
 // Orientation, dPdF and the stiffness averages C_volAvg / C_minMaxAvg of the
 // last response (homogenization_mechanical_response's second loop and the
 // averages of utilities_constitutiveResponse, grid_utilities.f90:163-214).
@@ -333,12 +335,13 @@ static int tangent_pass(dmk_handle* h, double dt) {
   if (h->status != ST_OK) return 0;
   kt_begin(h, KT_TANGENT);
   for (int p = 0; p < h->n_phases; p++)
-    CKL(dmk_launch_tangent(&h->mp, h->ph_dev + p, &h->ph[p], p, dt, h->flag, h->dPdF, h->nrm, h->st));
+    CKL(dmk_launch_tangent(&h->mp, h->ph_dev + p, &h->ph[p], p, dt, h->flag, h->dPdF, h->nrm, h->partial, h->pmax,
+                           h->pmin, h->st));
   kt_end(h, KT_TANGENT);
   kt_begin(h, KT_CAVG);
-  CKL(dmk_colsum(h->dPdF, h->N, h->N, 81, h->partial, h->small + SM_CVOL, h->wgt, h->st));
-  CKL(dmk_cminmax(h->dPdF, h->N, h->num.cref_rule == 1 ? 1.0e-12 : 0.0, h->nrm, h->pmax, h->pmin, h->csel, h->sel,
-                  h->ext, h->small + SM_CMM, h->st));
+  CKL(dmk_stiffness_averages(h->partial, h->pmax, h->pmin, cell_blocks(h->N), h->nrm, h->dPdF, h->N,
+                             h->num.cref_rule == 1 ? 1.0e-12 : 0.0, h->wgt, h->small + SM_CVOL, h->small + SM_CMM,
+                             h->st));
   kt_end(h, KT_CAVG);
   CK(hipMemcpyAsync(h->hsmall + SM_CVOL, h->small + SM_CVOL, sizeof(double) * 162, hipMemcpyDeviceToHost, h->st));
   CK(hipStreamSynchronize(h->st));
@@ -531,7 +534,8 @@ static int residual_enqueue_pol(dmk_handle* h, const double* X, double* r) {
   CKL(dmk_colsum(h->partial, nb, nb, 1, h->partial + nb, h->small + SM_REP + REP_DIV2, 1.0, h->st));
   kt_begin(h, KT_TANGENT);
   for (int p = 0; p < h->n_phases; p++)
-    CKL(dmk_launch_tangent(&h->mp, h->ph_dev + p, &h->ph[p], p, h->dt, h->flag, h->dPdF, h->nrm, h->st));
+    CKL(dmk_launch_tangent(&h->mp, h->ph_dev + p, &h->ph[p], p, h->dt, h->flag, h->dPdF, h->nrm, nullptr, nullptr, nullptr,
+                           h->st));
   kt_end(h, KT_TANGENT);
   CKL(dmk_pol_rF(N, &h->pol, F, Ft, h->P_hom, h->dPdF, rt, rF, h->st));
   AimArgs a;
@@ -552,7 +556,8 @@ static int residual_enqueue_gk(dmk_handle* h, const double* X, double* r) {
   if (rc) return rc;
   kt_begin(h, KT_TANGENT);
   for (int p = 0; p < h->n_phases; p++)
-    CKL(dmk_launch_tangent(&h->mp, h->ph_dev + p, &h->ph[p], p, h->dt, h->flag, h->dPdF, h->nrm, h->st));
+    CKL(dmk_launch_tangent(&h->mp, h->ph_dev + p, &h->ph[p], p, h->dt, h->flag, h->dPdF, h->nrm, nullptr, nullptr, nullptr,
+                           h->st));
   kt_end(h, KT_TANGENT);
   AimArgs a;
   aim_args(h, true, false, &a);
@@ -2097,16 +2102,14 @@ static int init_impl(dmk_handle* h, const int32_t cells[3], const double size[3]
   long nn = (long)(cells[0] + 1) * (cells[1] + 1) * (cells[2] + 1);
   if ((rc = dalloc(h, &h->xn_dev, 3 * nn))) return rc;
   if ((rc = dalloc(h, &h->xp_dev, 3 * N))) return rc;
-  long np = 82L * dmk_nchunk(std::max(nx, 9 * h->Nk)) + 4096;
+  // partial sums: of up to 82 vectors, or the tangent's 81 per work-group
+  long np = std::max(82L * dmk_nchunk(std::max(nx, 9 * h->Nk)) + 4096, 81L * cell_blocks(N));
   if ((rc = dalloc(h, &h->partial, np))) return rc;
   if ((rc = dalloc(h, &h->small, SM_SIZE))) return rc;
   if ((rc = dalloc(h, &h->divp, (size_t)dmk_gamma_conv_partials(&h->fft)))) return rc;
   if ((rc = dalloc(h, &h->nrm, N))) return rc;
-  if ((rc = dalloc(h, &h->pmax, dmk_nchunk(N)))) return rc;
-  if ((rc = dalloc(h, &h->pmin, dmk_nchunk(N)))) return rc;
-  if ((rc = dalloc(h, &h->ext, 2))) return rc;
-  if ((rc = dalloc(h, &h->sel, 2))) return rc;
-  if ((rc = dalloc(h, &h->csel, 2L * dmk_nchunk(N)))) return rc;
+  if ((rc = dalloc(h, &h->pmax, cell_blocks(N)))) return rc;
+  if ((rc = dalloc(h, &h->pmin, cell_blocks(N)))) return rc;
   if ((rc = dalloc(h, &h->flag, 4))) return rc;
   if ((rc = dalloc(h, &h->cnt, 4))) return rc;
   CK(hipHostMalloc((void**)&h->hsmall, sizeof(double) * SM_SIZE, hipHostMallocDefault));
