@@ -77,24 +77,73 @@ __global__ void __launch_bounds__(RB) dot_partial(const double* __restrict__ x, 
   if (threadIdx.x == 0) partial[(long)blockIdx.y * nchunk + blockIdx.x] = r;
 }
 
+// Dot products: a block takes its chunk of up to DOT_JB consecutive jobs.  Jobs
+// that follow each other mostly share x (a new residual or Krylov vector against
+// every stored one): its values stay in registers, and the sums of all jobs go
+// through LDS together, in the order of block_sum.  So a job reads one vector, not
+// two, and it is HBM-bound: 128^3 cells, about 8 jobs over 151 MB vectors, 224 us
+// instead of 311 as a block per chunk and job; 64^3 39 instead of 41 us (the
+// 256 MB cache held x there).  Few
+// chunks are spread over the jobs instead (dot_jobs_per_block).
+#define DOT_JB 8
+// 4 blocks a CU before jobs share a block
+__host__ __device__ inline int dot_jobs_per_block(int nchunk, int njobs) {
+  const long k = (long)nchunk * njobs / 1024;
+  return k < 1 ? 1 : (k > DOT_JB ? DOT_JB : (int)k);
+}
+
 __device__ __forceinline__ void dot_jobs_partial_body(const DotJobs& J, long n, double* __restrict__ partial,
-                                                      int nchunk, int bx, int j) {
-  const double* __restrict__ x = J.x[j];
-  const double* __restrict__ y = J.y[j];
-  long s = (long)bx * PER_BLOCK;
-  long e = min(s + PER_BLOCK, n);
-  double acc = 0.0;
-  if (J.mode[j] == 0) {
-    for (long i = s + threadIdx.x; i < e; i += RB) acc = fma(x[i], y[i], acc);
-  } else {
-    for (long i = s + threadIdx.x; i < e; i += RB) { double d = y[i] - x[i]; acc = fma(d, d, acc); }
+                                                      int nchunk, int bx, int group) {
+  constexpr int NV = PER_BLOCK / RB;
+  __shared__ double red[DOT_JB][RB];
+  const int t = threadIdx.x, jb = dot_jobs_per_block(nchunk, J.n), j0 = group * jb;
+  if (j0 >= J.n) return;
+  const int nj = min(jb, J.n - j0);
+  const long s = (long)bx * PER_BLOCK + t;
+  double x[NV];
+  const double* xp = nullptr;
+  for (int j = 0; j < nj; j++) {
+    const double* yp = J.y[j0 + j];
+    double y[NV];
+#pragma unroll
+    for (int k = 0; k < NV; k++) y[k] = s + k * RB < n ? yp[s + k * RB] : 0.0;
+    if (J.x[j0 + j] != xp) {
+      xp = J.x[j0 + j];
+      if (xp == yp) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) x[k] = y[k];
+      } else {
+#pragma unroll
+        for (int k = 0; k < NV; k++) x[k] = s + k * RB < n ? xp[s + k * RB] : 0.0;
+      }
+    }
+    double acc = 0.0;
+    if (J.mode[j0 + j] == 0) {
+#pragma unroll
+      for (int k = 0; k < NV; k++) acc = fma(x[k], y[k], acc);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NV; k++) { const double d = y[k] - x[k]; acc = fma(d, d, acc); }
+    }
+    red[j][t] = acc;
   }
-  double r = block_sum(acc);
-  if (threadIdx.x == 0) partial[(long)j * nchunk + bx] = r;
+  __syncthreads();
+  const int lane = t & 63;
+  for (int j = t >> 6; j < nj; j += RB / 64) {
+    double v = (red[j][lane] + red[j][lane + 128]) + (red[j][lane + 64] + red[j][lane + 192]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+    if (lane == 0) partial[(long)(j0 + j) * nchunk + bx] = v;
+  }
 }
 
 __global__ void __launch_bounds__(RB) dot_jobs_partial(DotJobs J, long n, double* __restrict__ partial, int nchunk) {
   dot_jobs_partial_body(J, n, partial, nchunk, blockIdx.x, blockIdx.y);
+}
+
+void launch_dot_jobs(const DotJobs& J, long n, double* partial, int nc, hipStream_t s) {
+  const int jb = dot_jobs_per_block(nc, J.n);
+  hipLaunchKernelGGL(dot_jobs_partial, dim3(nc, (J.n + jb - 1) / jb), dim3(RB), 0, s, J, n, partial, nc);
 }
 
 __device__ __forceinline__ void accept_P_body(const int* __restrict__ flag, const double* __restrict__ P_old,
@@ -300,7 +349,7 @@ __global__ void accept_P_batch(const DmkResidDev* __restrict__ R) {
 
 __global__ void __launch_bounds__(RB) dot_jobs_partial_batch(const DmkResidDev* __restrict__ R) {
   const DmkResidDev& q = R[blockIdx.z];
-  if ((int)blockIdx.x >= q.nc_dots || (int)blockIdx.y >= q.J.n) return;
+  if ((int)blockIdx.x >= q.nc_dots) return;
   dot_jobs_partial_body(q.J, q.nx, q.partial, q.nc_dots, blockIdx.x, blockIdx.y);
 }
 
@@ -545,7 +594,7 @@ int dmk_mdot(const double* x, const double* Y, long ldY, int l, int mode, long n
 int dmk_dots(const DotJobs* jobs, long n, double* partial, double* out, hipStream_t s) {
   if (jobs->n <= 0) return 0;
   int nc = dmk_nchunk(n);
-  hipLaunchKernelGGL(dot_jobs_partial, dim3(nc, jobs->n), dim3(RB), 0, s, *jobs, n, partial, nc);
+  launch_dot_jobs(*jobs, n, partial, nc, s);
   hipLaunchKernelGGL(finalize_sum, dim3(jobs->n), dim3(RB), 0, s, partial, nc, 1.0, out);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
@@ -566,7 +615,7 @@ int dmk_dots_sums(const DotJobs* jobs, long n, double* partial, double* out, con
   if (!extra) J.k = 0;
   int nc = dmk_nchunk(n);
   if (jobs && jobs->n > 0) {
-    hipLaunchKernelGGL(dot_jobs_partial, dim3(nc, jobs->n), dim3(RB), 0, s, *jobs, n, partial, nc);
+    launch_dot_jobs(*jobs, n, partial, nc, s);
     for (int j = 0; j < jobs->n; j++) {
       if (J.k >= DMK_MAX_SUMS) return 1;
       J.p[J.k] = partial + (long)j * nc;
