@@ -2316,11 +2316,11 @@ extern "C" int dmk_constitutive(dmk_handle* h, double dt, const double* F, doubl
                                 double* C_volAvg, double* C_minMaxAvg, int32_t* status) {
   if (!h || !F) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, F, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, 0, h->N, h->Fext, h->st));
   int rc = constitutive(h, h->Fext, dt, false, true);
   if (rc) return rc;
   if (P) {
-    CKL(dmk_soa_to_aos(h->P_hom, h->N, 9, h->Pext, h->st));
+    CKL(dmk_soa_to_aos(h->P_hom, h->N, 9, 0, h->N, h->Pext, h->st));
     CK(hipMemcpyAsync(P, h->Pext, sizeof(double) * h->n9, hipMemcpyDeviceToHost, h->st));
     CK(hipStreamSynchronize(h->st));
   }
@@ -2333,11 +2333,11 @@ extern "C" int dmk_constitutive(dmk_handle* h, double dt, const double* F, doubl
 
 extern "C" int dmk_constitutive_device(dmk_handle* h, double dt, const double* F_dev, double* P_dev, int32_t* status) {
   if (!h || !F_dev) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
-  CKL(dmk_aos_to_soa(F_dev, h->N, 9, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(F_dev, h->N, 9, 0, h->N, h->Fext, h->st));
   int rc = constitutive(h, h->Fext, dt, false, true);
   if (rc) return rc;
   if (P_dev) {
-    CKL(dmk_soa_to_aos(h->P_hom, h->N, 9, P_dev, h->st));
+    CKL(dmk_soa_to_aos(h->P_hom, h->N, 9, 0, h->N, P_dev, h->st));
     CK(hipStreamSynchronize(h->st));
   }
   if (status) *status = h->status;
@@ -2377,7 +2377,7 @@ extern "C" int dmk_mech_get_field(dmk_handle* h, int32_t what, double* dst) {
   if (field_dev(h, what, &p, &w)) { dmk_set_error("unknown field %d", what); return DMK_ERR_ARG; }
   double* tmp;
   CK(hipMallocAsync((void**)&tmp, sizeof(double) * w * h->N, h->st));
-  CKL(dmk_soa_to_aos(p, h->N, w, tmp, h->st));
+  CKL(dmk_soa_to_aos(p, h->N, w, 0, h->N, tmp, h->st));
   CK(hipMemcpyAsync(dst, tmp, sizeof(double) * w * h->N, hipMemcpyDeviceToHost, h->st));
   CK(hipFreeAsync(tmp, h->st));
   CK(hipStreamSynchronize(h->st));
@@ -2395,7 +2395,7 @@ extern "C" int dmk_mech_set_field(dmk_handle* h, int32_t what, const double* src
   double* tmp;
   CK(hipMallocAsync((void**)&tmp, sizeof(double) * w * h->N, h->st));
   CK(hipMemcpyAsync(tmp, src, sizeof(double) * w * h->N, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(tmp, h->N, w, (double*)p, h->st));
+  CKL(dmk_aos_to_soa(tmp, h->N, w, 0, h->N, (double*)p, h->st));
   CK(hipFreeAsync(tmp, h->st));
   // the restart also sets the increment-start copies (phase_mechanical.f90:1265-1280)
   const DmkMPDev& mp = h->mp;
@@ -2614,7 +2614,7 @@ extern "C" int dmk_grid_set_restart(dmk_handle* h, int32_t restart_inc) {
 extern "C" int dmk_gamma_convolution(dmk_handle* h, const double* field, const double aim[9], double* out) {
   if (!h || !field || !aim || !out) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, field, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, 0, h->N, h->Fext, h->st));
   // the transform path of the basic residual (x-y passes, z passes with Gamma)
   CKL(dmk_fft_r2c_xy(&h->fft, 9, h->Fext, h->Z, h->st));
   GammaArgs g = h->ga;
@@ -2625,7 +2625,7 @@ extern "C" int dmk_gamma_convolution(dmk_handle* h, const double* field, const d
   int nb;
   CKL(dmk_gamma_conv(&h->fft, h->Z, &g, h->divp, &nb, h->st));
   CKL(dmk_fft_c2r_xy(&h->fft, 9, h->Z, h->Fext, h->st));
-  CKL(dmk_soa_to_aos(h->Fext, h->N, 9, h->Pext, h->st));
+  CKL(dmk_soa_to_aos(h->Fext, h->N, 9, 0, h->N, h->Pext, h->st));
   CK(hipMemcpyAsync(out, h->Pext, sizeof(double) * h->n9, hipMemcpyDeviceToHost, h->st));
   CK(hipStreamSynchronize(h->st));
   return 0;
@@ -2635,7 +2635,7 @@ extern "C" int dmk_gamma_convolution(dmk_handle* h, const double* field, const d
 extern "C" int dmk_divergence_rms(dmk_handle* h, const double* field, double* out) {
   if (!h || !field || !out) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, field, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, 0, h->N, h->Fext, h->st));
   CKL(dmk_fft_r2c(&h->fft, 9, h->Fext, h->Z, h->st));
   GammaArgs g = h->ga;
   g.do_div = 1;
@@ -2655,7 +2655,7 @@ extern "C" int dmk_divergence_rms(dmk_handle* h, const double* field, double* ou
 extern "C" int dmk_curl_rms(dmk_handle* h, const double* field, double* out) {
   if (!h || !field || !out) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, field, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, 0, h->N, h->Fext, h->st));
   CKL(dmk_fft_r2c(&h->fft, 9, h->Fext, h->Z, h->st));
   CKL(dmk_curl_partial(h->Z, &h->ga, h->partial, h->st));
   int nb = dmk_gamma_div_blocks(&h->ga);
@@ -2673,7 +2673,7 @@ extern "C" int dmk_curl_rms(dmk_handle* h, const double* field, double* out) {
 extern "C" int dmk_fft_forward(dmk_handle* h, int32_t howmany, const double* in, double* out) {
   if (!h || !in || !out || howmany < 1 || howmany > 9) { dmk_set_error("bad argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, in, sizeof(double) * howmany * h->N, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, howmany, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, howmany, 0, h->N, h->Fext, h->st));
   CKL(dmk_fft_r2c(&h->fft, howmany, h->Fext, h->Z, h->st));
   std::vector<double> tmp(2 * howmany * h->Nk);
   CK(hipMemcpyAsync(tmp.data(), h->Z, sizeof(double) * tmp.size(), hipMemcpyDeviceToHost, h->st));
@@ -2697,7 +2697,7 @@ extern "C" int dmk_fft_backward(dmk_handle* h, int32_t howmany, const double* in
     }
   CK(hipMemcpyAsync(h->Z, tmp.data(), sizeof(double) * tmp.size(), hipMemcpyHostToDevice, h->st));
   CKL(dmk_fft_c2r(&h->fft, howmany, h->Z, h->Fext, h->st));
-  CKL(dmk_soa_to_aos(h->Fext, h->N, howmany, h->Pext, h->st));
+  CKL(dmk_soa_to_aos(h->Fext, h->N, howmany, 0, h->N, h->Pext, h->st));
   CK(hipMemcpyAsync(out, h->Pext, sizeof(double) * howmany * h->N, hipMemcpyDeviceToHost, h->st));
   CK(hipStreamSynchronize(h->st));
   return 0;
