@@ -887,11 +887,12 @@ static int sync_dots(dmk_handle* h, const DotJobs& J, double* out) {
 // GK_op: out = G * (K : v), DC term kept on the stress-controlled components
 static int gk_jv(dmk_handle* h, const double* v, double* out) {
   CKL(dmk_gk_apply(h->N, h->dPdF, v, h->T, h->st));
-  CKL(dmk_fft_r2c(&h->fft, 9, h->T, h->Z, h->st));
+  CKL(dmk_fft_r2c_xy(&h->fft, 9, h->T, h->Z, h->st));
   GalerkinArgs ga{};
   for (int k = 0; k < 9; k++) ga.stress_mask[k] = h->stress_mask[k];
-  CKL(dmk_galerkin(h->Z, &h->ga, &ga, h->partial, h->st));
-  CKL(dmk_fft_c2r(&h->fft, 9, h->Z, out, h->st));
+  int nb;
+  CKL(dmk_galerkin_conv(&h->fft, h->Z, &h->ga, &ga, h->divp, &nb, h->st));
+  CKL(dmk_fft_c2r_xy(&h->fft, 9, h->Z, out, h->st));
   return 0;
 }
 
@@ -2077,7 +2078,7 @@ static int init_impl(dmk_handle* h, const int32_t cells[3], const double size[3]
   const long nx = h->nx;
   double** sol[] = {&h->F, &h->F_lastinc, &h->Fdot, &h->R, &h->XM, &h->FM, &h->XA, &h->FA};
   for (auto pp : sol) if ((rc = dalloc(h, pp, nx))) return rc;
-  if ((rc = dalloc(h, &h->Fext, n9)) || (rc = dalloc(h, &h->Pext, n9))) return rc;
+  if ((rc = dalloc(h, &h->Fext, n9)) || (rc = dalloc(h, &h->Pext, std::max(n9, 96L)))) return rc;   // a cell of any field
   if (h->scheme != 0 && (rc = dalloc(h, &h->T, n9))) return rc;
   // NGMRES history (M pairs), or for the Galerkin scheme the 31 Krylov vectors of GMRES(30)
   if (h->scheme == 2) {
@@ -2375,11 +2376,15 @@ extern "C" int dmk_mech_get_field(dmk_handle* h, int32_t what, double* dst) {
   const double* p;
   int w;
   if (field_dev(h, what, &p, &w)) { dmk_set_error("unknown field %d", what); return DMK_ERR_ARG; }
-  double* tmp;
-  CK(hipMallocAsync((void**)&tmp, sizeof(double) * w * h->N, h->st));
-  CKL(dmk_soa_to_aos(p, h->N, w, 0, h->N, tmp, h->st));
-  CK(hipMemcpyAsync(dst, tmp, sizeof(double) * w * h->N, hipMemcpyDeviceToHost, h->st));
-  CK(hipFreeAsync(tmp, h->st));
+  // through the handle's staging field, as many cells at a time as it holds (with a
+  // buffer allocated for each call an increment of 64^3 cells and its F, P and xi
+  // took 3 % longer)
+  const long step = std::max(1L, h->n9 / w);
+  for (long e0 = 0; e0 < h->N; e0 += step) {
+    const long n = std::min(step, h->N - e0);
+    CKL(dmk_soa_to_aos(p, h->N, w, e0, n, h->Pext, h->st));
+    CK(hipMemcpyAsync(dst + e0 * w, h->Pext, sizeof(double) * w * n, hipMemcpyDeviceToHost, h->st));
+  }
   CK(hipStreamSynchronize(h->st));
   return 0;
 }
@@ -2392,11 +2397,12 @@ extern "C" int dmk_mech_set_field(dmk_handle* h, int32_t what, const double* src
     dmk_set_error("field %d cannot be set", what);
     return DMK_ERR_ARG;
   }
-  double* tmp;
-  CK(hipMallocAsync((void**)&tmp, sizeof(double) * w * h->N, h->st));
-  CK(hipMemcpyAsync(tmp, src, sizeof(double) * w * h->N, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(tmp, h->N, w, 0, h->N, (double*)p, h->st));
-  CK(hipFreeAsync(tmp, h->st));
+  const long step = std::max(1L, h->n9 / w);
+  for (long e0 = 0; e0 < h->N; e0 += step) {
+    const long n = std::min(step, h->N - e0);
+    CK(hipMemcpyAsync(h->Pext, src + e0 * w, sizeof(double) * w * n, hipMemcpyHostToDevice, h->st));
+    CKL(dmk_aos_to_soa(h->Pext, h->N, w, e0, n, (double*)p, h->st));
+  }
   // the restart also sets the increment-start copies (phase_mechanical.f90:1265-1280)
   const DmkMPDev& mp = h->mp;
   size_t b = sizeof(double) * w * h->N;
