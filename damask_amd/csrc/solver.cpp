@@ -563,7 +563,7 @@ static int residual_enqueue_gk(dmk_handle* h, const double* X, double* r) {
   aim_args(h, true, false, &a);
   CKL(dmk_gk_bc(&a, h->small + SM_PAV, h->flag, h->small + SM_REP, h->small + SM_GDC, h->st));
   kt_begin(h, KT_FFT_FWD);
-  CKL(dmk_fft_r2c(&h->fft, 9, h->P_hom, h->Z, h->st));
+  CKL(dmk_fft_r2c_xy(&h->fft, 9, h->P_hom, h->Z, h->st));
   kt_end(h, KT_FFT_FWD);
   GalerkinArgs ga{};
   ga.do_div = 1;
@@ -572,12 +572,11 @@ static int residual_enqueue_gk(dmk_handle* h, const double* X, double* r) {
   ga.dc_dev = h->small + SM_GDC;
   ga.dc_scale = 1.0 / h->wgt;
   kt_begin(h, KT_GAMMA);
-  CKL(dmk_galerkin(h->Z, &h->ga, &ga, h->partial, h->st));
+  CKL(dmk_galerkin_conv(&h->fft, h->Z, &h->ga, &ga, h->divp, &h->div_nb, h->st));
+  h->div_pending = true;
   kt_end(h, KT_GAMMA);
-  int nb = dmk_gamma_div_blocks(&h->ga);
-  CKL(dmk_colsum(h->partial, nb, nb, 1, h->partial + nb, h->small + SM_REP + REP_DIV2, 1.0, h->st));
   kt_begin(h, KT_FFT_INV);
-  CKL(dmk_fft_c2r(&h->fft, 9, h->Z, r, h->st));
+  CKL(dmk_fft_c2r_xy(&h->fft, 9, h->Z, r, h->st));
   kt_end(h, KT_FFT_INV);
   return 0;
 }
