@@ -52,6 +52,14 @@ constexpr int stress_waves(int nsl) { return nsl > 12 ? 1 : 2; }
 // polynomial constants are hoisted out of every enclosing loop and stay live
 // across the 9x9 Newton system.
 __device__ __noinline__ double pow_ool(double x, double y) { return pow(x, y); }
+// four at once: their chains overlap (31x45x27 cells, 24 systems, n = 17.3: 0.412
+// instead of 0.477 ms a launch; 64^3 cells, 12 systems 0.595 instead of 0.631)
+struct Four { double v[4]; };
+__device__ __noinline__ Four pow4_ool(Four x, Four y) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) x.v[j] = pow(x.v[j], y.v[j]);
+  return x;
+}
 __device__ __noinline__ double tanh_ool(double x) { return tanh(x); }
 
 // x^y for the power laws (phenopowerlaw n_sl, a_sl).  With QP (every
@@ -66,7 +74,7 @@ __device__ __noinline__ double tanh_ool(double x) { return tanh(x); }
 // largest odd multiples of 1/4 (y near 64, taken as (x^(1/4))^255).  It
 // follows pow's rules for zero, negative (NaN unless y is an integer, sign of
 // odd powers), infinite and NaN bases.  Phases with other exponents use the
-// library pow (within 2 ulp, 23 % slower per stress launch at 64^3).
+// library pow (within 2 ulp), four systems at a time (pow_laws).
 template <bool QP>
 DI double pow_law(double x, double y) {
   if (!QP) return pow_ool(x, y);
@@ -88,6 +96,25 @@ DI double pow_law(double x, double y) {
     if (k) b = b * b;
   }
   return r;
+}
+
+// xs_a <- xs_a^y_a of systems a0 .. a0 + n - 1 (LDS), n a multiple of 4
+template <bool QP, class Table>
+DI void pow_laws(Table y, int a0, int n, double* xs) {
+  if (QP) {
+#pragma unroll 1
+    for (int j = a0; j < a0 + n; j++) xs[j * SWG] = pow_law<QP>(xs[j * SWG], y[j]);
+  } else {
+#pragma unroll 1
+    for (int j = a0; j < a0 + n; j += 4) {
+      Four x, e;
+#pragma unroll
+      for (int k = 0; k < 4; k++) { x.v[k] = xs[(j + k) * SWG]; e.v[k] = y[j + k]; }
+      x = pow4_ool(x, e);
+#pragma unroll
+      for (int k = 0; k < 4; k++) xs[(j + k) * SWG] = x.v[k];
+    }
+  }
 }
 
 // the power laws' x^y on the device, for checking their arithmetic
@@ -287,8 +314,7 @@ DI void kinetics(PhPtr ph, const double* s, const double* ixs, double* gs, doubl
     } else {
 #pragma unroll
       for (int j = 0; j < CH; j++) gs[(a0 + j) * SWG] = NS ? x[j] : fabs(x[j]);
-#pragma unroll 1
-      for (int j = a0; j < a0 + CH; j++) gs[j * SWG] = pow_law<QP>(gs[j * SWG], ph->n[j]);
+      pow_laws<QP>(&ph->n[0], a0, CH, gs);
 #pragma unroll
       for (int j = 0; j < CH; j++) r[j] = gs[(a0 + j) * SWG];
     }
@@ -436,8 +462,7 @@ DI bool dot_state(PhPtr ph, const double* gs, double* ws) {
     } else {
 #pragma unroll
       for (int j = 0; j < CH; j++) ws[(r0 + j) * SWG] = fabs(x[j]);
-#pragma unroll 1
-      for (int j = r0; j < r0 + CH; j++) ws[j * SWG] = pow_law<QP>(ws[j * SWG], ph->a[j]);
+      pow_laws<QP>(&ph->a[0], r0, CH, ws);
 #pragma unroll
       for (int j = 0; j < CH; j++) p[j] = ws[(r0 + j) * SWG];
     }
