@@ -526,7 +526,7 @@ def main():
                    "cells_x_increments_per_s": args.cells**3 * args.steps / elapsed},
         "roofline": {"bound": "fp64-valu", "compute": "fp64 vector ALU, no MFMA on the path (MI355X fp64 vector "
                                                       "peak 78.6 TFLOP/s)",
-                     "kernel": "stress_kernel<12, true>", "achieved": achieved,
+                     "kernel": "stress_kernel<12, true, false>", "achieved": achieved,
                      "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s", "frac": achieved / PEAK_FP64_TFLOPS,
                      "traffic": args.traffic_bytes or None,
                      "algorithmic_bytes_per_launch": flops.stress_kernel_bytes(nsl) * args.cells**3,

@@ -4,37 +4,37 @@ division, square root or pow counts 1).  The counts multiply device-side
 iteration counters (Newton iterations, state-integrator iterations) to give
 the FLOPs of one response.
 
-Newton iteration of integrateStress (N_sl slip systems), per cell:
-  B = I - dt Lp                                  18
-  F_e = A B                                      54
-  Hooke: F_e^T F_e, E, Mandel C:E                94
-  kinetics: 2 per system tau (9 FMA), ratio, pow, sign, dgamma        26 N_sl
-  L_p = sum gamma_dot P                          18 N_sl
-  residual, norms, tolerance                     72
-  G = F_e^T A                                    54
-  Jacobian rank-N_sl update: G^T Q (27 FMA), scale, 9x9 outer (81 FMA)   226 N_sl
-  9x9 LU with partial pivoting + solve           650
-  step update                                    36
+Newton iteration of integrateStress (N_sl slip systems, Schmid law), per cell:
+  F_e = A - dt (A L_p)                           63
+  S: F_e^T F_e - I, coordinates                  43
+  kinetics: tau (5 products) 9, ratio, pow, rate and derivative 6, L_p (8 FMA) 16     32 N_sl
+  L_p from coordinates, residual, norms          79
+  sum u q x P: 15 symmetric + 15 skew FMA, factors                                    66 N_sl
+  G = F_e^T A                                    45
+  reduced 5x5 matrix (5 products G W_l)          370
+  right-hand side                                55
+  5x5 Householder QR and solve                   270
+  x = res - sum y_l W_l, step                    107
 State-integrator iteration (beyond its Newton iterations):
-  dotState: kinetics without tangent (23 N_sl), hardening h0 |1-xi/xi_inf|^a (H |gamma_dot|)
-  (2 N_sl + 8 per system), damper and state update (9 per state entry, 2 N_sl entries)
-  + the integrateStress prologue/epilogue (inverse F_p0, A, F_p, P, det regularisation) 320
-Tangent kernel (once per cell and response): kinetics 26 N_sl; K assembly
-  (G2 P, symmetrise, C:, 9x9 outer) 279 N_sl; LU 650; 9 columns of
-  (rhs 80, solve 162, 37 N_sl, 405); invariants / polar decomposition 300.
+  rates from derivatives 11, 1 - xi / xi_sat, pow, h 6, hardening row 2 N_sl + 1, damper and update
+  (18 per state entry, 2 N_sl entries) 36, 1/xi 1, per system; determinants, zeta 45; half of the
+  prologue and epilogue (F_p0^-1, A, F_p, S, P: 400 a cell, about two iterations) 200
+Tangent kernel (once per cell and response): kinetics 32 N_sl, moments 66 N_sl; inverses and
+  products of 3x3 360; reduced matrix 370, traces 175, QR 167; T_l 1350; 9 columns of (right-hand
+  side 20, solve 100, z_6 20, 6-term sums 108, norm 18); rotation 250.
 """
 
 
 def newton_flops(nsl: int) -> int:
-    return 18 + 54 + 94 + 26 * nsl + 18 * nsl + 72 + 54 + 226 * nsl + 650 + 36
+    return 63 + 43 + 79 + 45 + 370 + 55 + 270 + 107 + 98 * nsl
 
 
 def state_flops(nsl: int) -> int:
-    return 23 * nsl + nsl * (2 * nsl + 8) + 9 * 2 * nsl + 10 + 320
+    return nsl * (2 * nsl + 55) + 245
 
 
 def tangent_flops(nsl: int) -> int:
-    return 26 * nsl + 80 + 108 + 279 * nsl + 650 + 216 + 9 * (80 + 162 + 37 * nsl + 405) + 300
+    return 98 * nsl + 360 + 370 + 175 + 167 + 1350 + 9 * 266 + 250
 
 
 def stress_kernel_flops(nsl: int, newton_iterations: int, state_iterations: int) -> int:
