@@ -444,17 +444,35 @@ DI void moments_apply(const double (*H)[RK], const double (*K)[RK], const double
 }
 
 // phenopowerlaw_dotState without twins (src/phase_mechanical_plastic_phenopowerlaw.f90:356-397)
-// from the gamma rates gs = |slip rate|: ws = 1/xi -> xi rate.
+// from the gamma rates gs = |slip rate| at the state xi(r): ws <- xi rate.
 // xi_sat = xi_inf + f_sat sqrt(sum F_tw) and hf = h_0 (1 + c_1 (sum F_tw)^c_2) at sum F_tw = 0
 // are tabulated per phase.  Returns true when a rate is NaN.
-template <int NSL, bool QP>
-DI bool dot_state(PhPtr ph, const double* gs, double* ws) {
+// xi / xi_sat is the rounded quotient: xi times the rounded 1 / xi_sat, corrected by its
+// residual (Markstein, IBM J. Res. Dev. 34(1) 1990), so that 1 - xi / xi_sat is exactly 0
+// where xi = xi_sat, as a power a_sl < 1 of it needs.  1 / xi in ws would leave 2e-16 there.
+// The sums over the acting systems come first: xi is still on its way from memory.
+template <int NSL, bool QP, class State>
+DI bool dot_state(PhPtr ph, State xi, const double* gs, double* ws) {
+  double hg[NSL];
+#pragma unroll
+  for (int r = 0; r < NSL; r++) hg[r] = 0.0;
+  bool nan = false;
+#pragma unroll 48 / NSL
+  for (int a = 0; a < NSL; a++) {
+    const double ga = gs[a * SWG];
+    nan |= (ga != ga);
+#pragma unroll
+    for (int r = 0; r < NSL; r++) hg[r] = fma(ph->Hc[a][r], ga, hg[r]);
+  }
   const int ak = QP ? ph->a_k : 0;
-#pragma unroll 1
+#pragma unroll
   for (int r0 = 0; r0 < NSL; r0 += CH) {
     double x[CH], p[CH];
 #pragma unroll
-    for (int j = 0; j < CH; j++) x[j] = 1.0 - dmk_rcp(ws[(r0 + j) * SWG] * ph->xi_sat[r0 + j]);   // 1 - xi / xi_sat
+    for (int j = 0; j < CH; j++) {
+      const double v = xi(r0 + j), inv = ph->inv_xi_sat[r0 + j], q = v * inv;
+      x[j] = 1.0 - fma(fma(-q, ph->xi_sat[r0 + j], v), inv, q);
+    }
     if (QP && ak) {
 #pragma unroll
       for (int j = 0; j < CH; j++) p[j] = fabs(x[j]);
@@ -467,24 +485,11 @@ DI bool dot_state(PhPtr ph, const double* gs, double* ws) {
       for (int j = 0; j < CH; j++) p[j] = ws[(r0 + j) * SWG];
     }
 #pragma unroll
-    for (int j = 0; j < CH; j++) ws[(r0 + j) * SWG] = ph->hf[r0 + j] * copysign(p[j], x[j]);
-  }
-  double hg[NSL];
-#pragma unroll
-  for (int r = 0; r < NSL; r++) hg[r] = 0.0;
-  bool nan = false;
-#pragma unroll 48 / NSL
-  for (int a = 0; a < NSL; a++) {
-    const double ga = gs[a * SWG];
-    nan |= (ga != ga);
-#pragma unroll
-    for (int r = 0; r < NSL; r++) hg[r] = fma(ph->Hc[a][r], ga, hg[r]);
-  }
-#pragma unroll
-  for (int r = 0; r < NSL; r++) {
-    const double d = ws[r * SWG] * hg[r];
-    ws[r * SWG] = d;
-    nan |= (d != d);
+    for (int j = 0; j < CH; j++) {
+      const double d = ph->hf[r0 + j] * copysign(p[j], x[j]) * hg[r0 + j];
+      ws[(r0 + j) * SWG] = d;
+      nan |= (d != d);
+    }
   }
   return nan;
 }
@@ -510,16 +515,20 @@ DI MpPtr fresh(MpPtr m) {
   return m;
 }
 
-// a field's value where a sub-step has completed (started) comes from the
-// sub-step scratch q, else from the increment's field f.  Almost no wavefront
-// holds a started cell: the scratch is read only in those that do.
-DI double ld_start(const double* f, const double* q, bool started, const Lane& l, int c) {
-  double v = ld(f, l, c);
+// n rows of a field from row c on: where a sub-step has completed (started) they
+// come from the sub-step scratch q, else from the increment's field f.  Almost no
+// wavefront holds a started cell: the scratch is read only in those that do.
+template <int n>
+DI void ld_start(const double* f, const double* q, bool started, const Lane& l, int c, double* v) {
+#pragma unroll
+  for (int r = 0; r < n; r++) v[r] = ld(f, l, c + r);
   if (__builtin_expect(__any(started), 0)) {
-    const double u = ld(q, l, c);
-    v = started ? u : v;
+#pragma unroll
+    for (int r = 0; r < n; r++) {
+      const double u = ld(q, l, c + r);
+      v[r] = started ? u : v[r];
+    }
   }
-  return v;
 }
 
 DI void m_load_start(const double* f, const double* q, bool started, const Lane& l, double* T) {
@@ -706,23 +715,17 @@ DI int integrate_state_fpi(PhPtr ph, const DmkNumMech& num, MpPtr m,
     m_mul(F, invFp0, A);
     det_Fp0 = m_det(Fp0);
   }
-  // row r of the state's start
-  auto xi_start = [&](MpPtr q, int r) { return ld_start(q->xi0, q->st0s, started, ln, r); };
-  auto gam_start = [&](MpPtr q, int r) {
-    return ld_start(q->gam0, q->st0s + NSL * ln.sN, started, ln, r);
-  };
   {
     double S0[9], s[6], x0[NSL];
     unsigned posm;
     MpPtr q = fresh(m);
-#pragma unroll
-    for (int r = 0; r < NSL; r++) x0[r] = xi_start(q, r);
+    ld_start<NSL>(q->xi0, q->st0s, started, ln, 0, x0);
     m_load(s_cur ? q->S : q->S0, ln, S0);
 #pragma unroll
     for (int r = 0; r < NSL; r++) ws[r * SWG] = dmk_rcp(x0[r]);
     sym_proj<RK>(S0, s);
     kinetics<NSL, QP, NS, false>(ph, s, ws, gs, nullptr, nullptr, posm);
-    if (dot_state<NSL, QP>(ph, gs, ws)) return ST_FAIL_STATE;
+    if (dot_state<NSL, QP>(ph, [&](int r) { return x0[r]; }, gs, ws)) return ST_FAIL_STATE;
     MpPtr q2 = fresh(m);
 #pragma unroll
     for (int r = 0; r < NSL; r++) {
@@ -743,20 +746,18 @@ DI int integrate_state_fpi(PhPtr ph, const DmkNumMech& num, MpPtr m,
     double w1[2 * NSL], w2[2 * NSL], s0[2 * NSL];
 #pragma unroll
     for (int r = 0; r < 2 * NSL; r++) w1[r] = ld(w1p, ln, r);
+    ld_start<NSL>(q->xi0, q->st0s, started, ln, 0, s0);
+    // the converged Newton iterate evaluated kinetics_sl at this (S, xi): rates
+    // are in gs.  A NaN rate ends the iteration with the status of the stress
+    // integration, as the reference's exit does (phase_mechanical.f90:638)
+    const bool nan = dot_state<NSL, QP>(ph, [&](int r) { return fma(w1[r], dt, s0[r]); }, gs, ws);
+    ld_start<NSL>(q->gam0, q->st0s + NSL * ln.sN, started, ln, 0, s0 + NSL);
 #pragma unroll
     for (int r = 0; r < 2 * NSL; r++) w2[r] = 0.0;
     if (it > 1) {
 #pragma unroll
       for (int r = 0; r < 2 * NSL; r++) w2[r] = ld(w2p, ln, r);
     }
-    // the converged Newton iterate evaluated kinetics_sl at this (S, xi): rates
-    // are in gs.  A NaN rate ends the iteration with the status of the stress
-    // integration, as the reference's exit does (phase_mechanical.f90:638)
-    const bool nan = dot_state<NSL, QP>(ph, gs, ws);
-#pragma unroll
-    for (int r = 0; r < NSL; r++) s0[r] = xi_start(q, r);
-#pragma unroll
-    for (int r = 0; r < NSL; r++) s0[NSL + r] = gam_start(q, r);
     // damper (src/phase_mechanical.f90:653-674)
     double d12 = 0.0, d22 = 0.0, d01 = 0.0;
 #pragma unroll
@@ -886,8 +887,11 @@ DI void stress_body(MpPtr m, const double* __restrict__ Ftarget, PhPtr ph, int p
     m_store(q->S, ln, T);
 #pragma unroll 1
     for (int r = 0; r < NSL; r++) {
-      st(q->xi, ln, r, ld_start(q->xi0, q->st0s, started, ln, r));
-      st(q->gam, ln, r, ld_start(q->gam0, q->st0s + NSL * ln.sN, started, ln, r));
+      double v[2];
+      ld_start<1>(q->xi0, q->st0s, started, ln, r, v);
+      ld_start<1>(q->gam0, q->st0s + NSL * ln.sN, started, ln, r, v + 1);
+      st(q->xi, ln, r, v[0]);
+      st(q->gam, ln, r, v[1]);
     }
   }
   MpPtr q4 = fresh(m);

@@ -5,6 +5,7 @@
 //   notation (:1711-1759) and its contraction with the projections.
 // The slip-system directions/normals and the interaction-type tables are
 // crystallographic data and are necessarily the reference's values.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -221,7 +222,8 @@ int dmk_build_phase(const dmk_phase_desc* d, DmkPhaseDev* p) {
       p->c1[a] = d->c_1[f];
       p->c2[a] = d->c_2[f];
       p->fsat[a] = d->f_sat[f];
-      p->xi_sat[a] = d->xi_inf[f] + d->f_sat[f] * std::sqrt(0.0);
+      // an infinite xi_inf (hardening without saturation) as a finite one that leaves 1 - xi / xi_sat = 1
+      p->xi_sat[a] = std::min(d->xi_inf[f] + d->f_sat[f] * std::sqrt(0.0), 1.0e300);
       p->inv_xi_sat[a] = 1.0 / p->xi_sat[a];
       p->hf[a] = d->h_0[f] * (1.0 + d->c_1[f] * std::pow(0.0, d->c_2[f]));
     }
