@@ -252,14 +252,15 @@ void batch_launch_locked(DmkStressBatch* b, std::unique_lock<std::mutex>& lk) {
     if (!rc && !(r.resid && r.rq.idle) && hipStreamWaitEvent(b->st, b->ev_in[r.slot], 0) != hipSuccess)
       rc = DMK_ERR_HIP;
   struct Group { int key, off, n, blocks; };
-  Group g[4];
+  constexpr int NKEY = 8;            // 12 or 24 systems, Schmid law or not, quarter powers or not
+  Group g[NKEY];
   int ng = 0, off = 0;
   for (auto& r : b->reqs)
     for (int i = 0; i < r.n; i++) {
       int k = 0;
       while (k < ng && g[k].key != r.key[i]) k++;
       if (k == ng) {
-        if (ng == 4) { rc = DMK_ERR_CONFIG; break; }
+        if (ng == NKEY) { rc = DMK_ERR_CONFIG; break; }
         g[ng++] = Group{r.key[i], 0, 0, 0};
       }
     }
