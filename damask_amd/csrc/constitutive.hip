@@ -403,7 +403,8 @@ DI void slip_moments(PhPtr ph, const double* us, double scale, unsigned posm,
 
 // The 9x9 systems of the material point (identity plus one rank-1 term per
 // slip system) reduced to the RK symmetric directions: with W_l as above and
-// t_k(X) = E_k : (G X), N_kl = delta_kl / C_k + t_k(W_l).
+// t_k(X) = E_k : (G X), N_kl = delta_kl + C_k t_k(W_l), C_k the modulus of E_k (any
+// of them may be zero).
 template <int RK>
 DI void reduced_matrix(PhPtr ph, const double* G, const double (*H)[RK],
                        const double (*K)[RK], double* N) {
@@ -418,10 +419,8 @@ DI void reduced_matrix(PhPtr ph, const double* G, const double (*H)[RK],
     m_mul(G, W, GW);
     sym_proj<RK>(GW, t);
 #pragma unroll
-    for (int k = 0; k < RK; k++) N[RK * k + l] = t[k];
+    for (int k = 0; k < RK; k++) N[RK * k + l] = k == l ? fma(modulus<RK>(ph, k), t[k], 1.0) : modulus<RK>(ph, k) * t[k];
   }
-#pragma unroll
-  for (int k = 0; k < RK; k++) N[(RK + 1) * k] += 1.0 / modulus<RK>(ph, k);
 }
 
 // sum_l y_l W_l
@@ -582,7 +581,7 @@ DI void elastic_F(double dt, const double* A, const double* Lp, double* Fe) {
 // The Newton system (I9 + sum_a u_a vec(P_a) vec(G^T C:P_nS_a)^T) x = res,
 // G = F_e^T A, u_a = dt d rate_a / d tau_a, is the identity plus a map that sees
 // x only through t_k(x) = E_k : (G x): with y_l = C_l t_l(x),
-//   x = res - sum_l y_l W_l,   N y = t(res),   N_kl = delta_kl / C_k + t_k(W_l),
+//   x = res - sum_l y_l W_l,   N y = C t(res),   N_kl = delta_kl + C_k t_k(W_l),
 // W_l = sum_a u_a q_al P_a.  So a 5x5 system (6x6 with non-Schmid terms) is
 // assembled and solved instead of an 8x8 one: the same Newton step.
 template <int NSL, bool QP, bool NS>
@@ -643,6 +642,8 @@ DI int integrate_stress(PhPtr ph, const DmkNumMech& num, const double* A, double
       reduced_matrix<RK>(ph, G, H, K, N);
       m_mul(G, res, GX);
       sym_proj<RK>(GX, y);
+#pragma unroll
+      for (int k = 0; k < RK; k++) y[k] *= modulus<RK>(ph, k);
       if (dmk_qr_factor<RK>(N, rd, v0, tau)) return ST_FAIL_LP_DGESV;
       dmk_qr_apply_solve<RK>(N, rd, v0, tau, y);
     }
@@ -1061,8 +1062,8 @@ DI double wave_rows(double a, double b, double c, double d) {
 //
 // Column (k, l): dS = dS/dF_kl solves dS + dt sum_a dg_a C:sym(G2 P_a) (P_nS_a : dS)
 // = C:sym(X), X = F_e(k,:) (x) F_p^-1(l,:), G2 = F_e^T A2.  As in the stress
-// integration the sum acts through the E coordinates z of dS alone: N z = E:X with
-// N_kl = delta_kl / C_k + dt E_k : (G2 W_l), one 5x5 (6x6) factorisation for the
+// integration the sum acts through the E coordinates z of dS alone: N z = C E:X with
+// N_kl = delta_kl + dt C_k E_k : (G2 W_l), one 5x5 (6x6) factorisation for the
 // nine columns; then t = sum_a dg_a P_a (P_nS_a : dS) = sum_l z_l W_l,
 // dS = sum_k z_k E_k with z_6 = C_6 E_6 : (X - dt G2 t), and with
 // D = -dt F_p0^-1 t the derivative of F_p^-1
@@ -1191,12 +1192,10 @@ tangent_kernel(DmkMPDev mp, const DmkPhaseDev* __restrict__ ph_, int phase_id, d
 #pragma unroll
         for (int m = 0; m < 3; m++) X[3 * n + m] = fk[n] * pl[m];
       sym_proj<RK>(X, z[k]);
-      if (!sing) {
-        dmk_qr_apply_solve<RK>(N, rd, v0, tau, z[k]);
-      } else {                     // as after a failed solve: dS = C:sym(X)
 #pragma unroll
-        for (int q = 0; q < RK; q++) z[k][q] *= modulus<RK>(ph, q);
-      }
+      for (int q = 0; q < RK; q++) z[k][q] *= modulus<RK>(ph, q);
+      // (as after a failed solve where N is singular: dS = C:sym(X))
+      if (!sing) dmk_qr_apply_solve<RK>(N, rd, v0, tau, z[k]);
       if (RK == 5) {
         double v = (X[0] + X[4] + X[8]) * R3;
         if (!sing) {
