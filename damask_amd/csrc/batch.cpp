@@ -80,6 +80,8 @@ struct DmkStressBatch {
   double* rep_dev[NSTAGE] = {};
   double* rep_host[NSTAGE] = {};
   std::vector<int> slot_stage, rep_idx, order;
+  std::vector<DmkFFT> shapes;        // one per grid and choice of fused passes (dmk_stress_batch_shapes)
+  int64_t n_transforms = 0;          // launches of the transforms over the rounds' RVEs
   // DMK_BATCH_TIMING: host time of the submitting threads spent waiting for
   // the round to start (the other RVEs' submissions and the launch), waiting
   // for the round on the device, and the launches themselves
@@ -206,6 +208,7 @@ int resid_launch_locked(DmkStressBatch* b, int s, int nr) {
     int k1 = k0 + 1;
     while (k1 < ntr && same_fft(f, b->reqs[b->order[k1]].fft)) k1++;
     const int rc = dmk_transform_batch(f, R + k0, k1 - k0, b->st);
+    b->n_transforms++;
     if (rc == 1) {
       // no fused kernels for this configuration: each RVE's transform on its own
       for (int k = k0; k < k1; k++) {
@@ -503,6 +506,14 @@ int dmk_resid_batch_submit(DmkStressBatch* b, int slot, const DmkStressItem* ite
 
 bool dmk_stress_batch_resid(const DmkStressBatch* b) { return b && b->resid; }
 
+DmkFFTShapes dmk_stress_batch_shapes(DmkStressBatch* b, const DmkFFT* fft) {
+  std::lock_guard<std::mutex> lk(b->mu);
+  for (const DmkFFT& f : b->shapes)
+    if (std::equal(f.n, f.n + 3, fft->n) && !f.xy_threads == !fft->xy_threads && !f.zgz_g == !fft->zgz_g) return f;
+  b->shapes.push_back(*fft);
+  return *fft;
+}
+
 // lockstep groups (DMK_LOCKSTEP_GROUPS, default 1): thread t belongs to
 // group t % ng.  The groups' rounds are independent, so one group's host
 // work between rounds overlaps the other groups' rounds on the device.  On
@@ -541,9 +552,9 @@ static void print_timing(const std::vector<std::unique_ptr<DmkStressBatch>>& grp
     const double ns = (double)b.n_sub, nr = (double)std::max<uint64_t>(b.gen, 1);
     fprintf(stderr,
             "lockstep group %zu timing: %llu rounds, %lld submissions; per submission %.3f ms waiting for the round "
-            "to start, %.3f ms for the device; launches %.3f ms per round\n",
+            "to start, %.3f ms for the device; launches %.3f ms per round, transforms in %.2f launches of each kernel\n",
             k, (unsigned long long)b.gen, (long long)b.n_sub.load(), b.t_wait_ns * 1e-6 / ns, b.t_gpu_ns * 1e-6 / ns,
-            b.t_launch_ns * 1e-6 / nr);
+            b.t_launch_ns * 1e-6 / nr, (double)b.n_transforms / nr);
     if (b.stamp) {
       hipStreamSynchronize(b.st);     // the host functions of the last rounds
       double dev = 0.0, wake = 0.0;

@@ -21,6 +21,11 @@ void dmk_set_stress_batch(dmk_handle* h, DmkStressBatch* b, int slot);
 bool dmk_stress_batch_resid(const DmkStressBatch* b);
 struct DmkResidDev;
 struct DmkFFT;
+struct DmkFFTShapes;
+// Tile shapes for an RVE's transforms in the batch's rounds: those of the first
+// RVE of its grid, with the same passes fused, that asked.  Each handle times its
+// own, and RVEs whose shapes differ cannot share a launch.
+DmkFFTShapes dmk_stress_batch_shapes(DmkStressBatch* b, const DmkFFT* fft);
 // Hand a request of a lockstep round to the batch (struct DmkResidDev: a
 // whole residual evaluation with its stress items, an application of the
 // adjoint's operator, or dot products; fft is the RVE's FFT configuration and

@@ -31,16 +31,19 @@ struct FftPlan {
 // lines per block of the y and z passes; xy_threads > 0: the x and y passes
 // run fused, one block of that many threads per (field, z) plane (all picked
 // by dmk_fft_tune)
-struct DmkFFT {
-  int n[3];
-  int h;
-  FftPlan plan[3];
-  double2* tw[3] = {nullptr, nullptr, nullptr};
+struct DmkFFTShapes {
   int gx[3] = {0, 0, 0};
   int xy_threads = 0;
   int xy_ip = 0;                    // 1: the fused x-y kernels' single-buffer (in-place) variant
   int zgz_g = 0, zgz_threads = 0;   // > 0: z passes and Gamma fused, zgz_g columns per block
   int zgz_ip = 0;                   // 1: the fused z kernel's single-buffer variant
+};
+
+struct DmkFFT : DmkFFTShapes {
+  int n[3];
+  int h;
+  FftPlan plan[3];
+  double2* tw[3] = {nullptr, nullptr, nullptr};
 };
 
 struct GammaArgs {

@@ -193,6 +193,7 @@ struct dmk_handle {
   double wgt;
   hipStream_t st = nullptr;
   DmkFFT fft;
+  DmkFFTShapes fft_own;              // the shapes its own set-up picked (a lockstep batch lends others)
   int n_phases;
   std::vector<DmkPhaseDev> ph;
   DmkPhaseDev* ph_dev = nullptr;
@@ -258,6 +259,10 @@ struct dmk_handle {
 };
 
 void dmk_set_stress_batch(dmk_handle* h, DmkStressBatch* b, int slot) {
+  DmkFFTShapes& own = h->fft;
+  if (h->batch) own = h->fft_own;
+  h->fft_own = own;
+  if (b && dmk_stress_batch_resid(b)) own = dmk_stress_batch_shapes(b, &h->fft);
   h->batch = b;
   h->batch_slot = slot;
 }
