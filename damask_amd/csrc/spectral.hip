@@ -1024,7 +1024,8 @@ static FftPlan make_plan(int L) {
   p.half = dmk_fft_div(L / 2 + 1);
   // the first radix-8 stage writes every eighth entry: one pad per eight spreads
   // them over the banks.  64 | L keeps the other stages' strides constant; long
-  // lines are left dense for their LDS.  An odd line distance spreads the columns.
+  // lines are left dense for their LDS, and so are others where the padding does
+  // not fit a kernel's LDS (pad_or_dense).  An odd line distance spreads the columns.
   p.ps = L % 64 == 0 && L <= 1024 ? 3 : 31;
   p.ldl = (L + (p.ps < 31 ? L >> p.ps : 0)) | 1;
   return p;
@@ -1122,25 +1123,63 @@ static const size_t FFT_LDS_MAX = 64 * 1024;
 // the fused kernels may take more (the MI355X allows 160 KB per block)
 static const size_t FFT_XY_LDS_MAX = 160 * 1024;
 
-// LDS of `lines` lines of axis d in two buffers
-static size_t lines_lds(const DmkFFT* fft, int d, int lines) {
-  return 2 * sizeof(double2) * (size_t)lines * fft->plan[d].ldl;
+// beside a few static sums
+static const size_t FFT_ZGZ_LDS_MAX = FFT_XY_LDS_MAX - 256;
+
+static FftPlan dense(FftPlan p) {
+  p.ps = 31;
+  p.ldl = p.L | 1;
+  return p;
 }
 
-static size_t xy_lds(const DmkFFT* fft, int ip) {
-  return (ip ? 1 : 2) * sizeof(double2) * (size_t)xy_buf(fft->plan[0], fft->plan[1]);
+// `lines` lines of axis d in two buffers
+struct LinePlan {
+  FftPlan p;
+  size_t lds;
+};
+static LinePlan line_plan(const FftPlan& p, size_t lines, int buffers, size_t lds_max) {
+  const size_t lds = buffers * sizeof(double2) * lines * p.ldl;
+  if (lds <= lds_max || p.ps == 31) return LinePlan{p, lds};
+  const FftPlan q = dense(p);
+  return LinePlan{q, buffers * sizeof(double2) * lines * q.ldl};
 }
+static LinePlan line_plan(const DmkFFT* fft, int d, int lines) {
+  return line_plan(fft->plan[d], lines, 2, FFT_LDS_MAX);
+}
+static size_t lines_lds(const DmkFFT* fft, int d, int lines) { return line_plan(fft, d, lines).lds; }
+
+// the plans of a fused x-y kernel: padded lines where the plane then fits its
+// LDS, dense ones where it does not (64x144 cells and 74 other planes with edges
+// below 400 have no fused pass otherwise)
+struct PlanePlans {
+  FftPlan x, y;
+  size_t lds;
+};
+static PlanePlans xy_plans(const DmkFFT* fft, int ip) {
+  PlanePlans q{fft->plan[0], fft->plan[1], 0};
+  auto lds = [&] { return (ip ? 1 : 2) * sizeof(double2) * (size_t)xy_buf(q.x, q.y); };
+  q.lds = lds();
+  if (q.lds > FFT_XY_LDS_MAX) {
+    q.x = dense(q.x);
+    q.y = dense(q.y);
+    q.lds = lds();
+  }
+  return q;
+}
+static size_t xy_lds(const DmkFFT* fft, int ip) { return xy_plans(fft, ip).lds; }
 
 static void launch_xy_r2c(const DmkFFT* fft, int howmany, const double* in, double2* out, int threads, int ip,
                           hipStream_t s) {
-  hipLaunchKernelGGL(ip ? fft_xy_r2c_ip : fft_xy_r2c, dim3(howmany * fft->n[2]), dim3(threads), xy_lds(fft, ip), s, in,
-                     out, fft->n[2], fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
+  const PlanePlans q = xy_plans(fft, ip);
+  hipLaunchKernelGGL(ip ? fft_xy_r2c_ip : fft_xy_r2c, dim3(howmany * fft->n[2]), dim3(threads), q.lds, s, in, out,
+                     fft->n[2], q.x, fft->tw[0], q.y, fft->tw[1]);
 }
 
 static void launch_yx_c2r(const DmkFFT* fft, int howmany, const double2* in, double* out, int threads, int ip,
                           hipStream_t s) {
-  hipLaunchKernelGGL(ip ? fft_yx_c2r_ip : fft_yx_c2r, dim3(howmany * fft->n[2]), dim3(threads), xy_lds(fft, ip), s, in,
-                     out, fft->n[2], fft->plan[0], fft->tw[0], fft->plan[1], fft->tw[1]);
+  const PlanePlans q = xy_plans(fft, ip);
+  hipLaunchKernelGGL(ip ? fft_yx_c2r_ip : fft_yx_c2r, dim3(howmany * fft->n[2]), dim3(threads), q.lds, s, in, out,
+                     fft->n[2], q.x, fft->tw[0], q.y, fft->tw[1]);
 }
 
 // the in-place kernels need radix 2/4/8 plans and every stage of `lines` lines
@@ -1164,15 +1203,15 @@ static bool xy_ip_fits(const DmkFFT* fft, int threads) {
 static void launch_x_r2c(const DmkFFT* fft, int howmany, const double* in, double2* out, int ppb, hipStream_t s) {
   int nl = howmany * fft->n[1] * fft->n[2];
   int nblk = (nl + 2 * ppb - 1) / (2 * ppb);
-  hipLaunchKernelGGL(fft_x_r2c, dim3(nblk), dim3(256), lines_lds(fft, 0, ppb), s, in, out, nl, fft->plan[0],
-                     fft->tw[0], ppb);
+  const LinePlan q = line_plan(fft, 0, ppb);
+  hipLaunchKernelGGL(fft_x_r2c, dim3(nblk), dim3(256), q.lds, s, in, out, nl, q.p, fft->tw[0], ppb);
 }
 
 static void launch_x_c2r(const DmkFFT* fft, int howmany, const double2* in, double* out, int ppb, hipStream_t s) {
   int nl = howmany * fft->n[1] * fft->n[2];
   int nblk = (nl + 2 * ppb - 1) / (2 * ppb);
-  hipLaunchKernelGGL(fft_x_c2r, dim3(nblk), dim3(256), lines_lds(fft, 0, ppb), s, in, out, nl, fft->plan[0],
-                     fft->tw[0], ppb);
+  const LinePlan q = line_plan(fft, 0, ppb);
+  hipLaunchKernelGGL(fft_x_c2r, dim3(nblk), dim3(256), q.lds, s, in, out, nl, q.p, fft->tw[0], ppb);
 }
 
 // y (axis 1) or z (axis 2) pass over the half spectra, in place
@@ -1181,24 +1220,24 @@ static void launch_strided(const DmkFFT* fft, int howmany, double2* data, int ax
   const long Nk = (long)h * N2 * N3;
   const int nch = (h + gx - 1) / gx, M = axis == 1 ? N3 : N2;
   const long outer = axis == 1 ? (long)h * N2 : h, stride = axis == 1 ? h : (long)h * N2;
-  hipLaunchKernelGGL(sign < 0 ? fft_strided<-1> : fft_strided<+1>, dim3(howmany * M * nch), dim3(256),
-                     lines_lds(fft, axis, gx), s, data, h, dmk_fft_div(gx), M, Nk, outer, stride, fft->plan[axis],
-                     fft->tw[axis]);
+  const LinePlan q = line_plan(fft, axis, gx);
+  hipLaunchKernelGGL(sign < 0 ? fft_strided<-1> : fft_strided<+1>, dim3(howmany * M * nch), dim3(256), q.lds, s, data, h,
+                     dmk_fft_div(gx), M, Nk, outer, stride, q.p, fft->tw[axis]);
 }
 
-// (beside a few static sums)
-static const size_t FFT_ZGZ_LDS_MAX = FFT_XY_LDS_MAX - 256;
-static size_t zgz_lds(const DmkFFT* fft, int gz, int ip) {
-  return (ip ? 1 : 2) * sizeof(double2) * 9 * gz * (size_t)fft->plan[2].ldl;
+static LinePlan zgz_plan(const DmkFFT* fft, int gz, int ip) {
+  return line_plan(fft->plan[2], 9 * gz, ip ? 1 : 2, FFT_ZGZ_LDS_MAX);
 }
+static size_t zgz_lds(const DmkFFT* fft, int gz, int ip) { return zgz_plan(fft, gz, ip).lds; }
 
 template <class Op>
 static void launch_zgz(const DmkFFT* fft, double2* Z, const Op& op, int gz, int threads, int ip, double* div_partial,
                        hipStream_t s) {
   const long M = (long)fft->h * fft->n[1];
   unsigned nb = (unsigned)((M + gz - 1) / gz);
-  hipLaunchKernelGGL(ip ? fft_zgz_ip<Op> : fft_zgz<Op>, dim3(nb), dim3(threads), zgz_lds(fft, gz, ip), s, Z, op,
-                     fft->plan[2], fft->tw[2], dmk_fft_div(gz), div_partial);
+  const LinePlan q = zgz_plan(fft, gz, ip);
+  hipLaunchKernelGGL(ip ? fft_zgz_ip<Op> : fft_zgz<Op>, dim3(nb), dim3(threads), q.lds, s, Z, op, q.p, fft->tw[2],
+                     dmk_fft_div(gz), div_partial);
 }
 
 int dmk_fft_tune(DmkFFT* fft, double2* cscratch, double* rscratch, hipStream_t s) {
@@ -1330,14 +1369,15 @@ int dmk_transform_batch(const DmkFFT* fft, const DmkResidDev* R, int nr, hipStre
   const dim3 gxy(9 * N3, nr);
   const long M = (long)fft->h * N2;
   const dim3 gzz((unsigned)((M + fft->zgz_g - 1) / fft->zgz_g), nr);
-  const FftPlan &px = fft->plan[0], &py = fft->plan[1], &pz = fft->plan[2];
+  const PlanePlans q = xy_plans(fft, fft->xy_ip);
+  const LinePlan z = zgz_plan(fft, fft->zgz_g, fft->zgz_ip);
   const dim3 txy(fft->xy_threads), tz(fft->zgz_threads);
-  hipLaunchKernelGGL(fft->xy_ip ? fft_xy_r2c_batch<true> : fft_xy_r2c_batch<false>, gxy, txy, xy_lds(fft, fft->xy_ip),
-                     s, R, N3, px, fft->tw[0], py, fft->tw[1]);
-  hipLaunchKernelGGL(fft->zgz_ip ? fft_zgz_batch<true> : fft_zgz_batch<false>, gzz, tz,
-                     zgz_lds(fft, fft->zgz_g, fft->zgz_ip), s, R, pz, fft->tw[2], dmk_fft_div(fft->zgz_g));
-  hipLaunchKernelGGL(fft->xy_ip ? fft_yx_c2r_batch<true> : fft_yx_c2r_batch<false>, gxy, txy, xy_lds(fft, fft->xy_ip),
-                     s, R, N3, px, fft->tw[0], py, fft->tw[1]);
+  hipLaunchKernelGGL(fft->xy_ip ? fft_xy_r2c_batch<true> : fft_xy_r2c_batch<false>, gxy, txy, q.lds, s, R, N3, q.x,
+                     fft->tw[0], q.y, fft->tw[1]);
+  hipLaunchKernelGGL(fft->zgz_ip ? fft_zgz_batch<true> : fft_zgz_batch<false>, gzz, tz, z.lds, s, R, z.p, fft->tw[2],
+                     dmk_fft_div(fft->zgz_g));
+  hipLaunchKernelGGL(fft->xy_ip ? fft_yx_c2r_batch<true> : fft_yx_c2r_batch<false>, gxy, txy, q.lds, s, R, N3, q.x,
+                     fft->tw[0], q.y, fft->tw[1]);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 

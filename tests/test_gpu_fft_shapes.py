@@ -41,6 +41,16 @@ def test_transforms_against_numpy(gpu_lib, cells, xy, monkeypatch):
     g.close()
 
 
+@pytest.mark.parametrize("cells", [[64, 144, 2], [144, 64, 2], [128, 72, 1], [72, 128, 2], [192, 48, 1], [28, 320, 1]])
+def test_planes_too_large_for_padded_lines_stay_fused(gpu_lib, cells, monkeypatch):
+    """planes that fit the two-buffer x-y kernels' LDS with dense lines only"""
+    monkeypatch.setenv("DMK_FFT_XY", "1")
+    g, _ = _solver(cells)
+    assert g.scalar("fft_path")[0] > 0
+    g.close()
+    test_transforms_against_numpy(gpu_lib, cells, "1", monkeypatch)
+
+
 @pytest.mark.parametrize("zgz", ["0", "1", "2"])
 @pytest.mark.parametrize("cells", [[4, 6, 128], [2, 3, 192], [130, 2, 64], [6, 5, 22]])
 def test_gamma_convolution_against_oracle(gpu_lib, oracle, cells, zgz, monkeypatch):
