@@ -92,9 +92,9 @@ int dmk_forward_field(long N, int guess, double dt_old, double dt, const Forward
                       double* F_lastinc, double* Fdot, double* Fnew, hipStream_t s);
 int dmk_shift_field(long N, const ForwardArgs* fa, double* F, hipStream_t s);
 int dmk_copy_jobs(const CopyJobs* j, hipStream_t s);
-// w values a cell: cell-major a (of n cells) <-> component-major soa (of N cells) for the cells e0 .. e0 + n - 1
-int dmk_aos_to_soa(const double* a, long N, int w, long e0, long n, double* soa, hipStream_t s);
-int dmk_soa_to_aos(const double* soa, long N, int w, long e0, long n, double* a, hipStream_t s);
+// w values a cell: cell-major a <-> component-major soa
+int dmk_aos_to_soa(const double* a, long N, int w, double* soa, hipStream_t s);
+int dmk_soa_to_aos(const double* soa, long N, int w, double* a, hipStream_t s);
 
 // constitutive launchers (constitutive.hip)
 struct DmkMPDev;

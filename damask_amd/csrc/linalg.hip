@@ -556,30 +556,30 @@ __global__ void copy_jobs_kernel(CopyJobs j) {
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) dst[i] = src[i];
 }
 
-// Cell-major (w values a cell) <-> component-major (stride N) for the cells e0 ..
-// e0 + n - 1.  A block turns a tile of tc cells around in LDS, so that both sides
-// are read and written in whole lines; the odd pitch keeps the strided side free of
-// bank conflicts.  HBM-bound: 64x60x63 cells of 9 values, norm of the divergence
-// 58.2 -> 57.2 us against one value a thread and scattered lines.
+// Cell-major (w values a cell) <-> component-major (stride N).  A block turns a
+// tile of tc cells around in LDS, so that both sides are read and written in
+// whole lines; the odd pitch keeps the strided side free of bank conflicts.
+// HBM-bound: 64x60x63 cells of 9 values, norm of the divergence 58.2 -> 57.2 us
+// against one value a thread and scattered lines.
 #define TR_TILE 2560
 __host__ __device__ inline int tr_pitch(int w) { return w | 1; }
-// cells of a tile: 18 KB of LDS, fewer where that leaves less than 256 blocks (8^3
-// cells in two blocks made a response 2 % slower)
-inline int tr_cells(int w, long n) {
+// cells of a tile: at most 20 KB of LDS (18 KB for 9 values a cell), fewer where
+// that leaves less than 256 blocks (8^3 cells in two blocks made a response 2 % slower)
+inline int tr_cells(int w, long N) {
   int c = TR_TILE / tr_pitch(w) / 64 * 64;
-  while (c > 16 && n / c < 256) c /= 2;
+  while (c > 16 && N / c < 256) c /= 2;
   return c > 16 ? c : 16;
 }
 
 template <bool TO_SOA>
 __global__ void __launch_bounds__(RB) transpose_cells(const double* __restrict__ src, double* __restrict__ dst, long N,
-                                                      int w, long e0, long n, int tc) {
+                                                      int w, int tc) {
   extern __shared__ double tile[];
   const int pitch = tr_pitch(w), t = threadIdx.x;
   const long b0 = (long)blockIdx.x * tc;
-  const int nc = (int)min((long)tc, n - b0);
-  const double* __restrict__ in = TO_SOA ? src + b0 * w : src + e0 + b0;
-  double* __restrict__ out = TO_SOA ? dst + e0 + b0 : dst + b0 * w;
+  const int nc = (int)min((long)tc, N - b0);
+  const double* __restrict__ in = TO_SOA ? src + b0 * w : src + b0;
+  double* __restrict__ out = TO_SOA ? dst + b0 : dst + b0 * w;
   if (TO_SOA) {
     for (unsigned i = t; i < (unsigned)(nc * w); i += RB) {
       const unsigned e = i / (unsigned)w, c = i - e * (unsigned)w;
@@ -758,18 +758,16 @@ int dmk_copy_jobs(const CopyJobs* j, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
-int dmk_aos_to_soa(const double* a, long N, int w, long e0, long n, double* soa, hipStream_t s) {
-  if (n < 1) return 0;
-  const int tc = tr_cells(w, n);
-  hipLaunchKernelGGL(transpose_cells<true>, dim3((unsigned)((n + tc - 1) / tc)), dim3(RB),
-                     sizeof(double) * tc * tr_pitch(w), s, a, soa, N, w, e0, n, tc);
+int dmk_aos_to_soa(const double* a, long N, int w, double* soa, hipStream_t s) {
+  const int tc = tr_cells(w, N);
+  hipLaunchKernelGGL(transpose_cells<true>, dim3((unsigned)((N + tc - 1) / tc)), dim3(RB),
+                     sizeof(double) * tc * tr_pitch(w), s, a, soa, N, w, tc);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
-int dmk_soa_to_aos(const double* soa, long N, int w, long e0, long n, double* a, hipStream_t s) {
-  if (n < 1) return 0;
-  const int tc = tr_cells(w, n);
-  hipLaunchKernelGGL(transpose_cells<false>, dim3((unsigned)((n + tc - 1) / tc)), dim3(RB),
-                     sizeof(double) * tc * tr_pitch(w), s, soa, a, N, w, e0, n, tc);
+int dmk_soa_to_aos(const double* soa, long N, int w, double* a, hipStream_t s) {
+  const int tc = tr_cells(w, N);
+  hipLaunchKernelGGL(transpose_cells<false>, dim3((unsigned)((N + tc - 1) / tc)), dim3(RB),
+                     sizeof(double) * tc * tr_pitch(w), s, soa, a, N, w, tc);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }

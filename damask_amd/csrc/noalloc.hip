@@ -114,7 +114,7 @@ extern "C" int dmk_divergence_rms_noalloc(const int32_t cells[3], const double s
     dmk_set_error("dmk_divergence_rms_noalloc: FFT set-up failed: %s", hipGetErrorString(hipGetLastError()));
     return DMK_ERR_HIP;
   }
-  if (dmk_aos_to_soa(field_dev, N, 9, 0, N, soa, s) || dmk_fft_r2c(&fft, 9, soa, Z, s)) {
+  if (dmk_aos_to_soa(field_dev, N, 9, soa, s) || dmk_fft_r2c(&fft, 9, soa, Z, s)) {
     dmk_set_error("dmk_divergence_rms_noalloc: transform launch failed: %s", hipGetErrorString(hipGetLastError()));
     return DMK_ERR_HIP;
   }

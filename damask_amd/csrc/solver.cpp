@@ -19,6 +19,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "dmk_common.h"
@@ -204,6 +205,9 @@ struct dmk_handle {
   std::vector<void*> allocs;
   double *P_hom, *dPdF;
   double *F, *F_lastinc, *Fdot, *R, *XM, *FM, *XA, *FA, *Xh, *Fh, *Fext, *Pext;
+  double* stage = nullptr;           // fields to and from the host (stage_get), under stage_mu
+  size_t stage_n = 0;
+  std::mutex stage_mu;
   double2 *Z, *U;
   double *u3, *xn_dev, *xp_dev;
   double *partial, *small, *nrm, *pmax, *pmin;
@@ -1985,6 +1989,7 @@ extern "C" void dmk_mech_destroy(dmk_handle* h) {
     for (int k = 0; k < 8; k++) { hipEventDestroy(h->ev[k][0]); hipEventDestroy(h->ev[k][1]); }
   adj_free(h);
   for (void* p : h->allocs) hipFree(p);
+  if (h->stage) hipFree(h->stage);
   if (h->ph_dev) hipFree(h->ph_dev);
   if (h->hsmall) hipHostFree(h->hsmall);
   dmk_fft_free(&h->fft);
@@ -2082,7 +2087,7 @@ static int init_impl(dmk_handle* h, const int32_t cells[3], const double size[3]
   const long nx = h->nx;
   double** sol[] = {&h->F, &h->F_lastinc, &h->Fdot, &h->R, &h->XM, &h->FM, &h->XA, &h->FA};
   for (auto pp : sol) if ((rc = dalloc(h, pp, nx))) return rc;
-  if ((rc = dalloc(h, &h->Fext, n9)) || (rc = dalloc(h, &h->Pext, std::max(n9, 96L)))) return rc;   // a cell of any field
+  if ((rc = dalloc(h, &h->Fext, n9)) || (rc = dalloc(h, &h->Pext, n9))) return rc;
   if (h->scheme != 0 && (rc = dalloc(h, &h->T, n9))) return rc;
   // NGMRES history (M pairs), or for the Galerkin scheme the 31 Krylov vectors of GMRES(30)
   if (h->scheme == 2) {
@@ -2321,11 +2326,11 @@ extern "C" int dmk_constitutive(dmk_handle* h, double dt, const double* F, doubl
                                 double* C_volAvg, double* C_minMaxAvg, int32_t* status) {
   if (!h || !F) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, F, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, 0, h->N, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
   int rc = constitutive(h, h->Fext, dt, false, true);
   if (rc) return rc;
   if (P) {
-    CKL(dmk_soa_to_aos(h->P_hom, h->N, 9, 0, h->N, h->Pext, h->st));
+    CKL(dmk_soa_to_aos(h->P_hom, h->N, 9, h->Pext, h->st));
     CK(hipMemcpyAsync(P, h->Pext, sizeof(double) * h->n9, hipMemcpyDeviceToHost, h->st));
     CK(hipStreamSynchronize(h->st));
   }
@@ -2338,11 +2343,11 @@ extern "C" int dmk_constitutive(dmk_handle* h, double dt, const double* F, doubl
 
 extern "C" int dmk_constitutive_device(dmk_handle* h, double dt, const double* F_dev, double* P_dev, int32_t* status) {
   if (!h || !F_dev) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
-  CKL(dmk_aos_to_soa(F_dev, h->N, 9, 0, h->N, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(F_dev, h->N, 9, h->Fext, h->st));
   int rc = constitutive(h, h->Fext, dt, false, true);
   if (rc) return rc;
   if (P_dev) {
-    CKL(dmk_soa_to_aos(h->P_hom, h->N, 9, 0, h->N, P_dev, h->st));
+    CKL(dmk_soa_to_aos(h->P_hom, h->N, 9, P_dev, h->st));
     CK(hipStreamSynchronize(h->st));
   }
   if (status) *status = h->status;
@@ -2370,6 +2375,29 @@ static int field_dev(dmk_handle* h, int what, const double** p, int* w) {
   }
 }
 
+// Fields go to and from the host through a buffer that the handle keeps, as large as
+// the largest field asked for (with one allocated for each call an increment of
+// 64^3 cells and its F, P and xi took 3 % longer); the stiffness, 81 values a
+// cell, gets one for the call.  Several threads may read fields of one handle, also
+// while another runs its solver: the buffer serves nothing else and has a lock
+// of its own, and a field is taken whole, at one point of the handle's stream.
+static int stage_get(dmk_handle* h, int w, double** buf) {
+  const size_t n = (size_t)w * h->N;
+  if (w > DMK_NSL_MAX) {
+    CK(hipMallocAsync((void**)buf, sizeof(double) * n, h->st));
+    return 0;
+  }
+  if (h->stage_n < n) {
+    if (h->stage) CK(hipFree(h->stage));
+    h->stage = nullptr;
+    h->stage_n = 0;
+    CK(hipMalloc((void**)&h->stage, sizeof(double) * n));
+    h->stage_n = n;
+  }
+  *buf = h->stage;
+  return 0;
+}
+
 extern "C" int dmk_mech_get_field(dmk_handle* h, int32_t what, double* dst) {
   if (!h || !dst) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   if (what == 6) {   // F_i = I
@@ -2380,15 +2408,12 @@ extern "C" int dmk_mech_get_field(dmk_handle* h, int32_t what, double* dst) {
   const double* p;
   int w;
   if (field_dev(h, what, &p, &w)) { dmk_set_error("unknown field %d", what); return DMK_ERR_ARG; }
-  // through the handle's staging field, as many cells at a time as it holds (with a
-  // buffer allocated for each call an increment of 64^3 cells and its F, P and xi
-  // took 3 % longer)
-  const long step = std::max(1L, h->n9 / w);
-  for (long e0 = 0; e0 < h->N; e0 += step) {
-    const long n = std::min(step, h->N - e0);
-    CKL(dmk_soa_to_aos(p, h->N, w, e0, n, h->Pext, h->st));
-    CK(hipMemcpyAsync(dst + e0 * w, h->Pext, sizeof(double) * w * n, hipMemcpyDeviceToHost, h->st));
-  }
+  std::lock_guard<std::mutex> lk(h->stage_mu);
+  double* buf;
+  if (int rc = stage_get(h, w, &buf)) return rc;
+  CKL(dmk_soa_to_aos(p, h->N, w, buf, h->st));
+  CK(hipMemcpyAsync(dst, buf, sizeof(double) * w * h->N, hipMemcpyDeviceToHost, h->st));
+  if (buf != h->stage) CK(hipFreeAsync(buf, h->st));
   CK(hipStreamSynchronize(h->st));
   return 0;
 }
@@ -2401,12 +2426,11 @@ extern "C" int dmk_mech_set_field(dmk_handle* h, int32_t what, const double* src
     dmk_set_error("field %d cannot be set", what);
     return DMK_ERR_ARG;
   }
-  const long step = std::max(1L, h->n9 / w);
-  for (long e0 = 0; e0 < h->N; e0 += step) {
-    const long n = std::min(step, h->N - e0);
-    CK(hipMemcpyAsync(h->Pext, src + e0 * w, sizeof(double) * w * n, hipMemcpyHostToDevice, h->st));
-    CKL(dmk_aos_to_soa(h->Pext, h->N, w, e0, n, (double*)p, h->st));
-  }
+  std::lock_guard<std::mutex> lk(h->stage_mu);
+  double* buf;                       // (no settable field is wider than the kept buffer's)
+  if (int rc = stage_get(h, w, &buf)) return rc;
+  CK(hipMemcpyAsync(buf, src, sizeof(double) * w * h->N, hipMemcpyHostToDevice, h->st));
+  CKL(dmk_aos_to_soa(buf, h->N, w, (double*)p, h->st));
   // the restart also sets the increment-start copies (phase_mechanical.f90:1265-1280)
   const DmkMPDev& mp = h->mp;
   size_t b = sizeof(double) * w * h->N;
@@ -2624,7 +2648,7 @@ extern "C" int dmk_grid_set_restart(dmk_handle* h, int32_t restart_inc) {
 extern "C" int dmk_gamma_convolution(dmk_handle* h, const double* field, const double aim[9], double* out) {
   if (!h || !field || !aim || !out) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, field, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, 0, h->N, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
   // the transform path of the basic residual (x-y passes, z passes with Gamma)
   CKL(dmk_fft_r2c_xy(&h->fft, 9, h->Fext, h->Z, h->st));
   GammaArgs g = h->ga;
@@ -2635,7 +2659,7 @@ extern "C" int dmk_gamma_convolution(dmk_handle* h, const double* field, const d
   int nb;
   CKL(dmk_gamma_conv(&h->fft, h->Z, &g, h->divp, &nb, h->st));
   CKL(dmk_fft_c2r_xy(&h->fft, 9, h->Z, h->Fext, h->st));
-  CKL(dmk_soa_to_aos(h->Fext, h->N, 9, 0, h->N, h->Pext, h->st));
+  CKL(dmk_soa_to_aos(h->Fext, h->N, 9, h->Pext, h->st));
   CK(hipMemcpyAsync(out, h->Pext, sizeof(double) * h->n9, hipMemcpyDeviceToHost, h->st));
   CK(hipStreamSynchronize(h->st));
   return 0;
@@ -2645,7 +2669,7 @@ extern "C" int dmk_gamma_convolution(dmk_handle* h, const double* field, const d
 extern "C" int dmk_divergence_rms(dmk_handle* h, const double* field, double* out) {
   if (!h || !field || !out) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, field, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, 0, h->N, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
   CKL(dmk_fft_r2c(&h->fft, 9, h->Fext, h->Z, h->st));
   GammaArgs g = h->ga;
   g.do_div = 1;
@@ -2665,7 +2689,7 @@ extern "C" int dmk_divergence_rms(dmk_handle* h, const double* field, double* ou
 extern "C" int dmk_curl_rms(dmk_handle* h, const double* field, double* out) {
   if (!h || !field || !out) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, field, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, 0, h->N, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
   CKL(dmk_fft_r2c(&h->fft, 9, h->Fext, h->Z, h->st));
   CKL(dmk_curl_partial(h->Z, &h->ga, h->partial, h->st));
   int nb = dmk_gamma_div_blocks(&h->ga);
@@ -2683,7 +2707,7 @@ extern "C" int dmk_curl_rms(dmk_handle* h, const double* field, double* out) {
 extern "C" int dmk_fft_forward(dmk_handle* h, int32_t howmany, const double* in, double* out) {
   if (!h || !in || !out || howmany < 1 || howmany > 9) { dmk_set_error("bad argument"); return DMK_ERR_ARG; }
   CK(hipMemcpyAsync(h->Pext, in, sizeof(double) * howmany * h->N, hipMemcpyHostToDevice, h->st));
-  CKL(dmk_aos_to_soa(h->Pext, h->N, howmany, 0, h->N, h->Fext, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, howmany, h->Fext, h->st));
   CKL(dmk_fft_r2c(&h->fft, howmany, h->Fext, h->Z, h->st));
   std::vector<double> tmp(2 * howmany * h->Nk);
   CK(hipMemcpyAsync(tmp.data(), h->Z, sizeof(double) * tmp.size(), hipMemcpyDeviceToHost, h->st));
@@ -2707,7 +2731,7 @@ extern "C" int dmk_fft_backward(dmk_handle* h, int32_t howmany, const double* in
     }
   CK(hipMemcpyAsync(h->Z, tmp.data(), sizeof(double) * tmp.size(), hipMemcpyHostToDevice, h->st));
   CKL(dmk_fft_c2r(&h->fft, howmany, h->Z, h->Fext, h->st));
-  CKL(dmk_soa_to_aos(h->Fext, h->N, howmany, 0, h->N, h->Pext, h->st));
+  CKL(dmk_soa_to_aos(h->Fext, h->N, howmany, h->Pext, h->st));
   CK(hipMemcpyAsync(out, h->Pext, sizeof(double) * howmany * h->N, hipMemcpyDeviceToHost, h->st));
   CK(hipStreamSynchronize(h->st));
   return 0;

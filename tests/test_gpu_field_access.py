@@ -1,7 +1,6 @@
-"""Fields to and from the host through the staging buffer: one and two cells
-(fewer than a wide field needs of the buffer), a remainder of a tile, several
-passes for the fields wider than nine values.  Values are moved, not computed, so
-they come back bit for bit."""
+"""Fields to and from the host through the staging buffer: one and two cells, a
+remainder of a tile, fields of nine values and wider ones, for which the buffer
+grows.  Values are moved, not computed, so they come back bit for bit."""
 import numpy as np
 import pytest
 
