@@ -1233,6 +1233,7 @@ tangent_kernel(DmkMPDev mp, const DmkPhaseDev* __restrict__ ph_, int phase_id, d
       }
   }
   if (part) {
+    __syncthreads();       // sums: written by lanes 0, 16 and 32, read by all
     double mx = act && n2 > 0.0 ? n2 : 0.0, mn = act && n2 < DBL_MAX ? n2 : DBL_MAX;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
