@@ -593,8 +593,8 @@ DI int integrate_stress(PhPtr ph, const DmkNumMech& num, const double* A, double
   double* dir = &sh.dir[0][lane];
 #pragma unroll
   for (int k = 0; k < 9; k++) dir[k * SWG] = 0.0;
-  // norms are compared squared
-  const double er2 = num.eps_rel_Lp * num.eps_rel_Lp, ea2 = num.eps_abs_Lp * num.eps_abs_Lp;
+  // norms are compared squared (a tolerance whose square underflows still takes a residual of 0)
+  const double er2 = num.eps_rel_Lp * num.eps_rel_Lp, ea2 = fmax(num.eps_abs_Lp * num.eps_abs_Lp, 4.9e-324);
   double step = 1.0, res_old = DBL_MAX;
   int it = 0;
   for (;;) {
