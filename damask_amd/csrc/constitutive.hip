@@ -1348,3 +1348,58 @@ extern "C" int dmk_pow_law(const double* x, const double* y, double* out, int32_
   if (rc) dmk_set_error("dmk_pow_law: launch or copy failed");
   return rc;
 }
+
+enum { DMK_POWER_RATES = 0, DMK_POWER_HARDENING = 1, DMK_POWER_LIBRARY = 2 };   // path of dmk_power_laws
+
+// CH values of x a thread, as the per-cell kernels power CH systems at once
+__global__ void power_laws_kernel(const double* __restrict__ x, double y, int path, double* __restrict__ out, int n) {
+  const int i0 = (blockIdx.x * blockDim.x + threadIdx.x) * CH, k = (int)(4.0 * y);
+  if (i0 >= n) return;
+  double v[CH], r[CH];
+#pragma unroll
+  for (int j = 0; j < CH; j++) {
+    v[j] = i0 + j < n ? x[i0 + j] : 1.0;
+    r[j] = path == DMK_POWER_LIBRARY ? v[j] : fabs(v[j]);
+  }
+  if (path == DMK_POWER_RATES) {
+    quarter_power<CH>(r, k - 4);
+#pragma unroll
+    for (int j = 0; j < CH; j++) r[j] *= v[j];
+  } else if (path == DMK_POWER_HARDENING) {
+    quarter_power<CH>(r, k);
+  } else {
+#pragma unroll
+    for (int j = 0; j < CH; j += 4) {
+      Four a, e;
+#pragma unroll
+      for (int q = 0; q < 4; q++) { a.v[q] = r[j + q]; e.v[q] = y; }
+      a = pow4_ool(a, e);
+#pragma unroll
+      for (int q = 0; q < 4; q++) r[j + q] = a.v[q];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < CH; j++)
+    if (i0 + j < n) out[i0 + j] = r[j];
+}
+
+extern "C" int dmk_power_laws(const double* x, double* out, int32_t n, double y, int32_t path) {
+  const bool quarter = path == DMK_POWER_RATES || path == DMK_POWER_HARDENING;
+  if (!x || !out || n < 1 || (!quarter && path != DMK_POWER_LIBRARY) ||
+      (quarter && !(y > 0.0 && y <= 64.0 && y * 4.0 == std::rint(y * 4.0))) || (path == DMK_POWER_RATES && y < 1.0)) {
+    dmk_set_error("dmk_power_laws: invalid argument");
+    return DMK_ERR_ARG;
+  }
+  const size_t b = sizeof(double) * (size_t)n;
+  double* d = nullptr;
+  if (hipMalloc((void**)&d, 2 * b) != hipSuccess) { hipGetLastError(); dmk_set_error("dmk_power_laws: device memory"); return DMK_ERR_HIP; }
+  int rc = hipMemcpy(d, x, b, hipMemcpyHostToDevice) == hipSuccess ? 0 : DMK_ERR_HIP;
+  if (!rc) {
+    const unsigned nb = (unsigned)((n + 64 * CH - 1) / (64 * CH));
+    hipLaunchKernelGGL(power_laws_kernel, dim3(nb), dim3(64), 0, 0, d, y, path, d + n, n);
+    if (hipGetLastError() != hipSuccess || hipMemcpy(out, d + n, b, hipMemcpyDeviceToHost) != hipSuccess) rc = DMK_ERR_HIP;
+  }
+  hipFree(d);
+  if (rc) dmk_set_error("dmk_power_laws: launch or copy failed");
+  return rc;
+}

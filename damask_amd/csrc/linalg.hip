@@ -632,6 +632,31 @@ int dmk_dots(const DotJobs* jobs, long n, double* partial, double* out, hipStrea
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
+extern "C" int dmk_dot_products(const double* v, int64_t n, int32_t n_vec, const int32_t* x, const int32_t* y,
+                                const int32_t* mode, int32_t n_jobs, double* out) {
+  bool ok = v && x && y && mode && out && n > 0 && n_vec > 0 && n_jobs > 0 && n_jobs <= DMK_MAX_DOTS;
+  for (int j = 0; ok && j < n_jobs; j++)
+    ok = x[j] >= 0 && x[j] < n_vec && y[j] >= 0 && y[j] < n_vec && (mode[j] == 0 || mode[j] == 1);
+  if (!ok) { dmk_set_error("dmk_dot_products: invalid argument"); return DMK_ERR_ARG; }
+  const size_t nv = (size_t)n * n_vec, np = (size_t)n_jobs * dmk_nchunk(n);
+  double* d = nullptr;
+  if (hipMalloc((void**)&d, sizeof(double) * (nv + np + n_jobs)) != hipSuccess) {
+    hipGetLastError();
+    dmk_set_error("dmk_dot_products: device memory");
+    return DMK_ERR_HIP;
+  }
+  DotJobs J;
+  J.n = n_jobs;
+  for (int j = 0; j < n_jobs; j++) { J.x[j] = d + n * x[j]; J.y[j] = d + n * y[j]; J.mode[j] = mode[j]; }
+  int rc = 0;
+  if (hipMemcpy(d, v, sizeof(double) * nv, hipMemcpyHostToDevice) != hipSuccess || dmk_dots(&J, n, d + nv, d + nv + np, 0) ||
+      hipMemcpy(out, d + nv + np, sizeof(double) * n_jobs, hipMemcpyDeviceToHost) != hipSuccess)
+    rc = DMK_ERR_HIP;
+  hipFree(d);
+  if (rc) dmk_set_error("dmk_dot_products: launch or copy failed");
+  return rc;
+}
+
 int dmk_response_reduce(const int32_t* st, const int32_t* nn, const int32_t* nf, const double* P, long N,
                         double wgt, double* partial, int* flag, unsigned long long* cnt, double* pav,
                         const AimArgs* a, double* faim, double* report, double* aim, hipStream_t s) {

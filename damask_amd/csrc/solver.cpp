@@ -2665,6 +2665,23 @@ extern "C" int dmk_gamma_convolution(dmk_handle* h, const double* field, const d
   return 0;
 }
 
+// utilities_G_Convolution (spectral_utilities.f90:544-589) of a host field, DC term kept
+extern "C" int dmk_galerkin_convolution(dmk_handle* h, const double* field, double* out) {
+  if (!h || !field || !out) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
+  CK(hipMemcpyAsync(h->Pext, field, sizeof(double) * h->n9, hipMemcpyHostToDevice, h->st));
+  CKL(dmk_aos_to_soa(h->Pext, h->N, 9, h->Fext, h->st));
+  // the transform path of the Galerkin scheme's residual and Jacobian
+  CKL(dmk_fft_r2c_xy(&h->fft, 9, h->Fext, h->Z, h->st));
+  GalerkinArgs ga{};
+  int nb;
+  CKL(dmk_galerkin_conv(&h->fft, h->Z, &h->ga, &ga, h->divp, &nb, h->st));
+  CKL(dmk_fft_c2r_xy(&h->fft, 9, h->Z, h->Fext, h->st));
+  CKL(dmk_soa_to_aos(h->Fext, h->N, 9, h->Pext, h->st));
+  CK(hipMemcpyAsync(out, h->Pext, sizeof(double) * h->n9, hipMemcpyDeviceToHost, h->st));
+  CK(hipStreamSynchronize(h->st));
+  return 0;
+}
+
 // utilities_divergenceRMS (spectral_utilities.f90:650-691)
 extern "C" int dmk_divergence_rms(dmk_handle* h, const double* field, double* out) {
   if (!h || !field || !out) { dmk_set_error("null argument"); return DMK_ERR_ARG; }

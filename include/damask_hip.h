@@ -172,6 +172,10 @@ int dmk_grid_run_loadcase(dmk_handle* h, const dmk_loadcase* lc, double* t_io, d
 /* utilities_GammaConvolution (spectral_utilities.f90:436-501) on a (3,3,N)
  * host field with the handle's reference stiffness; aim = DC value */
 int dmk_gamma_convolution(dmk_handle* h, const double* field, const double aim[9], double* out);
+/* utilities_G_Convolution (spectral_utilities.f90:544-589) of a (3,3,N) host field,
+ * the DC term kept; out is N times the convolution (unnormalised transforms, as the
+ * solver takes it) */
+int dmk_galerkin_convolution(dmk_handle* h, const double* field, double* out);
 /* utilities_divergenceRMS (spectral_utilities.f90:650-691) of a (3,3,N) host field */
 int dmk_divergence_rms(dmk_handle* h, const double* field, double* out);
 
@@ -206,6 +210,18 @@ int dmk_inv_sym3333(const double* A, double* out);
  * positive multiples of 1/4 up to 64 (other exponents are rejected), else the
  * library pow.  A check of the kernels' arithmetic; it allocates. */
 int dmk_pow_law(const double* x, const double* y, double* out, int32_t n, int32_t quarter);
+/* the powers of several slip systems at once, as phases with one exponent for all
+ * systems take them, for n points (host arrays).  path 0: |x|^(y-1) x (slip rates,
+ * y >= 1), 1: |x|^y (hardening), y a multiple of 1/4 up to 64; 2: the library pow
+ * x^y, four at a time (other exponents).  A check of the kernels' arithmetic; it
+ * allocates. */
+int dmk_power_laws(const double* x, double* out, int32_t n, double y, int32_t path);
+/* dot products as a residual evaluation takes them, of n_vec host vectors v
+ * (n values each, one after the other): out[j] = v_x[j] . v_y[j] (mode[j] = 0) or
+ * |v_y[j] - v_x[j]|^2 (1), 1 <= n_jobs <= 64.  A check of the kernels' arithmetic; it
+ * allocates. */
+int dmk_dot_products(const double* v, int64_t n, int32_t n_vec, const int32_t* x, const int32_t* y,
+                     const int32_t* mode, int32_t n_jobs, double* out);
 /* unnormalised 3-D r2c / c2r of howmany (<= 9) interleaved fields, FFTW's
  * conventions (spectral_utilities.f90:239-261): real (howmany, N1, N2, N3) <->
  * complex (howmany, N1/2+1, N2, N3) as (re, im) pairs; c2r ignores the

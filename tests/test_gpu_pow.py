@@ -86,3 +86,75 @@ def test_quarter_path_rejects_other_exponents(gpu_lib):
     from damask_amd import _lib
     with pytest.raises(_lib.DamaskHipError):
         _eval(gpu_lib, np.array([0.5]), np.array([20.1]), True)
+
+
+# The powers of several systems at once (dmk_power_laws): the kernels' path for phases whose
+# systems share one exponent, and the library pow four at a time.
+RATES, HARDENING, LIBRARY = 0, 1, 2
+
+
+def _several(lib, x, y, path):
+    from damask_amd import _lib
+    x = np.ascontiguousarray(x, dtype=np.float64)
+    out = np.empty_like(x)
+    _lib.check(lib.dmk_power_laws(_lib.dptr(x), _lib.dptr(out), len(x), float(y), path), "dmk_power_laws")
+    return out
+
+
+def _root_bound(k):
+    """ulp of x^(k/4) by one powering, as in the module's docstring"""
+    if k == 0:
+        return 0.0
+    p, cb = (k // 4, 0.0) if k % 4 == 0 else ((k // 2, 1.0) if k % 2 == 0 else (k, 1.5))
+    return p * cb + (p - 1) + 1.0
+
+
+def test_shared_quarter_powers_against_long_double(gpu_lib):
+    """Hardening: the bound of the single powering.  Rates: |x|^(y-1) carries that of
+    k - 4, and the product with x one rounding more (at most 1 ulp)."""
+    rng = np.random.default_rng(3)
+    xb = _bases(rng)[:-1]                      # a remainder of the kernel's groups of 12
+    assert len(xb) % 12
+    worst = {}
+    for k in range(1, 257):
+        y = np.full_like(xb, k / 4.0)
+        e = _ulps(_several(gpu_lib, xb, k / 4.0, HARDENING), xb, y)
+        assert e.max() <= _root_bound(k), (k / 4.0, e.max())
+        worst[HARDENING, k] = e.max()
+        if k >= 4:
+            e = _ulps(_several(gpu_lib, xb, k / 4.0, RATES), xb, y)
+            assert e.max() <= _root_bound(k - 4) + 1.0, (k / 4.0, e.max())
+            worst[RATES, k] = e.max()
+    print("max ulp: n=20 %.1f, n=20.25 %.1f, a=2.25 %.1f, a=2 %.1f, over all %.1f"
+          % (worst[RATES, 80], worst[RATES, 81], worst[HARDENING, 9], worst[HARDENING, 8], max(worst.values())),
+          flush=True)
+
+
+def test_library_pow_of_four_against_long_double(gpu_lib):
+    rng = np.random.default_rng(5)
+    xb = _bases(rng)[:-1]
+    for y in rng.uniform(0.5, 40.0, 20):
+        e = _ulps(_several(gpu_lib, xb, y, LIBRARY), xb, np.full_like(xb, y))
+        assert e.max() <= 2.0, (y, e.max())
+
+
+def test_shared_powers_special_cases(gpu_lib):
+    """zero, negative, infinite and NaN bases: |x|^(y-1) x and |x|^y by pow's rules (the odd power of a
+    negative rate keeps its sign), x^y by pow's"""
+    x = np.array([0.0, -0.5, -2.0, np.inf, -np.inf, np.nan, 1.0])
+    for y in (1.0, 1.25, 20.0, 20.5, 63.75):
+        with np.errstate(invalid="ignore"):
+            for path, want in ((RATES, np.abs(x) ** (y - 1.0) * x), (HARDENING, np.abs(x) ** y), (LIBRARY, x ** y)):
+                got = _several(gpu_lib, x, y, path)
+                assert np.array_equal(np.isnan(got), np.isnan(want)), (y, path, got)
+                exact = np.isin(np.abs(x), [0.0, 1.0, np.inf])
+                assert np.array_equal(got[exact], want[exact]), (y, path, got)
+                fin = np.isfinite(want) & ~exact
+                assert np.allclose(got[fin], want[fin], rtol=400 * 2.0**-53, atol=0.0), (y, path, got)
+
+
+def test_several_powers_reject_what_no_phase_takes(gpu_lib):
+    from damask_amd import _lib
+    for y, path in ((20.1, RATES), (0.75, RATES), (64.25, HARDENING), (0.0, HARDENING), (2.0, 3)):
+        with pytest.raises(_lib.DamaskHipError):
+            _several(gpu_lib, np.array([0.5]), y, path)

@@ -40,6 +40,8 @@ def _phase(lattice, n, a, non_schmid):
     ("cI", [20.0], [2.0], True),             # 12 systems, non-Schmid terms
     ("cI", [20.0, 20.0], [2.0, 2.0], True),
     ("cI", [20.0, 16.0], [2.0, 1.25], True),
+    ("cI", [20.0], [2.1], True),             # library pow; n integer: a resolved stress may be negative in both senses
+    ("cI", [20.0, 20.0], [2.0, 2.1], True),
 ])
 def test_response_variants(gpu_lib, oracle, lattice, n, a, non_schmid, cells):
     from damask_amd import config, workloads
