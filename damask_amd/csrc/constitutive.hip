@@ -565,7 +565,7 @@ DI void flow(double dt, const double* Lp, double* B) {
 // F_e = A (I - dt L_p) as A - dt (A L_p): one rounding at the size of F_e per
 // entry.  The stress, and n times as much the rates, see this rounding through
 // the elastic stiffness; it is the floor of the Newton iteration's residual
-// (about 1e-11 of L_p).
+// (below 5e-12 of L_p: a 32^3 tension converges at that tolerance).
 DI void elastic_F(double dt, const double* A, const double* Lp, double* Fe) {
   m_mul(A, Lp, Fe);
 #pragma unroll
@@ -694,11 +694,10 @@ DI void finish_point(PhPtr ph, MpPtr m, const Lane& ln, bool started, const doub
 // integrateStateFPI (src/phase_mechanical.f90:591-676).  State = (xi, gamma),
 // started from xi0 / gam0 (the converged increment, or st0s after a completed
 // sub-step).  Every iterate of the state is its start plus dt times the last
-// damped rate, so only the rates are kept: the two previous ones
-// (dotState_last) in the ping-pong buffers mp.last1 / mp.last2; xi and gamma are
-// written once, on success.  The initial rate is taken at the stress S_0 after a
-// restore, else at the previous sub-step's S (s_cur).  A and Lp stay in
-// registers; on success Lp holds the converged L_p.
+// damped rate: the two previous ones (dotState_last) are kept in the ping-pong
+// buffers mp.last1 / mp.last2, and each iteration stores its xi and gamma.  The
+// initial rate is taken at the stress S_0 after a restore, else at the previous
+// sub-step's S (s_cur).  A and Lp stay in registers; on success Lp holds the converged L_p.
 template <int NSL, bool QP, bool NS>
 DI int integrate_state_fpi(PhPtr ph, const DmkNumMech& num, MpPtr m,
                            const double* Ftarget, const Lane& ln, bool started, bool s_cur, double step, double dt,

@@ -19,8 +19,10 @@
 #define DMK_DENSE __device__ __forceinline__
 
 // 1/x and 1/sqrt(x): the hardware approximation and two Newton steps each
-// (within 1 and 2 ulp for normal results), without the scaling and fix-up
-// sequences of a division and a square root.  An n = 5 factorisation has 5 of
+// (within 1 and 2 ulp for normal arguments and results; 0, infinity and NaN give
+// NaN), without the scaling and fix-up sequences of a division and a square
+// root.  The callers' arguments are positive finite state values, resolved
+// stresses of a non-zero rate, and norms of non-zero columns.  An n = 5 factorisation has 5 of
 // each in one dependent chain.
 DMK_DENSE double dmk_rcp(double x) {
   double r = __builtin_amdgcn_rcp(x);

@@ -52,14 +52,6 @@ DI void m_store(double* f, const Lane& l, const double* T) {
     for (int j = 0; j < 3; j++) st(f, l, i + 3 * j, T[3 * i + j]);
 }
 
-// Make a value opaque to the optimiser (no code emitted): address arithmetic
-// derived from it cannot be hoisted out of the enclosing loop.
-template <class T>
-DI T* opaque(T* p) {
-  asm volatile("" : "+v"(p));
-  return p;
-}
-
 DHI void m_mul(const double* A, const double* B, double* C) {
   double T[9];
 #pragma unroll
