@@ -446,23 +446,15 @@ DI void moments_apply(const double (*H)[RK], const double (*K)[RK], const double
 // from the gamma rates gs = |slip rate| at the state xi(r): ws <- xi rate.
 // xi_sat = xi_inf + f_sat sqrt(sum F_tw) and hf = h_0 (1 + c_1 (sum F_tw)^c_2) at sum F_tw = 0
 // are tabulated per phase.  Returns true when a rate is NaN.
-// xi / xi_sat is the rounded quotient: xi times the rounded 1 / xi_sat, corrected by its
-// residual (Markstein, IBM J. Res. Dev. 34(1) 1990), so that 1 - xi / xi_sat is exactly 0
-// where xi = xi_sat, as a power a_sl < 1 of it needs.  1 / xi in ws would leave 2e-16 there.
-// The sums over the acting systems come first: xi is still on its way from memory.
+// xi / xi_sat is the rounded quotient: xi times the rounded 1 / xi_sat, corrected
+// by its residual (Markstein, IBM J. Res. Dev. 34(1) 1990), so that 1 - xi / xi_sat is
+// exactly 0 where xi = xi_sat, as a power a_sl < 1 of it needs; 1 / xi in ws would
+// leave 2e-16 there.  It costs the way of xi from memory: a stress launch of 64^3
+// cells, 12 systems, 276 -> 286 us, of 45x50x54, 24 systems, 366 -> 363.  With the
+// sums over the acting systems first, while xi is on its way, it took 287 and 370
+// (hg stays in registers over the powering), with the other rows loaded ahead as well up to 335.
 template <int NSL, bool QP, class State>
 DI bool dot_state(PhPtr ph, State xi, const double* gs, double* ws) {
-  double hg[NSL];
-#pragma unroll
-  for (int r = 0; r < NSL; r++) hg[r] = 0.0;
-  bool nan = false;
-#pragma unroll 48 / NSL
-  for (int a = 0; a < NSL; a++) {
-    const double ga = gs[a * SWG];
-    nan |= (ga != ga);
-#pragma unroll
-    for (int r = 0; r < NSL; r++) hg[r] = fma(ph->Hc[a][r], ga, hg[r]);
-  }
   const int ak = QP ? ph->a_k : 0;
 #pragma unroll
   for (int r0 = 0; r0 < NSL; r0 += CH) {
@@ -484,11 +476,24 @@ DI bool dot_state(PhPtr ph, State xi, const double* gs, double* ws) {
       for (int j = 0; j < CH; j++) p[j] = ws[(r0 + j) * SWG];
     }
 #pragma unroll
-    for (int j = 0; j < CH; j++) {
-      const double d = ph->hf[r0 + j] * copysign(p[j], x[j]) * hg[r0 + j];
-      ws[(r0 + j) * SWG] = d;
-      nan |= (d != d);
-    }
+    for (int j = 0; j < CH; j++) ws[(r0 + j) * SWG] = ph->hf[r0 + j] * copysign(p[j], x[j]);
+  }
+  double hg[NSL];
+#pragma unroll
+  for (int r = 0; r < NSL; r++) hg[r] = 0.0;
+  bool nan = false;
+#pragma unroll 48 / NSL
+  for (int a = 0; a < NSL; a++) {
+    const double ga = gs[a * SWG];
+    nan |= (ga != ga);
+#pragma unroll
+    for (int r = 0; r < NSL; r++) hg[r] = fma(ph->Hc[a][r], ga, hg[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < NSL; r++) {
+    const double d = ws[r * SWG] * hg[r];
+    ws[r * SWG] = d;
+    nan |= (d != d);
   }
   return nan;
 }
@@ -745,12 +750,14 @@ DI int integrate_state_fpi(PhPtr ph, const DmkNumMech& num, MpPtr m,
     double* w2p = cur ? q->last1 : q->last2;
     double w1[2 * NSL], w2[2 * NSL], s0[2 * NSL];
 #pragma unroll
-    for (int r = 0; r < 2 * NSL; r++) w1[r] = ld(w1p, ln, r);
+    for (int r = 0; r < NSL; r++) w1[r] = ld(w1p, ln, r);
     ld_start<NSL>(q->xi0, q->st0s, started, ln, 0, s0);
     // the converged Newton iterate evaluated kinetics_sl at this (S, xi): rates
     // are in gs.  A NaN rate ends the iteration with the status of the stress
     // integration, as the reference's exit does (phase_mechanical.f90:638)
     const bool nan = dot_state<NSL, QP>(ph, [&](int r) { return fma(w1[r], dt, s0[r]); }, gs, ws);
+#pragma unroll
+    for (int r = NSL; r < 2 * NSL; r++) w1[r] = ld(w1p, ln, r);
     ld_start<NSL>(q->gam0, q->st0s + NSL * ln.sN, started, ln, 0, s0 + NSL);
 #pragma unroll
     for (int r = 0; r < 2 * NSL; r++) w2[r] = 0.0;
