@@ -205,8 +205,7 @@ struct dmk_handle {
   std::vector<void*> allocs;
   double *P_hom, *dPdF;
   double *F, *F_lastinc, *Fdot, *R, *XM, *FM, *XA, *FA, *Xh, *Fh, *Fext, *Pext;
-  double* stage = nullptr;           // fields to and from the host (stage_get), under stage_mu
-  size_t stage_n = 0;
+  double* stage;                     // fields to and from the host (stage_width values a cell), under stage_mu
   std::mutex stage_mu;
   double2 *Z, *U;
   double *u3, *xn_dev, *xp_dev;
@@ -302,6 +301,9 @@ static int dalloc(dmk_handle* h, T** p, size_t n) {
   *p = (T*)v;
   return 0;
 }
+
+// values a cell of the staging buffer: those of the widest field but the stiffness
+static int stage_width(const dmk_handle* h) { return std::max(9, h->nsl_max); }
 
 enum { SM_PAV = 0, SM_CVOL = 9, SM_CMM = 90, SM_DOTS = 180, SM_REP = 256, SM_FAIM = 352, SM_AIM = 368,
        // adjoint: aim bookkeeping, report, mean, dot products, maxima, tangent average
@@ -1989,7 +1991,6 @@ extern "C" void dmk_mech_destroy(dmk_handle* h) {
     for (int k = 0; k < 8; k++) { hipEventDestroy(h->ev[k][0]); hipEventDestroy(h->ev[k][1]); }
   adj_free(h);
   for (void* p : h->allocs) hipFree(p);
-  if (h->stage) hipFree(h->stage);
   if (h->ph_dev) hipFree(h->ph_dev);
   if (h->hsmall) hipHostFree(h->hsmall);
   dmk_fft_free(&h->fft);
@@ -2087,7 +2088,9 @@ static int init_impl(dmk_handle* h, const int32_t cells[3], const double size[3]
   const long nx = h->nx;
   double** sol[] = {&h->F, &h->F_lastinc, &h->Fdot, &h->R, &h->XM, &h->FM, &h->XA, &h->FA};
   for (auto pp : sol) if ((rc = dalloc(h, pp, nx))) return rc;
-  if ((rc = dalloc(h, &h->Fext, n9)) || (rc = dalloc(h, &h->Pext, n9))) return rc;
+  if ((rc = dalloc(h, &h->Fext, n9)) || (rc = dalloc(h, &h->Pext, n9)) ||
+      (rc = dalloc(h, &h->stage, (size_t)stage_width(h) * N)))
+    return rc;
   if (h->scheme != 0 && (rc = dalloc(h, &h->T, n9))) return rc;
   // NGMRES history (M pairs), or for the Galerkin scheme the 31 Krylov vectors of GMRES(30)
   if (h->scheme == 2) {
@@ -2375,29 +2378,12 @@ static int field_dev(dmk_handle* h, int what, const double** p, int* w) {
   }
 }
 
-// Fields go to and from the host through a buffer that the handle keeps, as large as
-// the largest field asked for (with one allocated for each call an increment of
-// 64^3 cells and its F, P and xi took 3 % longer); the stiffness, 81 values a
-// cell, gets one for the call.  Several threads may read fields of one handle, also
-// while another runs its solver: the buffer serves nothing else and has a lock
-// of its own, and a field is taken whole, at one point of the handle's stream.
-static int stage_get(dmk_handle* h, int w, double** buf) {
-  const size_t n = (size_t)w * h->N;
-  if (w > DMK_NSL_MAX) {
-    CK(hipMallocAsync((void**)buf, sizeof(double) * n, h->st));
-    return 0;
-  }
-  if (h->stage_n < n) {
-    if (h->stage) CK(hipFree(h->stage));
-    h->stage = nullptr;
-    h->stage_n = 0;
-    CK(hipMalloc((void**)&h->stage, sizeof(double) * n));
-    h->stage_n = n;
-  }
-  *buf = h->stage;
-  return 0;
-}
-
+// Fields go to and from the host through a buffer that the handle keeps (with one
+// allocated for each call an increment of 64^3 cells and its F, P and xi took 3 %
+// longer); the stiffness, 81 values a cell, gets one for the call.  Several threads
+// may read fields of one handle, also while another runs its solver: the buffer
+// serves nothing else and has a lock, and a field is taken whole, at one
+// point of the handle's stream.
 extern "C" int dmk_mech_get_field(dmk_handle* h, int32_t what, double* dst) {
   if (!h || !dst) { dmk_set_error("null argument"); return DMK_ERR_ARG; }
   if (what == 6) {   // F_i = I
@@ -2409,8 +2395,8 @@ extern "C" int dmk_mech_get_field(dmk_handle* h, int32_t what, double* dst) {
   int w;
   if (field_dev(h, what, &p, &w)) { dmk_set_error("unknown field %d", what); return DMK_ERR_ARG; }
   std::lock_guard<std::mutex> lk(h->stage_mu);
-  double* buf;
-  if (int rc = stage_get(h, w, &buf)) return rc;
+  double* buf = h->stage;
+  if (w > stage_width(h)) CK(hipMallocAsync((void**)&buf, sizeof(double) * w * h->N, h->st));
   CKL(dmk_soa_to_aos(p, h->N, w, buf, h->st));
   CK(hipMemcpyAsync(dst, buf, sizeof(double) * w * h->N, hipMemcpyDeviceToHost, h->st));
   if (buf != h->stage) CK(hipFreeAsync(buf, h->st));
@@ -2427,8 +2413,7 @@ extern "C" int dmk_mech_set_field(dmk_handle* h, int32_t what, const double* src
     return DMK_ERR_ARG;
   }
   std::lock_guard<std::mutex> lk(h->stage_mu);
-  double* buf;                       // (no settable field is wider than the kept buffer's)
-  if (int rc = stage_get(h, w, &buf)) return rc;
+  double* buf = h->stage;            // the stiffness, the only wider field, cannot be set
   CK(hipMemcpyAsync(buf, src, sizeof(double) * w * h->N, hipMemcpyHostToDevice, h->st));
   CKL(dmk_aos_to_soa(buf, h->N, w, (double*)p, h->st));
   // the restart also sets the increment-start copies (phase_mechanical.f90:1265-1280)

@@ -1,6 +1,6 @@
 """Fields to and from the host through the staging buffer: one and two cells, a
-remainder of a tile, fields of nine values and wider ones, for which the buffer
-grows.  Values are moved, not computed, so they come back bit for bit."""
+remainder of a tile, fields of nine values and wider ones, the stiffness through a
+buffer of its own.  Values are moved, not computed, so they come back bit for bit."""
 import numpy as np
 import pytest
 
