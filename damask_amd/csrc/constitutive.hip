@@ -21,7 +21,7 @@
 //
 // What bounds the stress kernel: FP64 issue and the latency of a wavefront's own
 // chain (Newton steps in sequence, each with a QR and scalar table loads), not
-// HBM.  64^3 cells of the cF tension, 5.5 Newton iterations a cell: 0.275 ms a
+// HBM.  64^3 cells of the cF tension, 5.5 Newton iterations a cell: 0.286 ms a
 // launch, 0.69 ms as an 8x8 system per Newton step with the state in global
 // scratch; 45x50x54 cells with 24 systems 0.36 against 0.95 ms; 16^3 cells (one
 // wavefront a CU) 0.09 against 0.21 ms.

@@ -24,7 +24,9 @@ struct DmkFFT;
 struct DmkFFTShapes;
 // Tile shapes for an RVE's transforms in the batch's rounds: those of the first
 // RVE of its grid, with the same passes fused, that asked.  Each handle times its
-// own, and RVEs whose shapes differ cannot share a launch.
+// own, and RVEs whose shapes differ cannot share a launch.  Fields do not depend on
+// the shapes; the divergence norm sums its blocks, so its last bits do, as they do
+// between two handles.
 DmkFFTShapes dmk_stress_batch_shapes(DmkStressBatch* b, const DmkFFT* fft);
 // Hand a request of a lockstep round to the batch (struct DmkResidDev: a
 // whole residual evaluation with its stress items, an application of the
