@@ -242,7 +242,9 @@ DI double resolved(PhPtr ph, int a, const double* s, bool& pos) {
 
 // x_j^(k/4) of n values with one binary powering of x, sqrt(x) or sqrt(sqrt(x)),
 // as pow_law takes one: the branches are taken once and the products are n
-// independent chains
+// independent chains.  Largest errors against long double: the rates' x^(n-1) x
+// 10.7 ulp at n = 20 (pow_law: 12) and 115 at n = 20.25, the hardening's x^a 11 at
+// a = 2.25 and 0.5 at a = 2.
 template <int n>
 DI void quarter_power(double* x, int k) {
   if (k & 3) {
